@@ -102,13 +102,10 @@ class Problem:
         F = self.fine
         return F.n_elem * (32 + 2) + F.n_node * 2 * b_v + (0 if self.uniform else F.n_elem * b_v)
 
-    def kernel_name(self, block, rows):
-        """The FP64 MatVec kernel instantiation for a stencil-row source (da.ROWS_*)."""
-        mass = "true" if self.uniform else "false"
-        uni = "true" if self.uniform else "false"
-        lane = "true" if rows == 1 else "false"
-        comb = "true" if rows == 2 and self.uniform else "false"
-        return f"dgh::tile_op_kernel<double, double, {mass}, 0, {block}, {uni}, {lane}, {comb}>"
+    def kernel_name(self, block):
+        """The FP64 MatVec kernel instantiation (factored element product)."""
+        mass = uni = "true" if self.uniform else "false"
+        return f"dgh::tile_op_kernel<double, double, {mass}, 0, {block}, {uni}, false, false, true>"
 
     def params(self, **kw):
         import dendro_amd as da
@@ -457,7 +454,7 @@ def matvec_section(P, args, dev, stream):
     x32, y32 = x.float(), torch.empty(F.n_node, dtype=torch.float32, device=dev)
     ms32, _ = time_matvec(mf, x32, y32, args.steps, args.warmup, stream, prec=da.F32)
     del x32, y32
-    kernel = P.kernel_name(tuned["block"], ti["lane_stencils"])
+    kernel = P.kernel_name(tuned["block"])
     res = {
         "ms": ms, "gdofs": F.n_node / (ms * 1e-3) / 1e9, "achieved": achieved, "alg": alg,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -355,7 +355,7 @@ class Mesh:
                 "n_node_entries": nn.value, "lds_bytes_f64": lds.value, "lane_stencils": on.value}
 
     def set_lane_stencils(self, on):
-        """Stencil-row source: ROWS_LANE (1) per lane from an LDS copy of the table;
+        """Stencil rows instead of the factored product: ROWS_LANE (1) per lane from an LDS copy of the table;
         ROWS_TYPE (0) per stencil type of a wavefront through the scalar cache; ROWS_CLASS (2)
         the element matrix of each (type, level) class (uniform coefficients only)."""
         check(lib().dgh_mesh_set_lane_stencils(self.h, int(on)))

@@ -37,6 +37,9 @@ static int op_rows_mode(const dgh_mesh m) {
   return (m->lane_rows == DGH_ROWS_CLASS && m->op.rk64.p) ? DGH_ROWS_TYPE : m->lane_rows;
 }
 
+// Whether the products run factored (no stencil rows): unless a row source was chosen.
+static bool op_factored(const dgh_mesh m) { return m->rows_auto; }
+
 // stencil rows of an operator launch: the class matrices for uniform coefficients (unless
 // rows are read per lane from LDS), else the child-0 Laplacian and mass rows
 template <class T> const T* kctab(const DevTiles& d);
@@ -60,6 +63,9 @@ template <int BLOCK>
 static void check_op_plan(dgh_mesh m) {
   if (m->op.block != BLOCK || m->op.plan.own_cap != op_own_cap(BLOCK))
     fail(DGH_ERR_STATE, "operator tiling built for block %d, launched with %d", m->op.block, BLOCK);
+  if (m->op.plan.max_touch > uint32_t(OP_XC * BLOCK) || m->op.plan.max_own > uint32_t(OP_OC * BLOCK))
+    fail(DGH_ERR_STATE, "operator tiles of %u touched and %u owned nodes exceed %d threads", m->op.plan.max_touch,
+         m->op.plan.max_own, BLOCK);
 }
 
 template <class T, int MODE, int BLOCK>
@@ -70,6 +76,24 @@ static void launch_op_b(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
   const size_t lds = op_lds_bytes<T>(m);
   const T* kap = rk<T>(m);
   const T* mas = rm<T>(m);
+  if constexpr (MODE != OP_DIAG) {
+    if (op_factored(m)) {
+      const double u1 = m->lap_fac * m->hFac / 2.0, u2 = m->mass_fac * m->hFac * m->hFac * m->hFac / 8.0;
+#define DGH_FACT_LAUNCH(MASS, UNI)                                                                              \
+  hipLaunchKernelGGL((tile_op_kernel<T, T, MASS, MODE, BLOCK, UNI, false, false, true>), dim3(grid), dim3(BLOCK), \
+                     lds, st, m->op.tiles.p, nt, m->op.lid.p, kap, mas, u1, u2, m->maxD, 1.0, (const T*)nullptr, \
+                     m->op.node_tab.p, m->op.texp.p, io)
+      if (!kap)
+        DGH_FACT_LAUNCH(true, true);
+      else if (!mas)
+        DGH_FACT_LAUNCH(false, false);
+      else
+        DGH_FACT_LAUNCH(true, false);
+#undef DGH_FACT_LAUNCH
+      HIP_CHECK(hipGetLastError());
+      return;
+    }
+  }
 #define DGH_OP_LAUNCH(MASS, UNI, LANE, COMB)                                                                   \
   hipLaunchKernelGGL((tile_op_kernel<T, T, MASS, MODE, BLOCK, UNI, LANE, COMB>), dim3(grid), dim3(BLOCK), lds, st, \
                      m->op.tiles.p, nt, m->op.lid.p, kap, mas, m->lap_fac, m->mass_fac, m->maxD,      \
@@ -215,7 +239,7 @@ void upload_coefs(dgh_mesh m, DevTiles& d) {
     }
     if (!std::isfinite(mx)) fail(DGH_ERR_ARG, "non-finite element coefficients");
     int e = -1022;
-    if (mx > 0.0) std::frexp(mx, &e);   // mx < 2^e
+    if (mx > 0.0) std::frexp(mx * FX_MARGIN, &e);   // mx < 2^e
     te[t] = make_int2(std::max(e, -1022), v);
   }
   d.texp.upload(te.data(), te.size());
@@ -262,7 +286,8 @@ void upload_coefs(dgh_mesh m, DevTiles& d) {
 }
 
 // The device form of a plan's records (load_rec): each record's 8 vertex ids with its class
-// (child-0 type | level << 5) in the top 2 bits of ids 0..4, so no class array is read.
+// (child-0 type | level << 5) in the top 2 bits of ids 0..4, so no class array is read, and its
+// hanging vertices (hang_bits) in those of ids 5..7.
 static std::vector<uint16_t> pack_records(const TilePlan& plan) {
   if (plan.max_touch > REC_MAX_TOUCH)
     fail(DGH_ERR_ARG, "a tile touches %u nodes (at most %u): use a smaller tile size", plan.max_touch, REC_MAX_TOUCH);
@@ -271,6 +296,8 @@ static std::vector<uint16_t> pack_records(const TilePlan& plan) {
     const uint32_t c = plan.meta[r];
     if (c >= 1024u) fail(DGH_ERR_MESH, "record class %u out of range", c);
     for (int q = 0; q < 5; ++q) p[r * 8 + q] = uint16_t(p[r * 8 + q] | (((c >> (2 * q)) & 3u) << 14));
+    const uint32_t hb = hang_bits(kEtypeMask[0][c & 31u]);
+    for (int q = 0; q < 3; ++q) p[r * 8 + 5 + q] = uint16_t(p[r * 8 + 5 + q] | (((hb >> (2 * q)) & 3u) << 14));
   }
   return p;
 }
@@ -514,48 +541,9 @@ static const void* precondition_raw(dgh_solver s, const double* r, hipStream_t s
   return vcycle<double>(s, top, r, st, x1_ready);
 }
 
-template <int BLOCK>
-static void launch_cg_b(dgh_mesh m, const double* p, double* w, double* part, hipStream_t st) {
-  check_op_plan<BLOCK>(m);
-  const int nt = int(m->op.plan.tiles.size());
-  const unsigned grid = unsigned(NXCD * ((nt + NXCD - 1) / NXCD));
-  const size_t lds = op_lds_bytes<double>(m);
-  const OpIO<double> io{p, w, nullptr, nullptr, 0.0, part};
-  const double* kap = m->op.rk64.p;
-  const double* mas = m->op.rm64.p;
-#define DGH_CG_LAUNCH(MASS, UNI, LANE, COMB)                                                                    \
-  hipLaunchKernelGGL((tile_op_kernel<double, double, MASS, OP_CG, BLOCK, UNI, LANE, COMB>), dim3(grid), dim3(BLOCK), \
-                     lds, st, m->op.tiles.p, nt, m->op.lid.p, kap, mas, m->lap_fac, m->mass_fac,      \
-                     m->maxD, m->hFac, op_rows<double>(m, COMB), m->op.node_tab.p, m->op.texp.p, io)
-  const int rows = op_rows_mode(m);
-  if (rows == DGH_ROWS_LANE) {
-    if (!kap)
-      DGH_CG_LAUNCH(true, true, true, false);
-    else if (!mas)
-      DGH_CG_LAUNCH(false, false, true, false);
-    else
-      DGH_CG_LAUNCH(true, false, true, false);
-  } else if (rows == DGH_ROWS_CLASS) {
-    DGH_CG_LAUNCH(true, true, false, true);
-  } else {
-    if (!kap)
-      DGH_CG_LAUNCH(true, true, false, false);
-    else if (!mas)
-      DGH_CG_LAUNCH(false, false, false, false);
-    else
-      DGH_CG_LAUNCH(true, false, false, false);
-  }
-#undef DGH_CG_LAUNCH
-  HIP_CHECK(hipGetLastError());
-}
-
 // w = A p and the tile partials of p.w -> part
 static void launch_cg(dgh_mesh m, const double* p, double* w, double* part, hipStream_t st) {
-  switch (m->block) {
-    case 256: launch_cg_b<256>(m, p, w, part, st); break;
-    case 512: launch_cg_b<512>(m, p, w, part, st); break;
-    default: launch_cg_b<1024>(m, p, w, part, st); break;
-  }
+  launch_op<double, OP_CG>(m, OpIO<double>{p, w, nullptr, nullptr, 0.0, part}, st);
 }
 
 // One CG iteration (everything between two stopping tests), on device scalars only:
@@ -993,7 +981,9 @@ int dgh_mesh_autotune(dgh_mesh m, int prec, uint32_t* tile_elems, uint32_t* bloc
     HIP_CHECK(hipEventCreate(&e1));
     float best = 1e30f;
     uint32_t bt = 0, bb = 0;
-    int bl = 0;
+    // the factored product, which beats every stencil-row source on every tiling measured (64 to
+    // 8192 elements per tile, 9k to 10M elements): the row source is back to the default's
+    m->rows_auto = true;
     // small levels need small tiles: enough workgroups to fill the device
     for (uint32_t T : {128u, 256u, 512u, 1024u, 2048u, 4096u, 8192u}) {
       for (int B : {256, 512, 1024}) {
@@ -1004,30 +994,23 @@ int dgh_mesh_autotune(dgh_mesh m, int prec, uint32_t* tile_elems, uint32_t* bloc
           continue;
         }
         if (m->op.plan.tile_elems != T) continue;   // reduced to fit LDS: tried already
-        // stencil rows per wavefront type, per lane from LDS, per (type, level) class
-        for (int L : {DGH_ROWS_TYPE, DGH_ROWS_LANE, DGH_ROWS_CLASS}) {
-          if (L == DGH_ROWS_CLASS && !m->h_kappa.empty()) continue;   // uniform coefficients only
-          m->lane_rows = L;
-          if (op_lds_bytes<double>(m) > size_t(g.max_lds)) continue;
-          auto run = [&] {
-            if (prec == DGH_F64)
-              launch_matvec<double>(m, xb.p, yb.p, nullptr);
-            else
-              launch_matvec<float>(m, reinterpret_cast<const float*>(xb.p), reinterpret_cast<float*>(yb.p), nullptr);
-          };
-          for (int i = 0; i < 3; ++i) run();
-          HIP_CHECK(hipEventRecord(e0, nullptr));
-          for (int i = 0; i < 10; ++i) run();
-          HIP_CHECK(hipEventRecord(e1, nullptr));
-          HIP_CHECK(hipEventSynchronize(e1));
-          float ms = 0.f;
-          HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-          if (ms < best) {
-            best = ms;
-            bt = T;
-            bb = uint32_t(B);
-            bl = L;
-          }
+        auto run = [&] {
+          if (prec == DGH_F64)
+            launch_matvec<double>(m, xb.p, yb.p, nullptr);
+          else
+            launch_matvec<float>(m, reinterpret_cast<const float*>(xb.p), reinterpret_cast<float*>(yb.p), nullptr);
+        };
+        for (int i = 0; i < 3; ++i) run();
+        HIP_CHECK(hipEventRecord(e0, nullptr));
+        for (int i = 0; i < 10; ++i) run();
+        HIP_CHECK(hipEventRecord(e1, nullptr));
+        HIP_CHECK(hipEventSynchronize(e1));
+        float ms = 0.f;
+        HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        if (ms < best) {
+          best = ms;
+          bt = T;
+          bb = uint32_t(B);
         }
       }
     }
@@ -1035,8 +1018,6 @@ int dgh_mesh_autotune(dgh_mesh m, int prec, uint32_t* tile_elems, uint32_t* bloc
     HIP_CHECK(hipEventDestroy(e1));
     if (!bt) fail(DGH_ERR_STATE, "no tiling candidate fits");
     m->block = int(bb);
-    m->lane_rows = bl;
-    m->rows_auto = false;
     plan_mesh(m, bt);
     if (tile_elems) *tile_elems = bt;
     if (block) *block = bb;

@@ -88,7 +88,7 @@ static void elas_matrices(dgh_mesh m) {
     while ((1u << v) < vmax) ++v;
     if (!std::isfinite(mx)) fail(DGH_ERR_ARG, "non-finite elasticity element matrices");
     int e = -1022;
-    if (mx > 0.0) std::frexp(mx, &e);
+    if (mx > 0.0) std::frexp(mx * FX_MARGIN, &e);
     te[t] = make_int2(std::max(e, -1022), v);
   }
   S.ke.upload(k0.data(), k0.size());

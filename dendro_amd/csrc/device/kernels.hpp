@@ -2,8 +2,8 @@
 //
 // The operator kernel is owner-computes over tiles of Morton-ordered elements (the host
 // plan of tiles.cpp): one workgroup per tile stages the tile's x values in LDS, evaluates
-// every record (own and halo elements) with the 18 child-0 stencils read through the scalar
-// cache, accumulates the rows of the nodes the tile owns with 64-bit fixed-point LDS
+// every record (own and halo elements) with the factored element product (or, on request, with
+// the 18 child-0 stencils' rows), accumulates the rows of the nodes the tile owns with 64-bit fixed-point LDS
 // atomics, and stores each owned node exactly once.  There are no global atomics, y needs no
 // zeroing, and the integer sums make the result independent of the order of the additions.
 #pragma once
@@ -78,13 +78,22 @@ struct Rec {
 };
 
 // A record on the device is 16 bytes: the 8 tile-local vertex ids in 14 bits each, the
-// record's class (child-0 type | level << 5, 10 bits) in the top 2 bits of ids 0..4
-// (pack_records).
+// record's class (child-0 type | level << 5, 10 bits) in the top 2 bits of ids 0..4 and its
+// hanging vertices (rec_hang) in the top 2 bits of ids 5..7 (pack_records).
 constexpr uint32_t REC_ID_MASK = 0x3fffu;
 constexpr uint32_t REC_MAX_TOUCH = REC_ID_MASK + 1u;
 __device__ __forceinline__ uint32_t rec_class(uint4 lp) {
   return ((lp.x >> 14) & 3u) | ((lp.x >> 30) << 2) | (((lp.y >> 14) & 3u) << 4) | ((lp.y >> 30) << 6) |
          (((lp.z >> 14) & 3u) << 8);
+}
+
+// Hanging vertices of a record in child 0's order, one bit each: vertices 1, 2, 4 (edge
+// midpoints) in bits 0..2, 3, 5, 6 (face centres) in bits 3..5.
+__host__ __device__ constexpr uint32_t hang_bits(uint32_t mask) {
+  return ((mask >> 1) & 3u) | (((mask >> 4) & 1u) << 2) | (((mask >> 3) & 1u) << 3) | (((mask >> 5) & 3u) << 4);
+}
+__device__ __forceinline__ uint32_t rec_hang(uint4 lp) {
+  return (lp.z >> 30) | ((lp.w >> 12) & 12u) | ((lp.w >> 26) & 48u);
 }
 
 // kappa/mass: per-record factors formed by the host, or nullptr for uniform coefficients
@@ -118,7 +127,8 @@ constexpr int KFSTRIDE = 128;
 // FP32.  FP64: a contribution c enters as the integer round(c 2^es), formed by one FMA with
 // 1.5 2^52: for |c 2^es| < 2^51 the bit pattern of fma(c, 2^es, 1.5 2^52) is that of
 // 1.5 2^52 plus round(c 2^es), so subtracting the former leaves the integer in two's
-// complement; es keeps every term below 2^FX_BITS.  FP32: round-to-nearest conversion of
+// complement; es keeps every term below 2^FX_BITS (the host's bounds leave a margin of 2^-20 for
+// the rounding of the term itself).  FP32: round-to-nearest conversion of
 // c 2^es (float), es keeping every term below 2^(FX32_BITS - v) where 2^v bounds the number of
 // terms a node of the tile receives, so the 32-bit sums cannot overflow.  es is chosen per
 // tile: the host bounds the element factors times the stencil row sums (texp[t].x: bound
@@ -128,8 +138,9 @@ constexpr int KFSTRIDE = 128;
 // floating-point ones on scattered addresses (ds_add_u64 about twice ds_add_f64, ds_add_u32
 // faster again) and do not depend on the order of the additions, so the operator is
 // bit-reproducible.
-constexpr int FX_BITS = 50;
+constexpr int FX_BITS = 51;
 constexpr int FX32_BITS = 30;
+constexpr double FX_MARGIN = 1.0 + 0x1p-20;
 constexpr double FX_MAGIC = 6755399441055744.0;   // 1.5 * 2^52
 constexpr unsigned long long FX_MAGIC_BITS = 0x4338000000000000ull;
 constexpr int FX_XMIN = -900;                      // |x| below 2^-900 counts as 2^-900
@@ -410,11 +421,174 @@ __device__ __forceinline__ void eval_rows_lane(const Rec& R, uint32_t own_bytes,
   }
 }
 
-// x gathers per thread in flight together: 12 (the 44M-element Helmholtz MatVec 507 -> 482 us
-// against 8), 8 in the FP32 residual and smoothing kernels that also hold the owned nodes' b
-// and invd (12 would take them past the registers of two workgroups per CU)
-constexpr int XCHUNK = 12;
-constexpr int XCHUNK_PREF = 8;
+// ---------------------------------------------------------------- factored element product
+// The element matrix without stencil rows.  The regular element's matrix is a sum of Kronecker
+// products of the 1D matrices [1 -1; -1 1] and [2 1; 1 2]/6, which share the eigenvectors
+// (1, 1) and (1, -1): with W the 8x8 Walsh-Hadamard transform, K_0 = W D W / 8, and D depends
+// only on the number p of difference axes of a mode.  A hanging element's matrix is
+// P_H^T K_0 P_H, P_H the interpolation of its hanging vertices (edge midpoints (x_0 + x_k)/2,
+// face centres (x_0 + x_a + x_b + x_k)/4; the 18 child-0 stencils equal these products to
+// rounding).  One product costs 24 + 24 additions and 8 multiplications, with or without a
+// mass term, plus at most 36 operations for hanging vertices, in one pass of the wavefront
+// whatever types its lanes hold, and reads nothing but its record and its x.  Stencil rows cost
+// 64 (128 with mass) FMAs per pass over a type or class, and each row's scalar load waits behind
+// the LDS additions in flight (they share a counter).  Measured, FP64 / FP32 products, best row
+// source before and this form with the next records prefetched, same tilings:
+//   9,374 elements        16.4 / 14.7 us ->  9.5 /  8.1 us
+//   318,081 elements      19.5 / 17.0    -> 10.2 /  8.9
+//   2.1M, kappa only      35.3 / 31.5    -> 26.6 / 20.9
+//   10.5M (1787 tiles)   129.1 / 100.2   -> 92.4 / 68.1 us; without the prefetch 98.4 / 75.5.
+// What bounds it now at 10.5M elements: 400 MB per product (records 215, node ids and x 129, y 56)
+// at 4.3 TB/s, of the 6 to 7 a copy of this size reaches; its LDS reads and additions take about
+// as long again and overlap only across workgroups.
+//   Laplacian on h: kappa h p 2 (1/6)^(p-1) (1/2)^(3-p); mass: m h^3 (1/6)^p (1/2)^(3-p);
+// FACT_LAP and FACT_MASS are these over 8 for the factors kappa h/2 and m h^3/8.
+__host__ __device__ constexpr double fact_lap(int p) {
+  return p == 0 ? 0.0 : p == 1 ? 0.125 : p == 2 ? 1.0 / 12.0 : 1.0 / 24.0;
+}
+__host__ __device__ constexpr double fact_mass(int p) {
+  return p == 0 ? 0.125 : p == 1 ? 1.0 / 24.0 : p == 2 ? 1.0 / 72.0 : 1.0 / 216.0;
+}
+
+// d[p]: the mode factors of an element with scaled factors f1 (Laplacian) and f2 (mass)
+template <class T, bool MASS>
+__device__ __forceinline__ void fact_modes(T f1, T f2, T d[4]) {
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    d[p] = f1 * T(fact_lap(p));
+    if (MASS) d[p] = p == 0 ? f2 * T(fact_mass(0)) : d[p] + f2 * T(fact_mass(p));
+  }
+}
+
+// DGH_NO_SELECT in a branch keeps it one: the compiler otherwise evaluates every vertex and
+// selects (75 more vector instructions per 64 records with hanging vertices), where records
+// sorted by type leave most wavefronts with few of the six branches taken.
+#define DGH_NO_SELECT asm volatile("")
+// v <- P_H v; q = 1/4 (a register: the compiler would otherwise scale
+// by a quarter with the slower ldexp)
+template <class T>
+__device__ __forceinline__ void hang_interp(T v[8], uint32_t hb, T q) {
+  if (hb == 0u) return;
+  if (hb & 8u) { DGH_NO_SELECT; v[3] = q * ((v[0] + v[1]) + (v[2] + v[3])); }
+  if (hb & 16u) { DGH_NO_SELECT; v[5] = q * ((v[0] + v[1]) + (v[4] + v[5])); }
+  if (hb & 32u) { DGH_NO_SELECT; v[6] = q * ((v[0] + v[2]) + (v[4] + v[6])); }
+  if (hb & 1u) { DGH_NO_SELECT; v[1] = T(0.5) * (v[0] + v[1]); }
+  if (hb & 2u) { DGH_NO_SELECT; v[2] = T(0.5) * (v[0] + v[2]); }
+  if (hb & 4u) { DGH_NO_SELECT; v[4] = T(0.5) * (v[0] + v[4]); }
+}
+// v <- P_H^T v
+template <class T>
+__device__ __forceinline__ void hang_interp_t(T v[8], uint32_t hb, T q) {
+  if (hb == 0u) return;
+  if (hb & 1u) { DGH_NO_SELECT; v[1] *= T(0.5); v[0] += v[1]; }
+  if (hb & 2u) { DGH_NO_SELECT; v[2] *= T(0.5); v[0] += v[2]; }
+  if (hb & 4u) { DGH_NO_SELECT; v[4] *= T(0.5); v[0] += v[4]; }
+  if (hb & 8u) { DGH_NO_SELECT; v[3] *= q; v[0] += v[3]; v[1] += v[3]; v[2] += v[3]; }
+  if (hb & 16u) { DGH_NO_SELECT; v[5] *= q; v[0] += v[5]; v[1] += v[5]; v[4] += v[5]; }
+  if (hb & 32u) { DGH_NO_SELECT; v[6] *= q; v[0] += v[6]; v[2] += v[6]; v[4] += v[6]; }
+}
+
+// v <- W diag(d[popcount]) W v.  Without a mass term the mean mode's factor is zero.
+template <class T, bool MASS>
+__device__ __forceinline__ void fact_product(T v[8], const T d[4]) {
+#pragma unroll
+  for (int b = 1; b < 8; b <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & b)) {
+        const T s = v[i] + v[i | b];
+        v[i | b] = v[i] - v[i | b];
+        v[i] = s;
+      }
+#pragma unroll
+  for (int i = MASS ? 0 : 1; i < 8; ++i) v[i] *= d[(i & 1) + ((i >> 1) & 1) + (i >> 2)];
+#pragma unroll
+  for (int b = 1; b < 8; b <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & b)) {
+        if (!MASS && b == 1 && i == 0) {
+          v[0] = v[1];
+          v[1] = -v[1];
+          continue;
+        }
+        const T s = v[i] + v[i | b];
+        v[i | b] = v[i] - v[i | b];
+        v[i] = s;
+      }
+}
+
+// Fixed-point term of an already scaled value (see FX_BITS).  The low word of the magic
+// number's bits is zero, so only the high word is corrected.
+__device__ __forceinline__ unsigned long long fx_round(double v) {
+  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v + FX_MAGIC));
+  const uint32_t hi = uint32_t(b >> 32) - uint32_t(FX_MAGIC_BITS >> 32);
+  return (static_cast<unsigned long long>(hi) << 32) | uint32_t(b);
+}
+__device__ __forceinline__ unsigned int fx_round(float v) {
+  return static_cast<unsigned int>(__float2int_rn(v));
+}
+
+// One record for the factored product, as loaded (unpacked where it is evaluated, so that it
+// holds four registers while the x gather runs), and its element factors (per record).
+template <class T>
+struct RecF {
+  uint4 lp;
+  T k1, k2;
+};
+template <class T, bool MASS, bool UNI>
+__device__ __forceinline__ void load_rec_fact(RecF<T>& R, uint32_t g, const uint16_t* __restrict__ lid,
+                                              const T* __restrict__ kappa, const T* __restrict__ mass) {
+  R.lp = reinterpret_cast<const uint4*>(lid)[g];
+  if (!UNI) {
+    R.k1 = kappa[g];
+    if (MASS) R.k2 = mass[g];
+  }
+}
+
+// u1 = lap_fac hFac / 2, u2 = mass_fac hFac^3 / 8: the factors of a uniform-coefficient
+// element of level lev are u1 2^(maxD - lev) and u2 8^(maxD - lev).
+template <class T, bool MASS, uint32_t XS, bool UNI>
+__device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, int es, double u1, double u2,
+                                          uint32_t maxD) {
+  const uint4 lp = R.lp;
+  const uint32_t w[4] = {lp.x, lp.y, lp.z, lp.w};
+  uint32_t l[8];   // LDS byte offsets of the vertices
+#pragma unroll
+  for (int j = 0; j < 8; ++j) l[j] = ((w[j >> 1] >> (16 * (j & 1))) & REC_ID_MASK) * uint32_t(sizeof(T));
+  const uint32_t hb = rec_hang(lp);
+  T v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = *lds_at<T>(XS + l[j]);
+  T f1, f2 = T(0);
+  if (UNI) {
+    const int hs = int(maxD - (rec_class(lp) >> 5));
+    f1 = T(ldexp(u1, hs + es));
+    if (MASS) f2 = T(ldexp(u2, 3 * hs + es));
+  } else if constexpr (sizeof(T) == 8) {
+    f1 = ldexp(R.k1, es);
+    if (MASS) f2 = ldexp(R.k2, es);
+  } else {
+    f1 = T(ldexp(double(R.k1), es));
+    if (MASS) f2 = T(ldexp(double(R.k2), es));
+  }
+  T d[4];
+  fact_modes<T, MASS>(f1, f2, d);
+  T q = T(0.25);
+  asm("" : "+s"(q));
+  hang_interp(v, hb, q);
+  fact_product<T, MASS>(v, d);
+  hang_interp_t(v, hb, q);
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (l[k] < own_bytes) lds_add(lds_at<fx_acc_t<T>>(l[k]), fx_round(v[k]));
+}
+
+// Touched and owned nodes per thread of a tile, from the plan's bounds (op_own_cap, op_budget):
+// at most 5.94 BLOCK touched and 4 BLOCK owned nodes.  One batch of OP_XC gathers therefore
+// covers a tile, with every index static: ids and held values stay in registers.
+constexpr int OP_XC = 6;
+constexpr int OP_OC = 4;
 
 // KF: [18][128] child-0 full stencil rows of precision T (Laplacian, then mass).
 // kappa/mass: per record (nullptr: uniform lap_fac / mass_fac).  MASS: mass term present.
@@ -429,7 +603,10 @@ constexpr int XCHUNK_PREF = 8;
 // passes through the scalar cache.
 // COMB (uniform coefficients, not LANE): KF is the tiling's class matrix table (fac1 L +
 // fac2 M per record class, eval_rows' COMB form) and the records' factors are not formed.
-template <class T, class TC, bool MASS, int MODE, int BLOCK, bool UNI = false, bool LANE = false, bool COMB = false>
+// FACT: the factored product (eval_fact) instead of stencil rows; KF and hFac are unused, and
+// lap_fac and mass_fac arrive scaled (lap_fac hFac / 2, mass_fac hFac^3 / 8).
+template <class T, class TC, bool MASS, int MODE, int BLOCK, bool UNI = false, bool LANE = false, bool COMB = false,
+          bool FACT = false>
 __global__ void __launch_bounds__(BLOCK)
 tile_op_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* __restrict__ lid,
                const TC* __restrict__ kappa,
@@ -452,166 +629,129 @@ tile_op_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* __
   const uint32_t* nodes = node_tab + rec.node_off;
   const uint32_t n_own = rec.n_own;
   // first record: its loads are issued before the x gather so both chains overlap
-  Rec R;
-  if (threadIdx.x < rec.n_elem)
-    load_rec<TC, MASS, sizeof(T), UNI ? 1 : 0, !COMB>(R, rec.elem_off + threadIdx.x, lid, kappa, mass, lap_fac,
-                                                      mass_fac, maxD, hFac);
+  static_assert(!FACT || (MODE != OP_DIAG && !LANE && !COMB && std::is_same<T, TC>::value),
+                "the factored product has no diagonal and reads no rows");
+  typename std::conditional<FACT, RecF<T>, Rec>::type R;
+  // the wavefront's records: w0, w0 + BLOCK, ... (64 each); lanes past the last record load it
+  // again and add nothing
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t w0 = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x - lane)));
+  auto load = [&](decltype(R)& r, uint32_t r0) {
+    const uint32_t g = rec.elem_off + min(r0 + lane, rec.n_elem - 1u);
+    if constexpr (FACT)
+      load_rec_fact<T, MASS, UNI>(r, g, lid, kappa, mass);
+    else
+      load_rec<TC, MASS, sizeof(T), UNI ? 1 : 0, !COMB>(r, g, lid, kappa, mass, lap_fac, mass_fac, maxD, hFac);
+  };
+  load(R, w0);
   const uint32_t kf = tile_kf_off<T>(XS, rec.n_touch);
   if (LANE) {   // the stencil table, copied while the gather runs (visible after the barrier)
     for (uint32_t i = threadIdx.x; i < KF_ELEMS; i += BLOCK) lds_at<T>(kf)[i] = KF[i];
   }
-  uint32_t xhi = 0;   // high word of max |x| over the values this thread staged
-  // FP32 residual and smoothing with up to 512 threads: the owned nodes' ids, b and invd are
-  // loaded with the first gather batch, so the store phase waits on no global load (tiles of
-  // at most XC * BLOCK owned nodes; larger ones reload them).  In FP64, and with 1024-thread
-  // tiles (two workgroups per CU need at most 64 VGPRs), the held values cost more than the
-  // reloads (8M-point octree, 1024-thread finest tiles: mixed PCG 36.4 ms holding 8 per
-  // thread, 47.9 ms holding 12, 36.0 ms holding none).
-  constexpr bool PREF = sizeof(T) == 4 && (MODE == OP_RESID || MODE == OP_SMOOTH) && BLOCK < 1024;
-  constexpr int XC = PREF ? XCHUNK_PREF : XCHUNK;
-  const bool pref = PREF && n_own <= uint32_t(XC * BLOCK);
-  uint32_t own_n[XC];
-  T own_b[XC], own_d[XC];
-  // the other kernels keep the owned nodes' ids from the gather for the store phase (tiles
-  // whose touched nodes fit one gather batch; larger ones reload them), except the Dirichlet
-  // product, whose boundary flags already take it past 64 VGPRs with them
-  constexpr bool KEEP = !PREF && MODE != OP_DIAG && MODE != OP_DIRMV;
-  const bool keep = KEEP && rec.n_touch <= uint32_t(XC * BLOCK);
+  // Gather.  Indexes past the end are clamped to the last node, so a thread's OP_XC id loads,
+  // then its x loads, go out together with no branch between them.  Owned nodes lead the list:
+  // nid[0 .. OP_OC) are also the ids of the store phase.
+  uint32_t nid[OP_XC];
+  const uint32_t last = rec.n_touch - 1u;
+#pragma unroll
+  for (int q = 0; q < OP_XC; ++q) nid[q] = nodes[min(threadIdx.x + uint32_t(q * BLOCK), last)];
+  // FP32 residual and smoothing: the owned nodes' b and invd are loaded with the gather, so the
+  // store phase waits on no global load.  FP64 loads them before the last barrier instead (held
+  // from the gather on, they would take the kernel past the 64 VGPRs of eight wavefronts per
+  // SIMD).  Lanes past the owned nodes load the first node's.
+  constexpr bool RS = MODE == OP_RESID || MODE == OP_SMOOTH;
+  constexpr bool EARLY = RS && sizeof(T) == 4;
+  T own_b[OP_OC], own_d[OP_OC];
+  auto load_own = [&] {
+    const uint32_t n0 = nodes[0];
+#pragma unroll
+    for (int q = 0; q < OP_OC; ++q) {
+      const uint32_t n = threadIdx.x + uint32_t(q * BLOCK) < n_own ? nid[q] : n0;
+      own_b[q] = io.b[n];
+      if (MODE == OP_SMOOTH) own_d[q] = io.invd[n];
+    }
+  };
+  uint32_t own_bdy = 0;   // DIRMV: boundary flags of this thread's owned nodes, one bit each
+  uint32_t xhi = 0;       // high word of max |x| over the values this thread staged
   if (MODE != OP_DIAG) {
-    for (uint32_t base = 0; base < rec.n_touch; base += XC * BLOCK) {
-      uint32_t nid[XC];
-      T v[XC];
+    T v[OP_XC];
 #pragma unroll
-      for (int q = 0; q < XC; ++q) {
-        const uint32_t i = base + threadIdx.x + q * BLOCK;
-        nid[q] = (i < rec.n_touch) ? nodes[i] : 0u;
-      }
-      if (KEEP && base == 0) {
+    for (int q = 0; q < OP_XC; ++q) v[q] = x[nid[q]];
+    if (MODE == OP_DIRMV) {   // flags loaded beside x (both wait on the node ids only)
+      uint8_t bf[OP_XC];
 #pragma unroll
-        for (int q = 0; q < XC; ++q) own_n[q] = nid[q];
-      }
-      if (PREF && base == 0) {
+      for (int q = 0; q < OP_XC; ++q) bf[q] = io.bdy[nid[q]];
 #pragma unroll
-        for (int q = 0; q < XC; ++q) {
-          const uint32_t i = threadIdx.x + q * BLOCK;
-          own_n[q] = nid[q];
-          own_b[q] = (pref && i < n_own) ? io.b[nid[q]] : T(0);
-          own_d[q] = (MODE == OP_SMOOTH && pref && i < n_own) ? io.invd[nid[q]] : T(0);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < XC; ++q) {
-        const uint32_t i = base + threadIdx.x + q * BLOCK;
-        v[q] = (i < rec.n_touch) ? x[nid[q]] : T(0);
-      }
-      if (MODE == OP_DIRMV) {   // flags loaded beside x (both wait on the node ids only)
-        uint8_t bf[XC];
-#pragma unroll
-        for (int q = 0; q < XC; ++q) {
-          const uint32_t i = base + threadIdx.x + q * BLOCK;
-          bf[q] = (i < rec.n_touch) ? io.bdy[nid[q]] : uint8_t(0);
-        }
-#pragma unroll
-        for (int q = 0; q < XC; ++q) v[q] = bf[q] ? T(0) : v[q];
-      }
-#pragma unroll
-      for (int q = 0; q < XC; ++q) {
-        const uint32_t i = base + threadIdx.x + q * BLOCK;
-        if (i < rec.n_touch) xs[i] = v[q];
-        xhi = max(xhi, uint32_t(uint64_t(__double_as_longlong(double(v[q]))) >> 32) & 0x7fffffffu);
+      for (int q = 0; q < OP_XC; ++q) {
+        v[q] = bf[q] ? T(0) : v[q];
+        if (q < OP_OC) own_bdy |= (bf[q] ? 1u : 0u) << q;
       }
     }
+    if (EARLY) load_own();
+#pragma unroll
+    for (int q = 0; q < OP_XC; ++q) {
+      const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+      if (i < rec.n_touch) xs[i] = v[q];
+      if constexpr (sizeof(T) == 8)
+        xhi = max(xhi, uint32_t(uint64_t(__double_as_longlong(v[q])) >> 32) & 0x7fffffffu);
+      else   // the FP32 bits order as |x| does; the maximum is converted once below
+        xhi = max(xhi, __float_as_uint(v[q]) & 0x7fffffffu);
+    }
   }
-  for (uint32_t i = threadIdx.x; i < n_own; i += BLOCK) acc[i] = 0;
+#pragma unroll
+  for (int q = 0; q < OP_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i < n_own) acc[i] = 0;
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) xhi = max(xhi, uint32_t(__shfl_xor(int(xhi), off)));
   if ((threadIdx.x & 63) == 0) s_xhi[threadIdx.x >> 6] = xhi;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NW; ++w) xhi = max(xhi, s_xhi[w]);
+  if constexpr (sizeof(T) == 4)
+    xhi = uint32_t(uint64_t(__double_as_longlong(double(__uint_as_float(xhi)))) >> 32);
   // max |x| < 2^ex; a non-finite x makes every owned output of the tile NaN
   const bool finite = (xhi >> 20) < 0x7ffu;
   const int ex = MODE == OP_DIAG ? 1 : max(int(xhi >> 20) - 1022, FX_XMIN);
   const int es = fx_scale<T>(texp[t], ex);
-  for (uint32_t base = 0;;) {
-    if (base + threadIdx.x < rec.n_elem) {
-      if (LANE)
-        eval_rows_lane<T, MASS, MODE, XS>(R, n_own * uint32_t(sizeof(T)), es, kf);
-      else
-        eval_rows<T, MASS, MODE, XS, COMB>(R, n_own * uint32_t(sizeof(T)), es, KF);
-    }
-    base += BLOCK;
-    if (base >= rec.n_elem) break;
-    if (base + threadIdx.x < rec.n_elem) {   // wave-uniform bases, lane offsets fixed
-      const uint32_t r0 = rec.elem_off + base;
-      load_rec<TC, MASS, sizeof(T), UNI ? 1 : 0, !COMB>(R, threadIdx.x, lid + size_t(r0) * 8,
-                                                 UNI ? kappa : kappa + r0, UNI || !MASS ? mass : mass + r0, lap_fac,
-                                                 mass_fac, maxD, hFac);
-    }
-  }
-  // FP32 residual and smoothing with kept ids: the owned nodes' b and invd are loaded before
-  // the barrier, in flight while the other wavefronts finish their records (8M-point octree,
-  // mixed PCG 35.2 -> 34.7 ms; in FP64 the 24 held values take the 1024-thread kernel past
-  // 64 VGPRs: FP64 PCG 43.9 -> 51.5 ms)
-  constexpr bool BPRE = KEEP && sizeof(T) == 4 && (MODE == OP_RESID || MODE == OP_SMOOTH);
-  if (BPRE && keep) {
-#pragma unroll
-    for (int q = 0; q < XC; ++q) {
-      const uint32_t i = threadIdx.x + q * BLOCK;
-      own_b[q] = i < n_own ? io.b[own_n[q]] : T(0);
-      own_d[q] = (MODE == OP_SMOOTH && i < n_own) ? io.invd[own_n[q]] : T(0);
-    }
-  }
-  __syncthreads();
-  if (PREF && pref) {
-#pragma unroll
-    for (int q = 0; q < XC; ++q) {
-      const uint32_t i = threadIdx.x + q * BLOCK;
-      if (i < n_own) {
-        const T v = finite ? T(fx_value<T>(acc[i], es)) : T(__builtin_nan(""));
-        if (MODE == OP_RESID)
-          io.y[own_n[q]] = own_b[q] - v;
-        else
-          io.y[own_n[q]] = xs[i] + io.omega * ((own_b[q] - v) * own_d[q]);
-      }
-    }
-    return;
-  }
-  double dot = 0.0;
-  for (uint32_t i = threadIdx.x, q = 0; i < n_own; i += BLOCK, ++q) {
-    uint32_t n = 0;
-    if (KEEP && keep) {
-#pragma unroll
-      for (int u = 0; u < XC; ++u) n = (uint32_t(u) == q) ? own_n[u] : n;
+  const uint32_t own_bytes = n_own * uint32_t(sizeof(T));
+  for (uint32_t r0 = w0; r0 < rec.n_elem; r0 += BLOCK) {
+    const bool in = r0 + lane < rec.n_elem;
+    if constexpr (FACT) {   // the next records' loads are in flight during the evaluation
+      decltype(R) Rn;
+      load(Rn, r0 + BLOCK);
+      eval_fact<T, MASS, XS, UNI>(R, in ? own_bytes : 0u, es, lap_fac, mass_fac, maxD);
+      R = Rn;
     } else {
-      n = nodes[i];
+      if (in) {
+        if constexpr (LANE)
+          eval_rows_lane<T, MASS, MODE, XS>(R, own_bytes, es, kf);
+        else
+          eval_rows<T, MASS, MODE, XS, COMB>(R, own_bytes, es, KF);
+      }
+      if (r0 + BLOCK < rec.n_elem) load(R, r0 + BLOCK);
     }
-    const double s = fx_value<T>(acc[i], es);
-    const T v = finite ? T(s) : T(__builtin_nan(""));
+  }
+  if (RS && !EARLY) load_own();   // in flight while the other wavefronts finish their records
+  __syncthreads();
+  double dot = 0.0;
+#pragma unroll
+  for (int q = 0; q < OP_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i >= n_own) break;
+    const uint32_t n = nid[q];
+    const T v = finite ? T(fx_value<T>(acc[i], es)) : T(__builtin_nan(""));
     if (MODE == OP_MATVEC) {
       io.y[n] = v;
     } else if (MODE == OP_DIAG) {   // with boundary flags, the Dirichlet diagonal: 1 there
       io.y[n] = (io.bdy && io.bdy[n]) ? T(1) : v;
     } else if (MODE == OP_DIRMV) {
-      io.y[n] = io.bdy[n] ? x[n] : v;
-    } else if (MODE == OP_RESID || MODE == OP_SMOOTH) {
-      T bn, dn;
-      if (BPRE && keep) {
-        bn = own_b[0];
-        dn = own_d[0];
-#pragma unroll
-        for (int u = 1; u < XC; ++u) {
-          bn = (uint32_t(u) == q) ? own_b[u] : bn;
-          dn = (uint32_t(u) == q) ? own_d[u] : dn;
-        }
-      } else {
-        bn = io.b[n];
-        dn = MODE == OP_SMOOTH ? io.invd[n] : T(0);
-      }
-      if (MODE == OP_RESID)
-        io.y[n] = bn - v;
-      else
-        io.y[n] = xs[i] + io.omega * ((bn - v) * dn);   // owned nodes lead the staged x
+      io.y[n] = (own_bdy >> q) & 1u ? x[n] : v;
+    } else if (MODE == OP_RESID) {
+      io.y[n] = own_b[q] - v;
+    } else if (MODE == OP_SMOOTH) {
+      io.y[n] = xs[i] + io.omega * ((own_b[q] - v) * own_d[q]);   // owned nodes lead the staged x
     } else {
       io.y[n] = v;
       dot += double(xs[i]) * double(v);
