@@ -11,7 +11,11 @@
 
 namespace dgh {
 
-constexpr uint32_t ELAS_TILE = 2048;   // element cap of an elasticity tile (the node budget cuts first)
+// Elements per elasticity tile: the 512 resident workgroups get one tile each as long as a tile has
+// at least 128 elements (below that the halo grows faster than the work spreads: 17k elements 6.8
+// us in tiles of 64, 6.0 of 128, 7.2 of 256) and at most 768 (1.0M elements: 40.2 us in tiles of
+// 512, 38.9 of 768, 42.2 of 2048, which the node budget cuts to about 1100).
+static uint32_t elas_tile_elems(uint32_t n_elem) { return std::min(768u, std::max(128u, n_elem / 512u)); }
 
 // Owner-computes tiling of the elasticity operator (the scalar operator's plan, with 24-byte
 // node slots: a smaller owned-node capacity and node budget) and the records' meta with the
@@ -19,38 +23,32 @@ constexpr uint32_t ELAS_TILE = 2048;   // element cap of an elasticity tile (the
 static void elas_plan(dgh_mesh m) {
   ElasState& S = m->elas;
   if (S.ready) return;
-  build_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), ELAS_TILE, S.plan,
+  build_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), elas_tile_elems(m->E), S.plan,
               ELAS_BUDGET, ELAS_OWN_CAP);
   if (elas_lds_bytes(S.plan.max_touch) > size_t(g.max_lds))
     fail(DGH_ERR_ARG, "elasticity tiles need %zu bytes of LDS (limit %d)", elas_lds_bytes(S.plan.max_touch), g.max_lds);
   const size_t R = S.plan.rec_elem.size();
-  std::vector<uint16_t> meta(R);
-  for (size_t r = 0; r < R; ++r) {   // child-0 hanging mask | child << 8 | level << 11
+  std::vector<uint16_t> rec(S.plan.lid);
+  for (size_t r = 0; r < R; ++r) {
     const uint32_t t = S.plan.meta[r] & 31u, lev = S.plan.meta[r] >> 5;
     if (t >= uint32_t(NSTENCIL) || lev > 31u) fail(DGH_ERR_MESH, "record class out of range");
-    meta[r] = uint16_t(kEtypeMask[0][t] | (uint32_t(m->h_child[S.plan.rec_elem[r]]) << 8) | (lev << 11));
+    elas_pack(&rec[r * 8], kEtypeMask[0][t], m->h_child[S.plan.rec_elem[r]], lev);
   }
   S.tiles.upload(S.plan.tiles.data(), S.plan.tiles.size());
-  S.lid.upload(S.plan.lid.data(), S.plan.lid.size());
-  S.meta.upload(meta.data(), R);
+  S.lid.upload(rec.data(), rec.size());
   S.node_tab.upload(S.plan.node_tab.data(), S.plan.node_tab.size());
   S.ready = true;
 }
 
-// The unit element's matrix K_0 = mu L_0 (x) I + (mu + lambda) GD_0 (child 0, no hanging
-// vertex; elasticityJac.C:171-206 applies fac = h/2 per element), and the per-tile
-// fixed-point bounds from the element matrices fac (mu L (x) I + (mu + lambda) GD) of the
-// (type, level) classes the tiling holds: texp[t].x = e with every row sum of |fac K_t| over
+// The per-tile fixed-point bounds from the element matrices fac (mu L (x) I + (mu + lambda) GD),
+// fac = h/2 (elasticityJac.C:171-206), of the (type, level) classes the tiling holds: texp[t].x = e with every row sum of |fac K_t| over
 // the tile's records below 2^e, texp[t].y = log2 bound of the terms per owned node.
 static void elas_matrices(dgh_mesh m) {
   ElasState& S = m->elas;
   std::vector<double> L(9216), G(size_t(144) * 576);
   generate_stencils(L.data(), nullptr, nullptr, nullptr);
   generate_graddiv(G.data());
-  std::vector<double> k0(576), ke(576), rowmax(NCLASS, 0.0);
-  for (int r = 0; r < 24; ++r)
-    for (int q = 0; q < 24; ++q)
-      k0[r * 24 + q] = S.mu * ((r % 3 == q % 3) ? L[(r / 3) * 8 + q / 3] : 0.0) + (S.mu + S.lam) * G[r * 24 + q];
+  std::vector<double> ke(576), rowmax(NCLASS, 0.0);
   std::vector<uint8_t> seen(NCLASS, 0);
   for (uint16_t c : S.plan.meta) {
     if (seen[c]) continue;
@@ -91,7 +89,6 @@ static void elas_matrices(dgh_mesh m) {
     if (mx > 0.0) std::frexp(mx * FX_MARGIN, &e);
     te[t] = make_int2(std::max(e, -1022), v);
   }
-  S.ke.upload(k0.data(), k0.size());
   S.texp.upload(te.data(), te.size());
 }
 
@@ -125,8 +122,8 @@ int dgh_matvec_elasticity(dgh_mesh m, const double* x, double* y, void* stream) 
       const unsigned grid = unsigned(NXCD * ((nt + NXCD - 1) / NXCD));
       const size_t lds = elas_lds_bytes(S.plan.max_touch);
       hipLaunchKernelGGL(elas_tile_kernel, dim3(grid), dim3(ELAS_BLOCK), lds, st, (const TileRec*)S.tiles.p, nt,
-                         (const uint16_t*)S.lid.p, (const uint16_t*)S.meta.p, (const uint32_t*)S.node_tab.p,
-                         (const int2*)S.texp.p, (const double*)S.ke.p, 0u, m->maxD, m->hFac, (const uint8_t*)m->bdy.p,
+                         (const uint16_t*)S.lid.p, (const uint32_t*)S.node_tab.p,
+                         (const int2*)S.texp.p, elas_modes(S.mu, S.lam), m->maxD, m->hFac, (const uint8_t*)m->bdy.p,
                          x, y);
     }
     HIP_CHECK(hipGetLastError());

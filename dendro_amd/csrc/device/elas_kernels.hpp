@@ -11,14 +11,14 @@
 // Element matrices: child c's element is child 0's with the vertex order k^c (the plan's
 // vertex permutation) and the signs s_a s_b on the (a, b) blocks (s_a = -1 when bit a of c is
 // set: the mirror flips axis a).  Child 0's element of hanging mask H is the regular one
-// constrained by the interpolation P_H of its hanging vertices, K_H = P_H^T K_0 P_H, where
-// row k of P_H is e_k for a regular vertex, (e_0 + e_k)/2 for a hanging edge midpoint
-// (k = 1, 2, 4) and (e_0 + e_a + e_b + e_k)/4 for a hanging face centre (k = a | b =
-// 3, 5, 6); the stencils of the 18 child-0 types are exactly these products (the shape
-// functions interpolate the parent's vertices).  So a lane applies P_H to its (sign-flipped)
-// inputs, the one 24x24 matrix K_0 = mu L_0 (x) I + (mu + lambda) GD_0 of the unit element
-// (every lane the same: wave-uniform rows through the scalar cache, no per-type passes), and
-// P_H^T to the result, and scales by its element's fac = h/2.
+// constrained by the interpolation P_H of its hanging vertices, K_H = P_H^T K_0 P_H (kernels.hpp).
+// K_0 is applied in the Walsh-Hadamard modes of its three components (bit a of a mode: difference
+// along axis a): the Laplacian and the (a, a) blocks are diagonal there, and the (a, b) block,
+// d_a phi_k d_b phi_j, is one entry per pair of modes, from mode n ^ a ^ b (bit a clear, bit b
+// set) of component b to mode n (bit a set, bit b clear) of component a: 24 + 12 products and
+// 144 additions instead of 576 FMAs with the matrix rows read through the scalar cache.  Every
+// lane uses the same seven constants (ElasModes), whatever its element's type; the mirror signs
+// fall on the 12 coupling products only, and the element's size on the final conversion.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,42 +28,86 @@
 
 namespace dgh {
 
-constexpr int ELAS_ROWS = 24;
 constexpr int ELAS_NSTRIDE = 24;   // LDS bytes per node: three doubles (sums or staged x)
-constexpr int ELAS_XCHUNK = 4;     // node gathers per thread in flight together
 
 // Threads per tile, owned-node capacity and node budget (owned capacity + touched nodes) of an
-// elasticity tile: the kernel's registers (about 160 VGPRs) allow three 256-thread workgroups
-// per CU, and the budget gives each the LDS of a third of a CU (24 B per node slot).  On the
-// 2M-element log-normal octree: 659 us per product for a two-pass (element outputs to HBM,
-// node gather) version, 387 us for per-(type, level) 24x24 class matrices, 234 us for the
-// P_H^T K_0 P_H form with 512-thread tiles of 1680 node slots, 182 us with 256 threads and
-// 170 us with this budget.
-constexpr int ELAS_BLOCK = 256;
-constexpr uint32_t ELAS_OWN_CAP = 640u;
-constexpr uint32_t ELAS_BUDGET = 2200u;
+// elasticity tile: 128 registers allow 16 wavefronts per CU, as two 512-thread workgroups with
+// half a CU's LDS each (24 B per node slot).  Products of 17k / 90k / 318k / 1.0M elements, tiles of
+// elas_tile_elems: 6.0 / 8.7 / 18.4 / 38.9 us; with 256 threads and a quarter of the LDS 7.1 / 8.9 /
+// 19.7 / 39.9.  Before (24x24 matrix rows, 256 threads, 2200 slots) 37.7 / 37.9 / 61.9 / 106 us.
+// It is bound by its 48 LDS operations per record (about 530 cycles per 64 records and CU: 20 us
+// at 1.0M elements) and, at as much again, by its vector instructions.
+constexpr int ELAS_BLOCK = 512;
+constexpr uint32_t ELAS_OWN_CAP = 1024u;
+constexpr uint32_t ELAS_BUDGET = 3360u;
+// touched and owned nodes per thread
+constexpr int ELAS_XC = int((ELAS_BUDGET - ELAS_OWN_CAP + ELAS_BLOCK - 1) / ELAS_BLOCK);
+constexpr int ELAS_OC = int((ELAS_OWN_CAP + ELAS_BLOCK - 1) / ELAS_BLOCK);
 constexpr uint32_t ELAS_XS_OFF = ELAS_NSTRIDE * ELAS_OWN_CAP + 64u;
 __host__ constexpr size_t elas_lds_bytes(uint32_t max_touch) {
   return size_t(ELAS_XS_OFF) + size_t(ELAS_NSTRIDE) * max_touch;
 }
 
-// The unit matrix is read through the constant address space: uniform loads from it are
-// scalar loads whatever the address arithmetic.
-template <class U>
-using const_ptr = const __attribute__((address_space(4))) U*;
-
-__device__ __forceinline__ double flip_sign(double v, uint32_t neg) {
-  return __longlong_as_double(__double_as_longlong(v) ^ (static_cast<long long>(neg) << 63));
+// K_0 = mu L + (mu + lambda) GD of the unit-size element over its modes (factor 1/8 of the
+// inverse transform included): d0[p], d1[p] = the diagonal of component a at a mode of p
+// difference axes with bit a clear / set; o[bit] = the coupling with third axis sum / difference.
+struct ElasModes {
+  double d0[4], d1[4], o[2];
+};
+__host__ inline ElasModes elas_modes(double mu, double lam) {
+  ElasModes m{};
+  for (int p = 1; p <= 3; ++p) {
+    double c = 2.0 / 8.0;   // 2 (1/6)^(p-1) (1/2)^(3-p) / 8
+    for (int i = 1; i < p; ++i) c /= 6.0;
+    for (int i = p; i < 3; ++i) c /= 2.0;
+    m.d0[p] = mu * p * c;
+    m.d1[p] = mu * p * c + (mu + lam) * c;
+  }
+  m.o[0] = (mu + lam) / 16.0;
+  m.o[1] = (mu + lam) / 48.0;
+  return m;
 }
 
-// meta: child-0 hanging mask | child << 8 | level << 11.  K0: the unit element's [24][24]
-// (rows 3k + a); kzero: 0.  texp[t]: exponent bound of the tile's row sums of |fac K_H| and log2 bound of
-// the terms per node (as for the scalar operator).
+// v with its sign flipped by bit 31 of s
+__device__ __forceinline__ double flip_sign(double v, uint32_t s) {
+  return __longlong_as_double(__double_as_longlong(v) ^ (static_cast<long long>(s & 0x80000000u) << 32));
+}
+
+// v <- W v
+__device__ __forceinline__ void wht8(double v[8]) {
+#pragma unroll
+  for (int b = 1; b < 8; b <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & b)) {
+        const double s = v[i] + v[i | b];
+        v[i | b] = v[i] - v[i | b];
+        v[i] = s;
+      }
+}
+
+// A record: 8 tile-local vertex ids in 14 bits, its hanging vertices in the top bits of ids 5..7
+// (rec_hang), the mirror signs s_x s_y, s_y s_z, s_z s_x in bits 14, 15 and 30 of the first word,
+// the level's low four bits in the second word's spare bits and its fifth in bit 31 of the first.
+__host__ inline void elas_pack(uint16_t id[8], uint32_t mask, uint32_t child, uint32_t lev) {
+  const uint32_t hb = hang_bits(mask);
+  const uint32_t sg = ((child ^ (child >> 1)) & 1u) | ((((child >> 1) ^ (child >> 2)) & 1u) << 1) |
+                      (((child >> 2) ^ child) & 1u) << 2;
+  const uint32_t top[8] = {sg & 3u, (sg >> 2) | ((lev >> 4) << 1), lev & 3u, (lev >> 2) & 3u, 0u,
+                           hb & 3u, (hb >> 2) & 3u, (hb >> 4) & 3u};
+  for (int q = 0; q < 8; ++q) id[q] = uint16_t(id[q] | (top[q] << 14));
+}
+__device__ __forceinline__ uint32_t elas_level(uint4 lp) {
+  return ((lp.y >> 14) & 3u) | ((lp.y >> 28) & 12u) | ((lp.x >> 27) & 16u);
+}
+
+// texp[t]: exponent bound of the tile's
+// row sums of |h K_H| and log2 bound of the terms per node (as for the scalar operator).
 __global__ void __launch_bounds__(ELAS_BLOCK)
 elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* __restrict__ lid,
-                 const uint16_t* __restrict__ meta, const uint32_t* __restrict__ node_tab,
-                 const int2* __restrict__ texp, const double* __restrict__ K0, uint32_t kzero, uint32_t maxD,
-                 double hFac, const uint8_t* __restrict__ bdy, const double* __restrict__ x, double* __restrict__ y) {
+                 const uint32_t* __restrict__ node_tab,
+                 const int2* __restrict__ texp, ElasModes md, uint32_t maxD, double hFac,
+                 const uint8_t* __restrict__ bdy, const double* __restrict__ x, double* __restrict__ y) {
   constexpr int BLOCK = ELAS_BLOCK;
   constexpr int NW = BLOCK / 64;
   constexpr uint32_t XS = ELAS_XS_OFF;
@@ -75,46 +119,41 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
   const TileRec rec = tiles[t];
   const uint32_t* nodes = node_tab + rec.node_off;
   const uint32_t n_own = rec.n_own;
-  uint4 lp = make_uint4(0, 0, 0, 0);
-  uint32_t mt = 0;
-  if (threadIdx.x < rec.n_elem) {
-    lp = reinterpret_cast<const uint4*>(lid)[rec.elem_off + threadIdx.x];
-    mt = meta[rec.elem_off + threadIdx.x];
+  // the wavefront's records: w0, w0 + BLOCK, ...; lanes past the last record load it again and
+  // add nothing
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t w0 = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x - lane)));
+  auto load = [&](uint32_t r0) {
+    return reinterpret_cast<const uint4*>(lid)[rec.elem_off + min(r0 + lane, rec.n_elem - 1u)];
+  };
+  uint4 lp = load(w0);
+  // stage the touched nodes' x (boundary nodes as 0: their columns drop out); indexes past the
+  // end are clamped, so that all loads go out together
+  uint32_t nid[ELAS_XC];
+  const uint32_t last = rec.n_touch - 1u;
+#pragma unroll
+  for (int q = 0; q < ELAS_XC; ++q) nid[q] = nodes[min(threadIdx.x + uint32_t(q * BLOCK), last)];
+  uint32_t xhi = 0, own_bdy = 0;
+  double v[ELAS_XC][3];
+#pragma unroll
+  for (int q = 0; q < ELAS_XC; ++q)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) v[q][a] = x[3 * size_t(nid[q]) + a];
+  if (bdy) {
+#pragma unroll
+    for (int q = 0; q < ELAS_XC; ++q)
+      if (bdy[nid[q]]) {
+        v[q][0] = v[q][1] = v[q][2] = 0.0;
+        own_bdy |= 1u << q;
+      }
   }
-  // stage the touched nodes' x (boundary nodes as 0: their columns drop out)
-  uint32_t xhi = 0;
-  for (uint32_t base = 0; base < rec.n_touch; base += ELAS_XCHUNK * BLOCK) {
-    uint32_t nid[ELAS_XCHUNK];
 #pragma unroll
-    for (int q = 0; q < ELAS_XCHUNK; ++q) {
-      const uint32_t i = base + threadIdx.x + q * BLOCK;
-      nid[q] = (i < rec.n_touch) ? nodes[i] : 0u;
-    }
-    double v[ELAS_XCHUNK][3];
+  for (int q = 0; q < ELAS_XC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
 #pragma unroll
-    for (int q = 0; q < ELAS_XCHUNK; ++q) {
-      const uint32_t i = base + threadIdx.x + q * BLOCK;
-      const bool in = i < rec.n_touch;
-#pragma unroll
-      for (int a = 0; a < 3; ++a) v[q][a] = in ? x[3 * size_t(nid[q]) + a] : 0.0;
-    }
-    if (bdy) {
-#pragma unroll
-      for (int q = 0; q < ELAS_XCHUNK; ++q) {
-        const uint32_t i = base + threadIdx.x + q * BLOCK;
-        if (i < rec.n_touch && bdy[nid[q]]) v[q][0] = v[q][1] = v[q][2] = 0.0;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < ELAS_XCHUNK; ++q) {
-      const uint32_t i = base + threadIdx.x + q * BLOCK;
-      if (i < rec.n_touch) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) *lds_at<double>(XS + ELAS_NSTRIDE * i + 8u * a) = v[q][a];
-      }
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-        xhi = max(xhi, uint32_t(uint64_t(__double_as_longlong(v[q][a])) >> 32) & 0x7fffffffu);
+    for (int a = 0; a < 3; ++a) {
+      if (i < rec.n_touch) *lds_at<double>(XS + ELAS_NSTRIDE * i + 8u * a) = v[q][a];
+      xhi = max(xhi, uint32_t(uint64_t(__double_as_longlong(v[q][a])) >> 32) & 0x7fffffffu);
     }
   }
   for (uint32_t i = threadIdx.x; i < 3 * n_own; i += BLOCK) lds_at<unsigned long long>(0)[i] = 0ull;
@@ -128,96 +167,81 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
   const int ex = max(int(xhi >> 20) - 1022, FX_XMIN);
   const int es = fx_scale<double>(texp[t], ex);
   const uint32_t own_bytes = n_own * ELAS_NSTRIDE;
-  for (uint32_t base = 0;;) {
-    if (base + threadIdx.x < rec.n_elem) {
-      uint32_t l[8];
-      l[0] = (lp.x & 0xffffu) * ELAS_NSTRIDE; l[1] = (lp.x >> 16) * ELAS_NSTRIDE;
-      l[2] = (lp.y & 0xffffu) * ELAS_NSTRIDE; l[3] = (lp.y >> 16) * ELAS_NSTRIDE;
-      l[4] = (lp.z & 0xffffu) * ELAS_NSTRIDE; l[5] = (lp.z >> 16) * ELAS_NSTRIDE;
-      l[6] = (lp.w & 0xffffu) * ELAS_NSTRIDE; l[7] = (lp.w >> 16) * ELAS_NSTRIDE;
-      const uint32_t hm = mt & 0xffu, c = (mt >> 8) & 7u, lev = mt >> 11;
-      const uint32_t neg[3] = {c & 1u, (c >> 1) & 1u, (c >> 2) & 1u};
-      // the element's fac = h/2 and 2^es in one scale per component (with the mirror sign)
-      const double sc = ldexp(hFac * double(1u << (maxD - lev)) / 2.0, es);
-      const double sa[3] = {flip_sign(sc, neg[0]), flip_sign(sc, neg[1]), flip_sign(sc, neg[2])};
-      double xe[ELAS_ROWS];
+  double quarter = 0.25;
+  asm("" : "+s"(quarter));
+  for (uint32_t r0 = w0; r0 < rec.n_elem; r0 += BLOCK) {
+    const uint4 lpn = load(r0 + BLOCK);   // in flight during the evaluation
+    const uint32_t w[4] = {lp.x, lp.y, lp.z, lp.w};
+    uint32_t l[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
+    for (int j = 0; j < 8; ++j) l[j] = ((w[j >> 1] >> (16 * (j & 1))) & REC_ID_MASK) * ELAS_NSTRIDE;
+    const uint32_t hb = rec_hang(lp);
+    // one component after the other (the fences keep the three from being interleaved, which
+    // takes 138 registers instead of 128)
+    double xe[3][8];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) xe[3 * k + a] = flip_sign(*lds_at<double>(XS + l[k] + 8u * a), neg[a]);
-      // per hanging vertex k: c_k = the weight of x_k in x'_k, d_k = the weight of each other
-      // value in it (edge k = 1, 2, 4: (x_0 + x_k)/2; face k = 3, 5, 6: (x_0 + x_a + x_b + x_k)/4)
-      double ck[7], dk[7];
+    for (int a = 0; a < 3; ++a) {
 #pragma unroll
-      for (int k = 1; k < 7; ++k) {
-        const bool h = (hm >> k) & 1u;
-        const double w = (k == 3 || k == 5 || k == 6) ? 0.25 : 0.5;
-        ck[k] = h ? w : 1.0;
-        dk[k] = h ? w : 0.0;
-      }
-      // x' = P_H x (faces first: they read the raw values of the edge vertices)
+      for (int k = 0; k < 8; ++k) xe[a][k] = *lds_at<double>(XS + l[k] + 8u * a);
+      hang_interp(xe[a], hb, quarter);
+      wht8(xe[a]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const uint32_t sg[3] = {lp.x << 17, lp.x << 16, lp.x << 1};   // mirror signs of (x,y), (y,z), (z,x)
+    // modes, in place
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const double x0 = xe[a], x1 = xe[3 + a], x2 = xe[6 + a], x4 = xe[12 + a];
-        xe[9 + a] = ck[3] * xe[9 + a] + dk[3] * ((x0 + x1) + x2);
-        xe[15 + a] = ck[5] * xe[15 + a] + dk[5] * ((x0 + x1) + x4);
-        xe[18 + a] = ck[6] * xe[18 + a] + dk[6] * ((x0 + x2) + x4);
-        xe[3 + a] = ck[1] * x1 + dk[1] * x0;
-        xe[6 + a] = ck[2] * x2 + dk[2] * x0;
-        xe[12 + a] = ck[4] * x4 + dk[4] * x0;
-      }
-      // y = P_H^T K_0 x', one row of K_0 at a time: row (k, a) of z = K_0 x' goes to y_k with
-      // weight c_k and to vertex 0 (and, for a face, its two edge vertices) with weight d_k.
-      // kzero is 0: each row's address formally depends on the round and on the previous
-      // row's first entry, so the compiler neither hoists the (loop-invariant) row loads out
-      // of the record loop nor issues them all at once (576 values, far more than the scalar
-      // registers would hold): the rows are read one after the other through the scalar cache.
-      const const_ptr<double> Kr0 = (const_ptr<double>)(K0 + size_t(kzero * __builtin_amdgcn_readfirstlane(base)));
-      const_ptr<double> Kr = Kr0;
-      double yv[ELAS_ROWS];
+    for (int a = 0; a < 3; ++a) {
+      const int A = 1 << a, B = 1 << (a + 1) % 3, C = 1 << (a + 2) % 3;
+      xe[a][B] *= md.d0[1];
+      xe[a][C] *= md.d0[1];
+      xe[a][B | C] *= md.d0[2];
+      xe[a][7] *= md.d1[3];
+      // (a, A|C) and (b, B|C): third axis c, difference; the mirror's sign s_a s_b
+      const int b = (a + 1) % 3;
+      const double o = flip_sign(md.o[1], sg[a]);
+      const double u = xe[a][A | C], v2 = xe[b][B | C];
+      xe[a][A | C] = md.d1[2] * u + o * v2;
+      xe[b][B | C] = md.d1[2] * v2 + o * u;
+    }
+    {   // (x, 1), (y, 2), (z, 4): third axis sum
+      const double oxy = flip_sign(md.o[0], sg[0]), oyz = flip_sign(md.o[0], sg[1]), ozx = flip_sign(md.o[0], sg[2]);
+      const double u = xe[0][1], v2 = xe[1][2], z = xe[2][4];
+      xe[0][1] = md.d1[1] * u + (oxy * v2 + ozx * z);
+      xe[1][2] = md.d1[1] * v2 + (oxy * u + oyz * z);
+      xe[2][4] = md.d1[1] * z + (ozx * u + oyz * v2);
+    }
+    // the element's size h and 2^es in one scale
+    const double sc = ldexp(hFac, int(maxD - elas_level(lp)) + es);
+    const uint32_t own = r0 + lane < rec.n_elem ? own_bytes : 0u;
 #pragma unroll
-      for (int r = 0; r < ELAS_ROWS; ++r) yv[r] = 0.0;
+    for (int a = 0; a < 3; ++a) {
+      double* y8 = xe[a];
+      y8[0] = y8[1];   // first step of the inverse transform: the mean mode is zero
+      y8[1] = -y8[1];
 #pragma unroll
-      for (int r = 0; r < ELAS_ROWS; ++r) {
-        double kr[ELAS_ROWS];
+      for (int b = 1; b < 8; b <<= 1)
 #pragma unroll
-        for (int q = 0; q < ELAS_ROWS; ++q) kr[q] = Kr[q];
-        Kr += ELAS_ROWS + size_t(kzero * uint32_t(__builtin_amdgcn_readfirstlane(int(__double_as_longlong(kr[0])))));
-        double zr = kr[0] * xe[0];
-#pragma unroll
-        for (int q = 1; q < ELAS_ROWS; ++q) zr += kr[q] * xe[q];
-        const int k = r / 3, a = r % 3;
-        if (k == 0 || k == 7) {
-          yv[r] += zr;
-        } else {
-          yv[r] += ck[k] * zr;
-          yv[a] += dk[k] * zr;
-          if (k == 3 || k == 5 || k == 6) {
-            const int e1 = k & -k, e2 = k & (k - 1);
-            yv[3 * e1 + a] += dk[k] * zr;
-            yv[3 * e2 + a] += dk[k] * zr;
+        for (int i = b == 1 ? 2 : 0; i < 8; ++i)
+          if (!(i & b)) {
+            const double s = y8[i] + y8[i | b];
+            y8[i | b] = y8[i] - y8[i | b];
+            y8[i] = s;
           }
-        }
-      }
+      hang_interp_t(xe[a], hb, quarter);
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (l[k] < own_bytes) {
-#pragma unroll
-          for (int a = 0; a < 3; ++a)
-            lds_add(lds_at<unsigned long long>(l[k] + 8u * a), fx_term(yv[3 * k + a], sa[a], 0.0, 0.0, false));
-        }
+        if (l[k] < own) lds_add(lds_at<unsigned long long>(l[k] + 8u * a), fx_round_fma(y8[k], sc));
+      __builtin_amdgcn_sched_barrier(0);
     }
-    base += BLOCK;
-    if (base >= rec.n_elem) break;
-    if (base + threadIdx.x < rec.n_elem) {
-      lp = reinterpret_cast<const uint4*>(lid)[rec.elem_off + base + threadIdx.x];
-      mt = meta[rec.elem_off + base + threadIdx.x];
-    }
+    lp = lpn;
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n_own; i += BLOCK) {
-    const uint32_t n = nodes[i];
-    const bool b = bdy && bdy[n];
+#pragma unroll
+  for (int q = 0; q < ELAS_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i >= n_own) break;
+    const uint32_t n = nid[q];
+    const bool b = (own_bdy >> q) & 1u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const double s = fx_value<double>(lds_at<unsigned long long>(0)[3 * i + a], es);

@@ -132,17 +132,15 @@ struct DevTiles {
 
 namespace dgh {
 // Elasticity operator plan of a mesh (elas_api.hip): owner-computes tiles with 24-byte node
-// slots, records' meta (child-0 hanging mask, child, level), per-tile fixed-point bounds and
-// the unit element's 24x24 matrix of the current Lame parameters.
+// slots, records with their hanging vertices, mirror signs and level, and per-tile fixed-point bounds.
 struct ElasState {
   bool ready = false;
   double mu = 1.0, lam = 1.0;
   TilePlan plan;
   DevBuf<TileRec> tiles;
-  DevBuf<uint16_t> lid, meta;   // meta: child-0 hanging mask | child << 8 | level << 11
+  DevBuf<uint16_t> lid;         // records (elas_pack)
   DevBuf<uint32_t> node_tab;
   DevBuf<int2> texp;
-  DevBuf<double> ke;            // K_0 [24][24]
 };
 }  // namespace dgh
 

@@ -525,6 +525,12 @@ __device__ __forceinline__ unsigned long long fx_round(double v) {
   const uint32_t hi = uint32_t(b >> 32) - uint32_t(FX_MAGIC_BITS >> 32);
   return (static_cast<unsigned long long>(hi) << 32) | uint32_t(b);
 }
+// the same of v * sc, rounded once
+__device__ __forceinline__ unsigned long long fx_round_fma(double v, double sc) {
+  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(__builtin_fma(v, sc, FX_MAGIC)));
+  const uint32_t hi = uint32_t(b >> 32) - uint32_t(FX_MAGIC_BITS >> 32);
+  return (static_cast<unsigned long long>(hi) << 32) | uint32_t(b);
+}
 __device__ __forceinline__ unsigned int fx_round(float v) {
   return static_cast<unsigned int>(__float2int_rn(v));
 }

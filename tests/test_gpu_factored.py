@@ -63,3 +63,26 @@ def test_factored_product(dev, mesh, coef):
     xt[L.n_node // 2] = float("inf")
     m.matvec(xt, y, prec=da.F32)
     assert torch.isnan(y[L.n_node // 2])
+
+
+@pytest.mark.parametrize("dirichlet", [False, True])
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+def test_factored_elasticity(dev, mesh, dirichlet):
+    h = hierarchy(*MESHES[mesh], 1, seed=6, min_coarse=1)
+    L = h.fine
+    bdy = h.damg.boundary(0) if dirichlet else None
+    x = np.random.default_rng(9).uniform(-1, 1, (L.n_node, 3))
+    m = da.Mesh(L)
+    m.set_boundary(bdy)
+    xt = torch.tensor(x, device=dev)
+    y = torch.empty_like(xt)
+    for mu, lam in ((1.0, 1.5), (0.7, -0.3)):
+        m.set_elasticity(mu, lam)
+        m.matvec_elasticity(xt, y)
+        ref = oracle.matvec_elasticity(L, x, mu, lam, bdy).reshape(-1, 3)
+        got = y.cpu().numpy()
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        print(f"{mesh} mu {mu} lambda {lam}: {err:.2e}")
+        assert err <= 1e-12
+        if dirichlet:
+            assert np.array_equal(got[bdy != 0], x[bdy != 0])
