@@ -32,9 +32,10 @@ static size_t op_lds_bytes(const dgh_mesh m) {
 }
 
 // Stencil-row source of a launch: class matrices need uniform coefficients (per-element ones
-// fall back to the per-type rows).
+// fall back to the per-type rows) and their own choice (until a source is set, only the diagonal
+// reads rows, and takes the per-type ones).
 static int op_rows_mode(const dgh_mesh m) {
-  return (m->lane_rows == DGH_ROWS_CLASS && m->op.rk64.p) ? DGH_ROWS_TYPE : m->lane_rows;
+  return (m->lane_rows == DGH_ROWS_CLASS && (m->op.rk64.p || m->rows_auto)) ? DGH_ROWS_TYPE : m->lane_rows;
 }
 
 // Whether the products run factored (no stencil rows): unless a row source was chosen.
@@ -202,6 +203,31 @@ static void launch_jac3(dgh_transfer t, const T* x, T* y, T* vf, T* wf, hipStrea
   launch_restrict<T>(t, wf, y, st);
 }
 
+// Uniform coefficients with DGH_ROWS_CLASS chosen: the element matrices K = fac1 L + fac2 M of the
+// operator tiling's record classes, with the factors elem_factors forms (each entry rounded once).
+// 768 KB per mesh, so built for that choice only.
+static void class_rows(dgh_mesh m) {
+  DevTiles& d = m->op;
+  d.kc64.release();
+  d.kc32.release();
+  if (m->rows_auto || m->lane_rows != DGH_ROWS_CLASS || !m->h_kappa.empty()) return;
+  std::vector<double> kc(size_t(NCLASS) * 64, 0.0);
+  std::vector<uint8_t> seen(NCLASS, 0);
+  for (size_t r = 0; r < d.plan.rec_elem.size(); ++r) {
+    const uint32_t c = d.plan.meta[r];
+    if (c >= uint32_t(NCLASS)) fail(DGH_ERR_MESH, "record class %u out of range", c);
+    if (seen[c]) continue;
+    seen[c] = 1;
+    const double h = m->hFac * double(1u << (m->maxD - (c >> 5)));
+    const double f1 = m->lap_fac * h / 2.0, f2 = m->mass_fac * h * h * h / 8.0;
+    const double* KF = g.hKF.data() + size_t(c & 31u) * KFSTRIDE;
+    for (int q = 0; q < 64; ++q) kc[size_t(c) * 64 + q] = f1 * KF[q] + f2 * KF[64 + q];
+  }
+  d.kc64.upload(kc.data(), kc.size());
+  std::vector<float> kcf(kc.begin(), kc.end());
+  d.kc32.upload(kcf.data(), kcf.size());
+}
+
 // Per-record element factors of a tiling (they follow its record order), and the per-tile
 // bounds of the fixed-point sums: texp[t].x = e with
 //   |fac1| max_k sum_j |L_t[k][j]| + |fac2| max_k sum_j |M_t[k][j]| < 2^e
@@ -243,26 +269,8 @@ void upload_coefs(dgh_mesh m, DevTiles& d) {
     te[t] = make_int2(std::max(e, -1022), v);
   }
   d.texp.upload(te.data(), te.size());
-  d.kc64.release();
-  d.kc32.release();
   if (!per_elem) {
-    // element matrices per record class, K = fac1 L + fac2 M with the factors elem_factors
-    // forms (each entry rounded once)
-    std::vector<double> kc(size_t(NCLASS) * 64, 0.0);
-    std::vector<uint8_t> seen(NCLASS, 0);
-    for (size_t r = 0; r < R; ++r) {
-      const uint32_t c = d.plan.meta[r];
-      if (c >= uint32_t(NCLASS)) fail(DGH_ERR_MESH, "record class %u out of range", c);
-      if (seen[c]) continue;
-      seen[c] = 1;
-      const double h = m->hFac * double(1u << (m->maxD - (c >> 5)));
-      const double f1 = m->lap_fac * h / 2.0, f2 = m->mass_fac * h * h * h / 8.0;
-      const double* KF = g.hKF.data() + size_t(c & 31u) * KFSTRIDE;
-      for (int q = 0; q < 64; ++q) kc[size_t(c) * 64 + q] = f1 * KF[q] + f2 * KF[64 + q];
-    }
-    d.kc64.upload(kc.data(), kc.size());
-    std::vector<float> kcf(kc.begin(), kc.end());
-    d.kc32.upload(kcf.data(), kcf.size());
+    if (&d == &m->op) class_rows(m);
     return;
   }
   std::vector<double> k(R);
@@ -337,6 +345,31 @@ static size_t op_lds_f64(const DevTiles& d) { return d.lds64; }
 static uint32_t op_budget(int block) {
   const int per_cu = std::max(1, 2048 / block);
   return uint32_t((OP_LDS_PER_CU / per_cu - 512) / 8);
+}
+
+// Elements and threads per tile of a mesh of E elements until dgh_mesh_set_tile or the autotuner
+// choose others.  FP64 / FP32 products, us, at the line's sides:
+//  - below 98k elements tiles of E/256, 64 to 192 elements, on 512 threads: the launch takes about 4
+//    us whatever the tile, and one pass over the records per thread finishes it (9.4k elements
+//    4.2 / 4.0 in tiles of 64, 9.6 / 8.4 of 2048; 37k 4.9 / 4.6 of 192, 10.4 / 8.9 of 2048);
+//  - up to 1.2M elements one tile of E/512 for each of 512 workgroups, at most half the slots of
+//    512-thread workgroups (297k: 8.9 / 7.3 in tiles of 512, 10.8 / 9.1 of 2048, 12.5 / 9.8 of 128,
+//    whose halo records outnumber their own; 630k: 11.8 / 9.1 of 1024, 13.4 / 10.6 of 2048);
+//  - above, 1024 threads and whole rounds of the 512 workgroup slots with a few to spare, since
+//    the node budget cuts some tiles short (2.0M elements: 23.2 / 17.7 in 511 tiles, 24.6 / 18.9 in
+//    975 of 512 threads, 31.4 / 23.5 in 328; 2.1M: 25.9 in 512 tiles, 29.5 in 513);
+//  - from 4M elements at most 8192 elements, which the node budget cuts to about 5500 (10.5M:
+//    92 / 68 against 95 / 74 in tiles of 4160 on either block; 5.5M 49.9 / 37.7, 2048 x 512 52.0 / 39.4).
+static void default_tiling(uint32_t E, uint32_t& T, int& block) {
+  block = E >= MID_MESH_ELEMS ? 1024 : 512;
+  if (E >= LARGE_MESH_ELEMS) {
+    T = 8192;
+  } else if (E >= MID_MESH_ELEMS) {
+    const uint32_t round = 496u, rounds = (E + round * 4400u - 1u) / (round * 4400u);
+    T = E / (round * rounds);
+  } else {
+    T = std::max(std::min(192u, std::max(64u, E / 256u)), E / 512u);
+  }
 }
 
 // (Re)builds the single right-hand-side tiling with tiles of at most T elements within the
@@ -914,13 +947,9 @@ int dgh_mesh_create(uint32_t n_elem, uint32_t n_node, uint32_t max_depth, const 
     m->h_lev.assign(lev, lev + n_elem);
     m->nl.upload(m->h_nl.data(), m->h_nl.size());
     m->cs.upload(m->h_cs.data(), n_elem);
-    // default tiling: larger tiles (fewer halo records) where the tiles still fill the device
-    if (n_elem >= LARGE_MESH_ELEMS) {
-      m->block = 1024;
-      plan_mesh(m.get(), 8192);
-    } else {
-      plan_mesh(m.get(), 2048);
-    }
+    uint32_t T = 0;
+    default_tiling(n_elem, T, m->block);
+    plan_mesh(m.get(), T);
     *out = m.release();
   });
 }
@@ -946,6 +975,7 @@ int dgh_mesh_set_lane_stencils(dgh_mesh m, int on) {
     ++m->gen;   // captured graphs hold the kernel choice
     m->lane_rows = on;
     m->rows_auto = false;
+    if (on == DGH_ROWS_CLASS && !m->op.kc64.p) class_rows(m);
   });
 }
 

@@ -63,12 +63,12 @@ static inline unsigned blocks_for(size_t n, int bs = VBLOCK) { return unsigned((
 
 // ---------------------------------------------------------------- library state
 constexpr int OP_LDS_PER_CU = 160 * 1024;   // LDS of one CU (gfx950)
-// Default stencil-row source: the class matrices from this many tiles up (four workgroups per
-// CU); on fewer tiles the launch is latency-bound and the fewer passes of per-type rows win.
+// Row source reported until one is set: class matrices from this many tiles up (among the row
+// forms the faster one there; on fewer tiles the fewer passes of per-type rows win).
 constexpr size_t CLASS_ROWS_MIN_TILES = 1024;
-// Meshes of at least this many elements are tiled by default with at most 8192 elements and
-// 1024 threads per tile (1.28 records per element on the 44M- and 21M-element finest levels
-// of the 8M and 4M point octrees, 8-9% faster than 2048/4096 x 512), smaller ones with 2048 x 512.
+// Default tiling of the single right-hand-side operator (default_tiling): from MID_MESH_ELEMS up
+// 1024-thread tiles, from LARGE_MESH_ELEMS up of at most 8192 elements.
+constexpr uint32_t MID_MESH_ELEMS = 1200000;
 constexpr uint32_t LARGE_MESH_ELEMS = 4000000;
 // Largest coarsest level solved with a dense inverse (n^2 doubles on the host and the device).
 constexpr int COARSE_DENSE_LIMIT = 40000;
@@ -122,8 +122,8 @@ struct DevTiles {
   DevBuf<double> rk64, rm64;    // per-record element factors (kappa h / 2, mass h^3 / 8)
   DevBuf<float> rk32, rm32;
   DevBuf<int2> texp;            // per tile: exponent bound of the contributions, log2 bound of the terms per node
-  // uniform coefficients: the element matrices fac1 L + fac2 M of every record class
-  // (child-0 type | level << 5), [NCLASS][64], rows of the classes the tiling holds
+  // uniform coefficients with class rows chosen: the element matrices fac1 L + fac2 M of every
+  // record class (child-0 type | level << 5), [NCLASS][64], rows of the classes the tiling holds
   DevBuf<double> kc64;
   DevBuf<float> kc32;
 };

@@ -96,16 +96,36 @@ void tile_bounds(uint32_t E, uint32_t N, const uint32_t* nl, uint32_t T, uint32_
   bounds.push_back(E);
 }
 
+static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                              const uint8_t* lev, const std::vector<uint32_t>& bounds, TilePlan& plan);
+
 void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                  const uint8_t* lev, uint32_t T, TilePlan& plan, uint32_t budget, uint32_t own_cap) {
   if (T < 64 || T > 16384) fail(DGH_ERR_ARG, "tile size %u out of range [64,16384]", T);
   if (own_cap && own_cap >= budget) fail(DGH_ERR_ARG, "owned-node capacity %u not below the budget %u", own_cap, budget);
-  plan = TilePlan();
-  plan.tile_elems = T;
-  plan.budget = budget;
-  plan.own_cap = own_cap;
+  auto build = [&](const std::vector<uint32_t>& bounds) {
+    plan = TilePlan();
+    plan.tile_elems = T;
+    plan.budget = budget;
+    plan.own_cap = own_cap;
+    build_from_bounds(E, N, nl, child, hn, lev, bounds, plan);
+  };
   std::vector<uint32_t> bounds;
+  // Tiles far below the budget are cut at T elements and checked afterwards: where none exceeds
+  // its capacities the greedy cut is the same one (it ends a tile early only when its next element
+  // would exceed them), and its node adjacency is most of the planning time (318k elements: 40 of
+  // 60 ms).
+  if (own_cap && T <= (budget - own_cap) / 2) {
+    tile_bounds(E, N, nl, T, 0, bounds, 0);
+    build(bounds);
+    if (plan.max_own <= own_cap && plan.max_touch <= budget - own_cap) return;
+  }
   tile_bounds(E, N, nl, T, budget, bounds, own_cap);
+  build(bounds);
+}
+
+static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                              const uint8_t* lev, const std::vector<uint32_t>& bounds, TilePlan& plan) {
   const uint32_t ntiles = uint32_t(bounds.size() - 1);
   std::vector<uint32_t> tile_of(E);
   for (uint32_t t = 0; t < ntiles; ++t)
@@ -157,12 +177,13 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
   std::vector<std::vector<uint32_t>> t_rec(ntiles), t_nodes(ntiles);
   std::vector<std::vector<uint16_t>> t_lid(ntiles);
   unsigned nt = std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
-  if (ntiles < 64) nt = 1;
+  nt = std::min(nt, std::max(1u, ntiles / 16u));   // a worker's start costs as much as a dozen small tiles
   std::vector<std::thread> th;
   std::vector<int> err(nt, 0);
   for (unsigned w = 0; w < nt; ++w) {
     th.emplace_back([&, w] {
       std::vector<int32_t> lid_of(N, -1);
+      std::vector<uint32_t> cls_end(1024), sorted;
       for (uint32_t t = w; t < ntiles; t += nt) {
         auto& recs = t_rec[t];
         const uint32_t e0 = bounds[t], e1 = bounds[t + 1];
@@ -170,23 +191,27 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
         std::iota(recs.begin(), recs.end(), e0);
         recs.insert(recs.end(), halo[t].begin(), halo[t].end());
         // classes: child-0 type, then level (uniform coefficients read one element matrix
-        // per (type, level) class)
-        auto cls = [&](uint32_t e) { return (uint32_t(tp[e]) << 8) | lev[e]; };
-        std::stable_sort(recs.begin(), recs.end(), [&](uint32_t a, uint32_t b) { return cls(a) < cls(b); });
+        // per (type, level) class); a counting sort keeps the Morton order inside a class
+        auto cls = [&](uint32_t e) { return (uint32_t(tp[e]) << 5) | lev[e]; };
+        std::fill(cls_end.begin(), cls_end.end(), 0u);
+        for (uint32_t e : recs) ++cls_end[cls(e)];
+        uint32_t at = 0;
+        for (uint32_t& c : cls_end) {
+          const uint32_t n = c;
+          c = at;
+          at += n;
+        }
+        sorted.resize(recs.size());
+        for (uint32_t e : recs) sorted[cls_end[cls(e)]++] = e;
         // Inside each class, deal the Morton-ordered records round-robin over the class's
         // wavefronts: the 64 lanes of a wavefront then hold elements about n/64 apart, so
         // siblings (which share the parent-centre node after the mirror permutation) do
         // not collide on one LDS address in the same atomic instruction.
-        for (size_t a = 0; a < recs.size();) {
-          size_t b = a;
-          while (b < recs.size() && cls(recs[b]) == cls(recs[a])) ++b;
-          const size_t n = b - a, W = (n + 63) / 64;
-          if (W > 1) {
-            std::vector<uint32_t> seg(recs.begin() + a, recs.begin() + b);
-            size_t q = a;
-            for (size_t w = 0; w < W; ++w)
-              for (size_t i = w; i < n; i += W) recs[q++] = seg[i];
-          }
+        size_t q = 0;
+        for (size_t a = 0; a < sorted.size();) {
+          const size_t b = cls_end[cls(sorted[a])], W = (b - a + 63) / 64;
+          for (size_t w2 = 0; w2 < W; ++w2)
+            for (size_t i = a + w2; i < b; i += W) recs[q++] = sorted[i];
           a = b;
         }
         auto& nodes = t_nodes[t];

@@ -189,8 +189,9 @@ int dgh_mesh_set_coefficients(dgh_mesh m, const double* kappa, const double* mas
                               double lap_fac, double mass_fac);
 int dgh_mesh_info(dgh_mesh m, uint32_t* n_elem, uint32_t* n_node);
 /* Re-tiles the operator kernel with tiles of at most tile_elems Morton-consecutive elements
- * (default 2048 with 512 threads, or 8192 with 1024 threads on meshes of at least 4M
- * elements; reduced automatically until the tile's LDS fits) and block threads per
+ * (the default follows the mesh size: 64 elements with 512 threads on the smallest meshes, about
+ * 512 tiles up to 2M elements, 8192 with 1024 threads from 4M elements up; reduced automatically
+ * until the tile's LDS fits) and block threads per
  * workgroup (256, 512 or 1024; 0 keeps the current value).  No reference counterpart: the
  * tuning hook of the tile autotuner. */
 int dgh_mesh_set_tile(dgh_mesh m, uint32_t tile_elems, uint32_t block);
@@ -206,9 +207,9 @@ int dgh_mesh_tile_info(dgh_mesh m, uint32_t* tile_elems, uint32_t* n_tiles, uint
  * DGH_ROWS_CLASS = uniform coefficients only (per-element ones use DGH_ROWS_TYPE): the
  * element matrix lap_fac h/2 L + mass_fac h^3/8 M of each (type, level) class, read through
  * the scalar cache once per class present in a wavefront (half the products per row).
- * All forms agree to rounding.  The diagonal always reads rows: those of the source set, else
- * DGH_ROWS_CLASS for tilings of at least 1024 tiles and DGH_ROWS_TYPE otherwise, which is what
- * dgh_mesh_lane_stencils reports until one is set.  DGH_ROWS_LANE fails if the tiling leaves
+ * All forms agree to rounding.  Until one is set, dgh_mesh_lane_stencils reports
+ * DGH_ROWS_CLASS for tilings of at least 1024 tiles and DGH_ROWS_TYPE otherwise.  The diagonal
+ * reads the rows of the source set, else per type.  DGH_ROWS_LANE fails if the tiling leaves
  * no LDS room for the table.  No reference counterpart: a kernel choice; dgh_mesh_autotune
  * returns to the factored form. */
 #define DGH_ROWS_TYPE 0
