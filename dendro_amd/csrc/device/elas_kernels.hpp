@@ -183,7 +183,7 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
     for (int a = 0; a < 3; ++a) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) xe[a][k] = *lds_at<double>(XS + l[k] + 8u * a);
-      hang_interp(xe[a], hb, quarter);
+      hang_interp(reinterpret_cast<double(&)[1][8]>(xe[a]), hb, quarter);
       wht8(xe[a]);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -227,7 +227,7 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
             y8[i | b] = y8[i] - y8[i | b];
             y8[i] = s;
           }
-      hang_interp_t(xe[a], hb, quarter);
+      hang_interp_t(reinterpret_cast<double(&)[1][8]>(xe[a]), hb, quarter);
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (l[k] < own) lds_add(lds_at<unsigned long long>(l[k] + 8u * a), fx_round_fma(y8[k], sc));

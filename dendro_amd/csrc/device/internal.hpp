@@ -164,7 +164,7 @@ struct dgh_mesh_s {
   int block = 512;              // threads per operator workgroup (256, 512 or 1024)
   DevTiles mop;
   uint32_t mtile = 0;           // batched tile size (0: default)
-  int mvariant = 0;             // batched FP32 products: 0 vector ALUs, 1 matrix cores
+  int mvariant = 6;             // batched FP32 products (multi_api.hip): 1 matrix cores, others vector ALUs
   uint64_t gen = 0;             // bumped whenever device tilings or coefficients are rebuilt
   uint64_t coef_gen = 0;        // bumped by dgh_mesh_set_coefficients
   uint64_t bdy_gen = 0;         // bumped by dgh_mesh_set_boundary

@@ -143,7 +143,13 @@ constexpr int FX32_BITS = 30;
 constexpr double FX_MARGIN = 1.0 + 0x1p-20;
 constexpr double FX_MAGIC = 6755399441055744.0;   // 1.5 * 2^52
 constexpr unsigned long long FX_MAGIC_BITS = 0x4338000000000000ull;
-constexpr int FX_XMIN = -900;                      // |x| below 2^-900 counts as 2^-900
+constexpr int FX_XMIN = -900;                      // |x| below 2^-900 counts as 2^-900,
+constexpr int FX32_XMIN = -96;                     // FP32: below 2^-96 (the scaled factors stay finite)
+// max |x| < 2^ex of a tile (or column) from the high word of its max |x| in FP64
+template <class T>
+__device__ __forceinline__ int fx_ex(uint32_t hi) {
+  return max(int(hi >> 20) - 1022, sizeof(T) == 8 ? FX_XMIN : FX32_XMIN);
+}
 
 template <class T>
 using fx_acc_t = typename std::conditional<sizeof(T) == 8, unsigned long long, unsigned int>::type;
@@ -213,79 +219,6 @@ __device__ __forceinline__ lds_ptr<U> lds_at(uint32_t byte) {
 template <class U>
 __device__ __forceinline__ void lds_add(lds_ptr<U> p, U v) {
   __atomic_fetch_add(p, v, __ATOMIC_RELAXED);
-}
-
-// Batched kernels: evaluates one record for CPL adjacent columns with stencil triangles
-// Ls/Ms held in scalar registers (one pass over the 36 triangle entries: each stencil value
-// feeds both rows it belongs to) and adds the rows of owned nodes, column q scaled by
-// 2^es[q], to the fixed-point sums.  R.l holds the nodes' tile-local ids; node l's values
-// of the lane's columns sit at LDS byte address xb + l * RS * sizeof(T) (x) and
-// yb + l * RS * sizeof(acc) (sums), one 24-bit multiply-add per address (written out: the
-// compiler shares l * stride between the two addresses and adds twice; the strides are at
-// most 64, inline constants).
-template <class T, bool MASS, int MODE, int CPL, int RS>
-__device__ __forceinline__ void eval_rec_tri(const Rec& R, uint32_t n_own, const int* es, const T* Ls,
-                                             const T* Ms, uint32_t xb, uint32_t yb) {
-  using TA = fx_acc_t<T>;
-  const T fac1 = T(R.k1), fac2 = T(R.k2);
-  T f1s[CPL], f2s[CPL];
-#pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    if constexpr (sizeof(T) == 4) {
-      f1s[q] = ldexpf(fac1, es[q]);
-      f2s[q] = MASS ? ldexpf(fac2, es[q]) : T(0);
-    } else {
-      f1s[q] = ldexp(fac1, es[q]);
-      f2s[q] = MASS ? ldexp(fac2, es[q]) : T(0);
-    }
-  }
-  T xv[CPL][8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    uint32_t a;
-    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(a) : "v"(R.l[j]), "n"(int(RS * sizeof(T))), "v"(xb));
-#pragma unroll
-    for (int q = 0; q < CPL; ++q) xv[q][j] = *lds_at<T>(a + q * uint32_t(sizeof(T)));
-  }
-  T a[CPL][8], bm[CPL][8];
-#pragma unroll
-  for (int q = 0; q < CPL; ++q)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a[q][k] = T(0);
-      bm[q][k] = T(0);
-    }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-#pragma unroll
-    for (int q = 0; q < CPL; ++q) {
-      a[q][k] += Ls[tri(k, k)] * xv[q][k];
-      if (MASS) bm[q][k] += Ms[tri(k, k)] * xv[q][k];
-    }
-#pragma unroll
-    for (int j = k + 1; j < 8; ++j) {
-      const T l = Ls[tri(k, j)];
-      const T m = MASS ? Ms[tri(k, j)] : T(0);
-#pragma unroll
-      for (int q = 0; q < CPL; ++q) {
-        a[q][k] += l * xv[q][j];
-        a[q][j] += l * xv[q][k];
-        if (MASS) {
-          bm[q][k] += m * xv[q][j];
-          bm[q][j] += m * xv[q][k];
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k)
-    if (R.l[k] < n_own) {
-      uint32_t ya;
-      asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(ya) : "v"(R.l[k]), "n"(int(RS * sizeof(TA))), "v"(yb));
-#pragma unroll
-      for (int q = 0; q < CPL; ++q)
-        lds_add(lds_at<TA>(ya + q * uint32_t(sizeof(TA))), fx_term(a[q][k], f1s[q], bm[q][k], f2s[q], MASS));
-    }
 }
 
 // Evaluates the rows of the owned vertices of one record and adds them, scaled by 2^es, to
@@ -464,28 +397,34 @@ __device__ __forceinline__ void fact_modes(T f1, T f2, T d[4]) {
 // selects (75 more vector instructions per 64 records with hanging vertices), where records
 // sorted by type leave most wavefronts with few of the six branches taken.
 #define DGH_NO_SELECT asm volatile("")
-// v <- P_H v; q = 1/4 (a register: the compiler would otherwise scale
-// by a quarter with the slower ldexp)
-template <class T>
-__device__ __forceinline__ void hang_interp(T v[8], uint32_t hb, T q) {
+// v[c] <- P_H v[c] for N columns; q = 1/4 (a register: the compiler would otherwise scale by a
+// quarter with the slower ldexp)
+template <int N, class T>
+__device__ __forceinline__ void hang_interp(T (&v)[N][8], uint32_t hb, T q) {
   if (hb == 0u) return;
-  if (hb & 8u) { DGH_NO_SELECT; v[3] = q * ((v[0] + v[1]) + (v[2] + v[3])); }
-  if (hb & 16u) { DGH_NO_SELECT; v[5] = q * ((v[0] + v[1]) + (v[4] + v[5])); }
-  if (hb & 32u) { DGH_NO_SELECT; v[6] = q * ((v[0] + v[2]) + (v[4] + v[6])); }
-  if (hb & 1u) { DGH_NO_SELECT; v[1] = T(0.5) * (v[0] + v[1]); }
-  if (hb & 2u) { DGH_NO_SELECT; v[2] = T(0.5) * (v[0] + v[2]); }
-  if (hb & 4u) { DGH_NO_SELECT; v[4] = T(0.5) * (v[0] + v[4]); }
+#define DGH_HANG(bit, expr)                       \
+  if (hb & (bit)) {                               \
+    DGH_NO_SELECT;                                \
+    _Pragma("unroll") for (int c = 0; c < N; ++c) { expr; } \
+  }
+  DGH_HANG(8u, v[c][3] = q * ((v[c][0] + v[c][1]) + (v[c][2] + v[c][3])))
+  DGH_HANG(16u, v[c][5] = q * ((v[c][0] + v[c][1]) + (v[c][4] + v[c][5])))
+  DGH_HANG(32u, v[c][6] = q * ((v[c][0] + v[c][2]) + (v[c][4] + v[c][6])))
+  DGH_HANG(1u, v[c][1] = T(0.5) * (v[c][0] + v[c][1]))
+  DGH_HANG(2u, v[c][2] = T(0.5) * (v[c][0] + v[c][2]))
+  DGH_HANG(4u, v[c][4] = T(0.5) * (v[c][0] + v[c][4]))
 }
-// v <- P_H^T v
-template <class T>
-__device__ __forceinline__ void hang_interp_t(T v[8], uint32_t hb, T q) {
+// v[c] <- P_H^T v[c]
+template <int N, class T>
+__device__ __forceinline__ void hang_interp_t(T (&v)[N][8], uint32_t hb, T q) {
   if (hb == 0u) return;
-  if (hb & 1u) { DGH_NO_SELECT; v[1] *= T(0.5); v[0] += v[1]; }
-  if (hb & 2u) { DGH_NO_SELECT; v[2] *= T(0.5); v[0] += v[2]; }
-  if (hb & 4u) { DGH_NO_SELECT; v[4] *= T(0.5); v[0] += v[4]; }
-  if (hb & 8u) { DGH_NO_SELECT; v[3] *= q; v[0] += v[3]; v[1] += v[3]; v[2] += v[3]; }
-  if (hb & 16u) { DGH_NO_SELECT; v[5] *= q; v[0] += v[5]; v[1] += v[5]; v[4] += v[5]; }
-  if (hb & 32u) { DGH_NO_SELECT; v[6] *= q; v[0] += v[6]; v[2] += v[6]; v[4] += v[6]; }
+  DGH_HANG(1u, v[c][0] += T(0.5) * v[c][1]; v[c][1] *= T(0.5))
+  DGH_HANG(2u, v[c][0] += T(0.5) * v[c][2]; v[c][2] *= T(0.5))
+  DGH_HANG(4u, v[c][0] += T(0.5) * v[c][4]; v[c][4] *= T(0.5))
+  DGH_HANG(8u, v[c][0] += q * v[c][3]; v[c][1] += q * v[c][3]; v[c][2] += q * v[c][3]; v[c][3] *= q)
+  DGH_HANG(16u, v[c][0] += q * v[c][5]; v[c][1] += q * v[c][5]; v[c][4] += q * v[c][5]; v[c][5] *= q)
+  DGH_HANG(32u, v[c][0] += q * v[c][6]; v[c][2] += q * v[c][6]; v[c][4] += q * v[c][6]; v[c][6] *= q)
+#undef DGH_HANG
 }
 
 // v <- W diag(d[popcount]) W v.  Without a mass term the mean mode's factor is zero.
@@ -531,6 +470,9 @@ __device__ __forceinline__ unsigned long long fx_round_fma(double v, double sc) 
   const uint32_t hi = uint32_t(b >> 32) - uint32_t(FX_MAGIC_BITS >> 32);
   return (static_cast<unsigned long long>(hi) << 32) | uint32_t(b);
 }
+// FP32: halves to even.  Halves up would be one instruction instead of two, but half of the values
+// in [2^22, 2^23) are exact halves: the bias made a null-space solve's FP32 V-cycle ten times less
+// exact.
 __device__ __forceinline__ unsigned int fx_round(float v) {
   return static_cast<unsigned int>(__float2int_rn(v));
 }
@@ -563,9 +505,9 @@ __device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, 
 #pragma unroll
   for (int j = 0; j < 8; ++j) l[j] = ((w[j >> 1] >> (16 * (j & 1))) & REC_ID_MASK) * uint32_t(sizeof(T));
   const uint32_t hb = rec_hang(lp);
-  T v[8];
+  T v[1][8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = *lds_at<T>(XS + l[j]);
+  for (int j = 0; j < 8; ++j) v[0][j] = *lds_at<T>(XS + l[j]);
   T f1, f2 = T(0);
   if (UNI) {
     const int hs = int(maxD - (rec_class(lp) >> 5));
@@ -583,11 +525,11 @@ __device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, 
   T q = T(0.25);
   asm("" : "+s"(q));
   hang_interp(v, hb, q);
-  fact_product<T, MASS>(v, d);
+  fact_product<T, MASS>(v[0], d);
   hang_interp_t(v, hb, q);
 #pragma unroll
   for (int k = 0; k < 8; ++k)
-    if (l[k] < own_bytes) lds_add(lds_at<fx_acc_t<T>>(l[k]), fx_round(v[k]));
+    if (l[k] < own_bytes) lds_add(lds_at<fx_acc_t<T>>(l[k]), fx_round(v[0][k]));
 }
 
 // Touched and owned nodes per thread of a tile, from the plan's bounds (op_own_cap, op_budget):
@@ -719,7 +661,7 @@ tile_op_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* __
     xhi = uint32_t(uint64_t(__double_as_longlong(double(__uint_as_float(xhi)))) >> 32);
   // max |x| < 2^ex; a non-finite x makes every owned output of the tile NaN
   const bool finite = (xhi >> 20) < 0x7ffu;
-  const int ex = MODE == OP_DIAG ? 1 : max(int(xhi >> 20) - 1022, FX_XMIN);
+  const int ex = MODE == OP_DIAG ? 1 : fx_ex<T>(xhi);
   const int es = fx_scale<T>(texp[t], ex);
   const uint32_t own_bytes = n_own * uint32_t(sizeof(T));
   for (uint32_t r0 = w0; r0 < rec.n_elem; r0 += BLOCK) {

@@ -24,7 +24,7 @@ namespace dgh {
 constexpr int KS = 8;            // right-hand sides per workgroup slice (FP32)
 constexpr int KS64 = 4;          // right-hand sides per workgroup slice (FP64: same LDS bytes)
 constexpr int MAXK = 32;         // right-hand sides per batch
-constexpr int MBLOCK = 512;      // threads per batched-operator workgroup (default)
+constexpr int MBLOCK = 512;      // threads per batched-operator workgroup
 
 template <class T>
 struct MultiIO {
@@ -47,36 +47,101 @@ template <class T> using vec16_t = typename Vec16<T>::type;
 
 // Vector-ALU batched operator.  Lane = (element of the round, CPL adjacent right-hand sides
 // c .. c + CPL - 1 of the slice): the KSL / CPL lanes of an element share its record, read
-// the element's 8 node values of their columns from LDS and accumulate its 8 rows; the
-// stencil comes through the scalar cache (per-type wavefront loop), so LDS carries only the
-// minimum per element and column: 8 reads and at most 8 additions, while the record, the
-// stencil walk and the LDS addresses are shared by the CPL columns of a lane.  Sums
+// the element's 8 node values of their columns from LDS, apply the factored element product
+// (fact_product, kernels.hpp) and accumulate its 8 rows, so LDS carries only the minimum per
+// element and column: 8 reads and at most 8 additions, while the record, its hanging vertices,
+// the mode factors and the LDS addresses are shared by the CPL columns of a lane.  Sums
 // accumulate in fixed point as in the single right-hand-side kernel (64-bit integers for
-// FP64, 32-bit for FP32), with one scale per column of the slice.  Gathers and stores move
-// 16-byte vectors of a node's slice.  LDS rows are padded to KSL + 1 values so the lanes of
-// different elements spread over the banks.  LDS: owned sums [ys_len][KSL + 1] (fixed
-// point), touched x [max_touch][KSL + 1] (T).
+// FP64, 32-bit for FP32), with one scale per column of the slice; two adjacent FP32 columns of a
+// lane are added as one 64-bit integer (PACK).  Gathers and stores move 16-byte vectors of a
+// node's slice.  LDS rows are padded so the lanes of different elements spread over the banks.
+// FP32, k = 32, 630k elements with a coefficient: 316 us with stencil triangles in scalar registers
+// (tiles of 1024, one column per lane) -> 143 us in tiles of 512, two columns per lane; FP64 376 ->
+// 238.  It is bound by the vector ALUs (95% of their issue slots): about 118 instructions per element
+// and column, 56 of them the product, 24 the conversion and packing of the sums, the rest record
+// unpacking, hanging vertices and addresses; 1.67 records per element (halo).  Eight
+// columns per lane (143 us), 256 or 1024 threads (165, 159 us) do not pay.
+// LDS: owned sums [ys_len][multi_row_y] (fixed point), touched x [max_touch][multi_row] (T).
 template <class T>
 __host__ __device__ constexpr int multi_row(int ksl) { return ksl + 1; }
+template <class T>
+__host__ __device__ constexpr int multi_row_y(int ksl) { return sizeof(T) == 4 ? ksl + 2 : ksl + 1; }
+
+// Two FP32 columns' fixed-point terms as one 64-bit integer hi 2^32 + lo: sums of such integers
+// hold both 32-bit sums exactly (neither overflows, see FX32_BITS): the low word is the lower
+// column's, and the high word is the upper one's minus one where the lower one's is negative.
+__device__ __forceinline__ unsigned long long fx_pack(unsigned int lo, unsigned int hi) {
+  return (static_cast<unsigned long long>(hi + static_cast<unsigned int>(static_cast<int>(lo) >> 31)) << 32) | lo;
+}
+
+// One record for CPL columns.  n_own = 0 adds nothing; d[p]: the record's mode factors scaled by
+// the tile's bound, cs[q]: the column's scale; node l's values sit at LDS byte address
+// xb + l RSX sizeof(T) (x) and yb + l RSY sizeof(acc) (sums), one 24-bit multiply-add each
+// (written out: the compiler shares l * stride between the two addresses and adds twice; the
+// strides are at most 64, inline constants).
+template <class T, bool MASS, int CPL, int RSX, int RSY, bool PACK>
+__device__ __forceinline__ void eval_multi(uint4 lp, uint32_t n_own, const T d[4], const T cs[CPL], uint32_t xb,
+                                           uint32_t yb) {
+  using TA = fx_acc_t<T>;
+  const uint32_t w[4] = {lp.x, lp.y, lp.z, lp.w};
+  uint32_t l[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) l[j] = (w[j >> 1] >> (16 * (j & 1))) & REC_ID_MASK;
+  const uint32_t hb = rec_hang(lp);
+  T v[CPL][8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    uint32_t a;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(a) : "v"(l[j]), "n"(int(RSX * sizeof(T))), "v"(xb));
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) v[q][j] = *lds_at<T>(a + q * uint32_t(sizeof(T)));
+  }
+  T quarter = T(0.25);
+  asm("" : "+s"(quarter));
+  hang_interp(v, hb, quarter);
+#pragma unroll
+  for (int q = 0; q < CPL; ++q) {
+    T dq[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) dq[p] = d[p] * cs[q];
+    fact_product<T, MASS>(v[q], dq);
+  }
+  hang_interp_t(v, hb, quarter);
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (l[k] < n_own) {
+      uint32_t ya;
+      asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(ya) : "v"(l[k]), "n"(int(RSY * sizeof(TA))), "v"(yb));
+      if constexpr (PACK) {
+#pragma unroll
+        for (int q = 0; q < CPL; q += 2)
+          lds_add(lds_at<unsigned long long>(ya + q * 4u), fx_pack(fx_round(v[q][k]), fx_round(v[q + 1][k])));
+      } else {
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) lds_add(lds_at<TA>(ya + q * uint32_t(sizeof(TA))), fx_round(v[q][k]));
+      }
+    }
+}
 
 template <class T, bool MASS, int MODE, int KSL, int MB, int CPL>
 __global__ void __launch_bounds__(MB)
 tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
                   const uint16_t* __restrict__ lid,
                   const T* __restrict__ kappa, const T* __restrict__ mass, double lap_fac,
-                  double mass_fac, uint32_t maxD, double hFac, const T* __restrict__ K0,
+                  double mass_fac, uint32_t maxD, double hFac,
                   const uint32_t* __restrict__ node_tab, const int2* __restrict__ texp, uint32_t ys_len,
                   MultiIO<T> io) {
   static_assert(MODE != OP_DIAG, "the diagonal does not depend on the right-hand side");
   constexpr int LPE = KSL / CPL;              // lanes per element
   static_assert(KSL % CPL == 0 && 64 % LPE == 0, "a wavefront holds whole elements");
   using TA = fx_acc_t<T>;
-  constexpr int RS = multi_row<T>(KSL);      // padded LDS row
+  constexpr int RS = multi_row<T>(KSL), RSY = multi_row_y<T>(KSL);   // padded LDS rows
+  constexpr bool PACK = sizeof(T) == 4 && CPL % 2 == 0;
   constexpr int NW = MB / 64;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ uint32_t s_xhi[NW][KSL];
   TA* ys = reinterpret_cast<TA*>(smem_raw);
-  T* xs = reinterpret_cast<T*>(ys + size_t(ys_len) * RS);
+  T* xs = reinterpret_cast<T*>(ys + size_t(ys_len) * RSY);
   const int np = ntiles * nslices;
   const int pidx = xcd_tile(blockIdx.x, np);   // the slices of a tile stay on one XCD
   if (pidx >= np) return;
@@ -94,7 +159,7 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
   static_assert(KSL % VEC == 0 && MB % LPN == 0, "whole vectors per node slice");
   using V = vec16_t<T>;
   const int cv = int(threadIdx.x % LPN) * VEC;
-  uint32_t xhv[VEC];   // high words of max |x| of this thread's gather columns
+  uint32_t xhv[VEC];   // high words (FP32: bits) of max |x| of this thread's gather columns
 #pragma unroll
   for (int e = 0; e < VEC; ++e) xhv[e] = 0u;
   // The owned nodes lead the tile's node list, so when they fit in the first batch of
@@ -125,12 +190,15 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           d[e] = v[u][e];
-          xhv[e] = max(xhv[e], uint32_t(uint64_t(__double_as_longlong(double(v[u][e]))) >> 32) & 0x7fffffffu);
+          if constexpr (sizeof(T) == 8)
+            xhv[e] = max(xhv[e], uint32_t(uint64_t(__double_as_longlong(v[u][e])) >> 32) & 0x7fffffffu);
+          else   // FP32 bits order as |x| does; the maximum is converted by col_exp
+            xhv[e] = max(xhv[e], __float_as_uint(v[u][e]) & 0x7fffffffu);
         }
       }
     }
   }
-  for (uint32_t i = threadIdx.x; i < n_own * RS; i += MB) ys[i] = TA(0);
+  for (uint32_t i = threadIdx.x; i < n_own * RSY; i += MB) ys[i] = TA(0);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int es = lane / LPE, c = (lane % LPE) * CPL;   // element of the round, first column
 #pragma unroll
@@ -141,55 +209,52 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
 #pragma unroll
     for (int e = 0; e < VEC; ++e) s_xhi[wv][cv + e] = xhv[e];
   __syncthreads();
-  // per column: max |x| < 2^ex, fixed-point scale 2^esc; a non-finite column gives NaN.
-  // (esc: columns c .. c + CPL - 1 of the products)
-  int esc[CPL];
+  // Per column: max |x| < 2^ex; a non-finite column gives NaN.  A term's scale 2^(es0 - ex) is the
+  // tile's part 2^es0, taken into the record's mode factors, times the column's cs = 2^-ex.
+  auto col_hi = [&](int col) {   // high word of the column's max |x| in FP64
+    uint32_t h = 0;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    uint32_t xhi = 0;
+    for (int w = 0; w < NW; ++w) h = max(h, s_xhi[w][col]);
+    if constexpr (sizeof(T) == 4) h = uint32_t(uint64_t(__double_as_longlong(double(__uint_as_float(h)))) >> 32);
+    return h;
+  };
+  const int es0 = fx_scale<T>(texp[t], 0);
+  T cs[CPL];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) xhi = max(xhi, s_xhi[w][c + q]);
-    esc[q] = fx_scale<T>(texp[t], max(int(xhi >> 20) - 1022, FX_XMIN));
-  }
+  for (int q = 0; q < CPL; ++q) cs[q] = T(ldexp(1.0, -fx_ex<T>(col_hi(c + q))));
   // LDS byte addresses of the lane's first column in row 0 of the staged x and of the sums
   const uint32_t xbase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<T>)(xs + c)));
   const uint32_t ybase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<TA>)(ys + c)));
-  constexpr int EPW = 64 / LPE;               // elements per wavefront round
-  constexpr int STRIDE = (MB / 64) * EPW;
-  // the records of the next round are loaded while the current round is evaluated; the
-  // stencil of the wavefront's current type stays in scalar registers across rounds
-  Rec Rn;
-  uint32_t r0 = uint32_t(wv) * EPW;
-  bool hn = r0 + es < rec.n_elem;
-  if (hn) load_rec<T, MASS>(Rn, rec.elem_off + r0 + es, lid, kappa, mass, lap_fac, mass_fac, maxD, hFac);
-  uint32_t cur = 0xffffffffu;
-  T Lr[36], Mr[36];
+  constexpr uint32_t EPW = 64 / LPE;          // elements per wavefront round
+  constexpr uint32_t STRIDE = (MB / 64) * EPW;
+  // the records of the next round are loaded while the current round is evaluated; lanes past
+  // the last record load it again and add nothing
+  const double u1 = lap_fac * hFac / 2.0, u2 = mass_fac * hFac * hFac * hFac / 8.0;
+  RecF<T> R;
+  auto load = [&](uint32_t r0) {
+    const uint32_t g = rec.elem_off + min(r0 + uint32_t(es), rec.n_elem - 1u);
+    if (kappa)
+      load_rec_fact<T, MASS, false>(R, g, lid, kappa, mass);
+    else
+      load_rec_fact<T, MASS, true>(R, g, lid, kappa, mass);
+  };
+  uint32_t r0 = uint32_t(__builtin_amdgcn_readfirstlane(wv)) * EPW;
+  load(r0);
   for (; r0 < rec.n_elem; r0 += STRIDE) {
-    const Rec R = Rn;
-    const bool h = hn;
-    const uint32_t rn = r0 + STRIDE + es;
-    hn = rn < rec.n_elem;
-    if (hn) load_rec<T, MASS>(Rn, rec.elem_off + rn, lid, kappa, mass, lap_fac, mass_fac, maxD, hFac);
-    const uint32_t tp = R.mt & 31u;
-    bool done = !h;
-    for (;;) {
-      const uint64_t pend = __ballot(!done);
-      if (pend == 0) break;
-      const uint32_t tu = __builtin_amdgcn_readlane(tp, __builtin_ctzll(pend));
-      if (tu != cur) {
-        const T* Ls = K0 + tu * KSTRIDE;
-#pragma unroll
-        for (int q = 0; q < 36; ++q) {
-          Lr[q] = Ls[q];
-          if (MASS) Mr[q] = Ls[36 + q];
-        }
-        cur = tu;
-      }
-      if (!done && tp == tu) {
-        eval_rec_tri<T, MASS, MODE, CPL, RS>(R, n_own, esc, Lr, Mr, xbase, ybase);
-        done = true;
-      }
+    const RecF<T> Rc = R;
+    load(r0 + STRIDE);
+    T f1, f2 = T(0);
+    if (kappa) {
+      f1 = T(ldexp(double(Rc.k1), es0));
+      if (MASS) f2 = T(ldexp(double(Rc.k2), es0));
+    } else {
+      const int hs = int(maxD - (rec_class(Rc.lp) >> 5));
+      f1 = T(ldexp(u1, hs + es0));
+      if (MASS) f2 = T(ldexp(u2, 3 * hs + es0));
     }
+    T d[4];
+    fact_modes<T, MASS>(f1, f2, d);
+    eval_multi<T, MASS, CPL, RS, RSY, PACK>(Rc.lp, r0 + uint32_t(es) < rec.n_elem ? n_own : 0u, d, cs, xbase, ybase);
   }
   // the store's right-hand sides and diagonals of the kept owned nodes: loaded before the
   // barrier, so they are in flight while the other wavefronts finish their records
@@ -210,11 +275,9 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
   bool fins[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
-    uint32_t h = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) h = max(h, s_xhi[w][cv + e]);
+    const uint32_t h = col_hi(cv + e);
     fins[e] = (h >> 20) < 0x7ffu;
-    ess[e] = fx_scale<T>(texp[t], max(int(h >> 20) - 1022, FX_XMIN));
+    ess[e] = es0 - fx_ex<T>(h);
   }
   // stores: 16-byte vectors as in the gather, MSU (= MGU, the batch of own_n) per thread
   // with their loads in flight together
@@ -246,7 +309,11 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
       V out;
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const T v = fins[e] ? T(fx_value<T>(ys[nd * RS + cv + e], ess[e])) : T(__builtin_nan(""));
+        TA sum = ys[nd * RSY + cv + e];
+        if constexpr (PACK) {   // the upper column of a pair: see fx_pack
+          if (e & 1) sum += TA(static_cast<int>(ys[nd * RSY + cv + e - 1]) < 0 ? 1 : 0);
+        }
+        const T v = fins[e] ? T(fx_value<T>(sum, ess[e])) : T(__builtin_nan(""));
         if (MODE == OP_MATVEC || MODE == OP_CG) out[e] = v;
         else if (MODE == OP_RESID) out[e] = bv[u][e] - v;
         else out[e] = xs[nd * RS + cv + e] + io.omega * ((bv[u][e] - v) * dv[u]);

@@ -26,7 +26,8 @@ template <> const float* dm<float>(const DevTiles& d) { return d.rm32.p; }
 // the matrix-core variant adds the full stencil table.
 template <class T, int KSL>
 static size_t multi_lds_valu(const DevTiles& d) {
-  return size_t(multi_row<T>(KSL)) * (sizeof(fx_acc_t<T>) * d.ys_len + sizeof(T) * d.plan.max_touch);
+  return size_t(multi_row_y<T>(KSL)) * sizeof(fx_acc_t<T>) * d.ys_len +
+         size_t(multi_row<T>(KSL)) * sizeof(T) * d.plan.max_touch;
 }
 static size_t multi_lds_mfma(const DevTiles& d, bool mass) {
   return sizeof(double) * KS * d.ys_len + sizeof(float) * KS * d.plan.max_touch +
@@ -46,8 +47,19 @@ static void plan_multi(dgh_mesh m, uint32_t T) {
   m->mtile = m->mop.plan.tile_elems;
 }
 
+// Default tile size of the batched operator, with variant 6 (4 columns per slice, 2 per lane): at
+// most 512 elements, which three (FP32 k = 32: four) workgroups per CU hold, and on small meshes
+// E/100 (at least 96) so that the slices of all tiles fill the device.  FP32 / FP64 products, us:
+//   2.5k elements, k = 32   tiles of 96   5.5 /   5.8, of 512   8.6 /  10.6, of 1024  11.3 /  14.7
+//   40k, k = 32             of 384       17.7 /  24.6, of 128  20.1 /  30.4, of 1024  20.7 /  31.2
+//   630k, k = 32            of 512        143 /   238, of 192   186 /   349, of 1024   144 /   310
+//   630k, k = 8             of 512       40.3 /  62.7, of 192  50.7 /  88.0, of 1024  39.8 /  75.8
+// Variants 4 and 5 (8 columns per slice) reach 140 and 137 us at 630k, k = 32, but take 8.6 and 7.4
+// against 5.6 on the smallest meshes at k = 8, which have half as many workgroups with them.
+static uint32_t multi_tile_elems(uint32_t n_elem) { return std::min(512u, std::max(96u, n_elem / 100u)); }
+
 void ensure_multi(dgh_mesh m) {
-  if (m->mop.plan.tiles.empty()) plan_multi(m, m->mtile ? m->mtile : 1024);
+  if (m->mop.plan.tiles.empty()) plan_multi(m, m->mtile ? m->mtile : multi_tile_elems(m->E));
 }
 
 static void check_k(int k) {
@@ -63,7 +75,7 @@ static void launch_valu(dgh_mesh m, const DevTiles& d, const T* kap, const T* ma
   const size_t lds = multi_lds_valu<T, KSL>(d);
   hipLaunchKernelGGL((tile_multi_kernel<T, MASS, MODE, KSL, MB, CPL>), dim3(grid), dim3(MB), lds, st,
                      d.tiles.p, nt, io.k / KSL, d.lid.p, kap, mas, m->lap_fac, m->mass_fac, m->maxD,
-                     m->hFac, Ktab<T>(), d.node_tab.p, (const int2*)d.texp.p, d.ys_len, io);
+                     m->hFac, d.node_tab.p, (const int2*)d.texp.p, d.ys_len, io);
 }
 
 template <bool MASS, int MODE>

@@ -271,7 +271,8 @@ int dgh_matvec_multi(dgh_mesh m, int prec, int k, const void* x_dev, void* y_dev
  * and the FP32 product variant (0: vector ALUs, 8 columns per workgroup slice, 512
  * threads, one column per lane; 1: matrix cores; 2: as 0 with 1024 threads; 3: as 0 with 4
  * columns per slice; 4, 5: as 0 with 2, 4 columns per lane; 6: as 3 with 2 columns per
- * lane).  No reference counterpart (tuning hook). */
+ * lane).  The default is variant 6 with 96 to 512 elements by mesh size.  No reference
+ * counterpart (tuning hook). */
 int dgh_mesh_set_tile_multi(dgh_mesh m, uint32_t tile_elems, int variant);
 /* Times the FP32 batched operator for k columns over the candidate tile sizes and all
  * product variants and keeps the fastest; outputs (may be NULL) the tile size, the variant
