@@ -70,7 +70,7 @@ static void check_op_plan(dgh_mesh m) {
 }
 
 template <class T, int MODE, int BLOCK>
-static void launch_op_b(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
+static void launch_op_b(dgh_mesh m, const T* x, const OpIO<T>& io, hipStream_t st) {
   check_op_plan<BLOCK>(m);
   const int nt = int(m->op.plan.tiles.size());
   const unsigned grid = unsigned(NXCD * ((nt + NXCD - 1) / NXCD));
@@ -82,8 +82,8 @@ static void launch_op_b(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
       const double u1 = m->lap_fac * m->hFac / 2.0, u2 = m->mass_fac * m->hFac * m->hFac * m->hFac / 8.0;
 #define DGH_FACT_LAUNCH(MASS, UNI)                                                                              \
   hipLaunchKernelGGL((tile_op_kernel<T, T, MASS, MODE, BLOCK, UNI, false, false, true>), dim3(grid), dim3(BLOCK), \
-                     lds, st, m->op.tiles.p, nt, m->op.lid.p, kap, mas, u1, u2, m->maxD, 1.0, (const T*)nullptr, \
-                     m->op.node_tab.p, m->op.texp.p, io)
+                     lds, st, m->op.tiles.p, m->op.node_tab.p, x, m->op.lid.p, m->op.texp.p, nt, m->op.pitch, kap, \
+                     mas, io, u1, u2, m->maxD, 1.0, (const T*)nullptr)
       if (!kap)
         DGH_FACT_LAUNCH(true, true);
       else if (!mas)
@@ -97,8 +97,8 @@ static void launch_op_b(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
   }
 #define DGH_OP_LAUNCH(MASS, UNI, LANE, COMB)                                                                   \
   hipLaunchKernelGGL((tile_op_kernel<T, T, MASS, MODE, BLOCK, UNI, LANE, COMB>), dim3(grid), dim3(BLOCK), lds, st, \
-                     m->op.tiles.p, nt, m->op.lid.p, kap, mas, m->lap_fac, m->mass_fac, m->maxD,      \
-                     m->hFac, op_rows<T>(m, COMB), m->op.node_tab.p, m->op.texp.p, io)
+                     m->op.tiles.p, m->op.node_tab.p, x, m->op.lid.p, m->op.texp.p, nt, m->op.pitch, kap, mas, io,  \
+                     m->lap_fac, m->mass_fac, m->maxD, m->hFac, op_rows<T>(m, COMB))
   const int rows = op_rows_mode(m);
   if (rows == DGH_ROWS_LANE) {
     if (!kap)
@@ -122,35 +122,35 @@ static void launch_op_b(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
 }
 
 template <class T, int MODE>
-static void launch_op(dgh_mesh m, const OpIO<T>& io, hipStream_t st) {
+static void launch_op(dgh_mesh m, const T* x, const OpIO<T>& io, hipStream_t st) {
   if (m->op.plan.tiles.empty()) return;
   switch (m->block) {
-    case 256: launch_op_b<T, MODE, 256>(m, io, st); break;
-    case 512: launch_op_b<T, MODE, 512>(m, io, st); break;
-    default: launch_op_b<T, MODE, 1024>(m, io, st); break;
+    case 256: launch_op_b<T, MODE, 256>(m, x, io, st); break;
+    case 512: launch_op_b<T, MODE, 512>(m, x, io, st); break;
+    default: launch_op_b<T, MODE, 1024>(m, x, io, st); break;
   }
 }
 
 template <class T>
 static void launch_matvec(dgh_mesh m, const T* x, T* y, hipStream_t st) {
-  launch_op<T, OP_MATVEC>(m, OpIO<T>{x, y, nullptr, nullptr, T(0)}, st);
+  launch_op<T, OP_MATVEC>(m, x, OpIO<T>{y, nullptr, nullptr, T(0)}, st);
 }
 
 template <class T>
 static void launch_diag(dgh_mesh m, T* d, hipStream_t st) {
-  launch_op<T, OP_DIAG>(m, OpIO<T>{nullptr, d, nullptr, nullptr, T(0)}, st);
+  launch_op<T, OP_DIAG>(m, nullptr, OpIO<T>{d, nullptr, nullptr, T(0)}, st);
 }
 
 // r = b - A x
 template <class T>
 static void launch_resid(dgh_mesh m, const T* x, const T* b, T* r, hipStream_t st) {
-  launch_op<T, OP_RESID>(m, OpIO<T>{x, r, b, nullptr, T(0)}, st);
+  launch_op<T, OP_RESID>(m, x, OpIO<T>{r, b, nullptr, T(0)}, st);
 }
 
 // x_out = x + omega invd (b - A x)
 template <class T>
 static void launch_smooth(dgh_mesh m, const T* x, const T* b, const T* invd, T omega, T* x_out, hipStream_t st) {
-  launch_op<T, OP_SMOOTH>(m, OpIO<T>{x, x_out, b, invd, omega}, st);
+  launch_op<T, OP_SMOOTH>(m, x, OpIO<T>{x_out, b, invd, omega}, st);
 }
 
 // c = R f; with x1 given, also x1 = omega (c * invd) (the first sweep on the coarse level)
@@ -191,7 +191,7 @@ static void launch_prolong(dgh_transfer t, const T* c, const T* f_in, T* f_out, 
 // y = A_D x, the Dirichlet-masked operator (one launch)
 template <class T>
 static void launch_dirmv(dgh_mesh m, const T* x, T* y, hipStream_t st) {
-  launch_op<T, OP_DIRMV>(m, OpIO<T>{x, y, nullptr, nullptr, T(0), nullptr, m->bdy.p}, st);
+  launch_op<T, OP_DIRMV>(m, x, OpIO<T>{y, nullptr, nullptr, T(0), nullptr, m->bdy.p}, st);
 }
 
 // Jacobian3 on the coarse level of t: y = R (A_f (P x)) with the fine mesh's own coefficients,
@@ -333,7 +333,20 @@ void build_devtiles(dgh_mesh m, DevTiles& d, uint32_t T, size_t (*lds)(const Dev
   d.tiles.upload(d.plan.tiles.data(), d.plan.tiles.size());
   const std::vector<uint16_t> packed = pack_records(d.plan);
   d.lid.upload(packed.data(), packed.size());
-  d.node_tab.upload(d.plan.node_tab.data(), d.plan.node_tab.size());
+  if (block > 0) {   // single right-hand-side kernels: a fixed pitch, padded with each tile's last node
+    d.pitch = d.plan.max_touch;
+    std::vector<uint32_t> tab(d.plan.tiles.size() * size_t(d.pitch));
+    for (size_t t = 0; t < d.plan.tiles.size(); ++t) {
+      const TileRec& tr = d.plan.tiles[t];
+      const uint32_t* src = d.plan.node_tab.data() + tr.node_off;
+      uint32_t* dst = tab.data() + t * d.pitch;
+      std::copy(src, src + tr.n_touch, dst);
+      std::fill(dst + tr.n_touch, dst + d.pitch, src[tr.n_touch - 1]);
+    }
+    d.node_tab.upload(tab.data(), tab.size());
+  } else {
+    d.node_tab.upload(d.plan.node_tab.data(), d.plan.node_tab.size());
+  }
   upload_coefs(m, d);
 }
 
@@ -576,7 +589,7 @@ static const void* precondition_raw(dgh_solver s, const double* r, hipStream_t s
 
 // w = A p and the tile partials of p.w -> part
 static void launch_cg(dgh_mesh m, const double* p, double* w, double* part, hipStream_t st) {
-  launch_op<double, OP_CG>(m, OpIO<double>{p, w, nullptr, nullptr, 0.0, part}, st);
+  launch_op<double, OP_CG>(m, p, OpIO<double>{w, nullptr, nullptr, 0.0, part}, st);
 }
 
 // One CG iteration (everything between two stopping tests), on device scalars only:
@@ -635,8 +648,8 @@ static void cg_iteration(dgh_solver s, hipStream_t st) {
 // Jacobi diagonal of level l (the Dirichlet one, 1 on boundary nodes, for the Dirichlet problem)
 static void solver_diag(dgh_solver s, int l, double* d) {
   dgh_mesh m = s->meshes[l];
-  launch_op<double, OP_DIAG>(m, OpIO<double>{nullptr, d, nullptr, nullptr, 0.0, nullptr,
-                                             s->dirichlet ? m->bdy.p : nullptr}, s->st);
+  launch_op<double, OP_DIAG>(m, nullptr, OpIO<double>{d, nullptr, nullptr, 0.0, nullptr,
+                                                      s->dirichlet ? m->bdy.p : nullptr}, s->st);
 }
 
 // Jacobian3 coarsest matrix (BUILD_FULL_JAC_TYPE3_BLOCK, examples/src/backend/omgJac.C:2341-2448)
@@ -933,8 +946,11 @@ int dgh_mesh_create(uint32_t n_elem, uint32_t n_node, uint32_t max_depth, const 
     m->maxD = max_depth;
     m->hFac = 1.0 / double(1u << (max_depth - 1));
     m->h_cs.resize(n_elem);
+    int8_t types[8][256];
+    for (int c = 0; c < 8; ++c)
+      for (int h = 0; h < 256; ++h) types[c][h] = int8_t(etype_of(c, uint8_t(h)));
     for (uint32_t e = 0; e < n_elem; ++e) {
-      const int t = etype_of(child[e], hn_mask[e]);
+      const int t = child[e] < 8 ? types[child[e]][hn_mask[e]] : -1;
       if (t < 0) fail(DGH_ERR_MESH, "element %u: hanging mask %u invalid for child %u", e, hn_mask[e], child[e]);
       if (lev[e] < 1 || lev[e] >= max_depth + 1) fail(DGH_ERR_MESH, "element %u: level %u out of range", e, lev[e]);
       m->h_cs[e] = uint8_t(18 * child[e] + t);
@@ -1175,7 +1191,7 @@ int dgh_matvec_dirichlet(dgh_mesh m, int prec, const void* x, void* y, void* str
     // one operator launch: the gather stages boundary x as 0, the store writes x on boundary rows
     auto run = [&](auto* xt, auto* yt) {
       using T = std::remove_const_t<std::remove_pointer_t<decltype(xt)>>;
-      launch_op<T, OP_DIRMV>(m, OpIO<T>{xt, yt, nullptr, nullptr, T(0), nullptr, m->bdy.p}, st);
+      launch_op<T, OP_DIRMV>(m, xt, OpIO<T>{yt, nullptr, nullptr, T(0), nullptr, m->bdy.p}, st);
     };
     if (prec == DGH_F64)
       run(static_cast<const double*>(x), static_cast<double*>(y));
@@ -1195,11 +1211,11 @@ int dgh_diagonal_dirichlet(dgh_mesh m, int prec, void* d, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     // the diagonal's store writes 1 on boundary nodes
     if (prec == DGH_F64)
-      launch_op<double, OP_DIAG>(m, OpIO<double>{nullptr, static_cast<double*>(d), nullptr, nullptr, 0.0, nullptr,
-                                                 m->bdy.p}, st);
+      launch_op<double, OP_DIAG>(m, nullptr, OpIO<double>{static_cast<double*>(d), nullptr, nullptr, 0.0, nullptr,
+                                                          m->bdy.p}, st);
     else if (prec == DGH_F32)
-      launch_op<float, OP_DIAG>(m, OpIO<float>{nullptr, static_cast<float*>(d), nullptr, nullptr, 0.f, nullptr,
-                                               m->bdy.p}, st);
+      launch_op<float, OP_DIAG>(m, nullptr, OpIO<float>{static_cast<float*>(d), nullptr, nullptr, 0.f, nullptr,
+                                                        m->bdy.p}, st);
     else
       fail(DGH_ERR_ARG, "unknown precision %d", prec);
   });

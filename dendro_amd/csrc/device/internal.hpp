@@ -116,6 +116,7 @@ struct DevTiles {
   uint32_t ys_len = 0;          // owned-node slots per tile (>= max_own, even; batched kernels)
   uint32_t lds64 = 0, lds32 = 0;  // single right-hand-side kernel: LDS bytes of a launch
   int block = 0;                  // single right-hand-side kernel: block size of the plan
+  uint32_t pitch = 0;             // single right-hand-side kernel: node_tab is [tiles][pitch], padded
   DevBuf<TileRec> tiles;
   DevBuf<uint16_t> lid;         // records: 8 vertex ids with the class in spare bits (pack_records)
   DevBuf<uint32_t> node_tab;

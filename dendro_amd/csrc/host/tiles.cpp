@@ -165,10 +165,13 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
     std::vector<uint32_t> fillp(own_cnt.begin(), own_cnt.end() - 1);
     for (uint32_t n = 0; n < N; ++n) owned[fillp[owner[n]]++] = n;
   }
-  // element class t' (child-0 type of the mirrored mask)
+  // element class t' (child-0 type of the mirrored mask), by child and mask
+  std::vector<int8_t> type_of(8 * 256);
+  for (int c = 0; c < 8; ++c)
+    for (int h = 0; h < 256; ++h) type_of[c * 256 + h] = int8_t(etype_of(0, mirror_mask(uint8_t(h), c)));
   std::vector<uint8_t> tp(E);
   for (uint32_t e = 0; e < E; ++e) {
-    const int t0 = etype_of(0, mirror_mask(hn[e], child[e]));
+    const int t0 = type_of[child[e] * 256 + hn[e]];
     if (t0 < 0) fail(DGH_ERR_MESH, "element %u: mirrored hanging mask is not a child-0 type", e);
     tp[e] = uint8_t(t0);
   }
