@@ -3,7 +3,9 @@
 // examples/src/backend/omgRhs.C).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 #include "internal.hpp"
@@ -21,17 +23,10 @@ static FnDev fn_dev(const dgh_function* f) {
   return d;
 }
 
+constexpr int L2_BLOCKS = 4096;   // workgroups of the error pass: one chunk each up to 1M elements
+
 static void require_geometry(dgh_mesh m) {
   if (m->E && m->geo.n != m->E) fail(DGH_ERR_STATE, "dgh_mesh_set_geometry has not been called on this mesh");
-}
-
-static const double* shfn_table() {
-  if (!g.SF.p) {
-    std::vector<double> S(size_t(144) * 8 * NQ);
-    generate_shfn(S.data());
-    g.SF.upload(S.data(), S.size());
-  }
-  return g.SF.p;
 }
 
 }  // namespace dgh
@@ -47,7 +42,11 @@ int dgh_mesh_set_geometry(dgh_mesh m, const uint32_t* anchor) {
     for (uint32_t e = 0; e < m->E; ++e) {
       const uint32_t* a = anchor + size_t(e) * 3;
       if (a[0] >= lim || a[1] >= lim || a[2] >= lim) fail(DGH_ERR_MESH, "element %u: anchor outside the domain", e);
-      geo[e] = make_int4(int(a[0]), int(a[1]), int(a[2]), int(m->h_lev[e]));
+      // child 0's hanging vertices (the mirror maps vertex k to k ^ child)
+      uint32_t mask = 0;
+      for (uint32_t k = 0; k < 8; ++k) mask |= ((uint32_t(m->h_hn[e]) >> (k ^ m->h_child[e])) & 1u) << k;
+      geo[e] = make_int4(int(a[0]), int(a[1]), int(a[2]),
+                         int(uint32_t(m->h_lev[e]) | (uint32_t(m->h_child[e]) << 8) | (hang_bits(mask) << 16)));
     }
     m->geo.upload(geo.data(), geo.size());
   });
@@ -59,12 +58,12 @@ int dgh_rhs_quadrature(dgh_mesh m, const dgh_function* f, double* b, void* strea
     if (!m || !b) fail(DGH_ERR_ARG, "NULL argument");
     const FnDev fd = fn_dev(f);
     require_geometry(m);
-    const double* SF = shfn_table();
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (m->N) hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(m->N)), dim3(VBLOCK), 0, st, b, 0.0, m->N);
+    auto* kern = fd.kind == DGH_FN_COS_SUM ? rhs_quad_kernel<true> : rhs_quad_kernel<false>;
     if (m->E)
-      hipLaunchKernelGGL(rhs_quad_kernel, dim3(blocks_for(m->E)), dim3(VBLOCK), 0, st, m->E, m->maxD,
-                         (const int4*)m->geo.p, (const uint32_t*)m->nl.p, (const uint8_t*)m->cs.p, SF, fd, b);
+      hipLaunchKernelGGL(kern, dim3(blocks_for(m->E)), dim3(VBLOCK), sizeof(RhsShared), st, m->E, m->maxD,
+                         (const int4*)m->geo.p, (const uint32_t*)m->nl.p, fd, b);
     HIP_CHECK(hipGetLastError());
   });
 }
@@ -90,15 +89,22 @@ int dgh_l2_error(dgh_mesh m, const dgh_function* f, const double* u, double* err
     if (!m || !u || !err) fail(DGH_ERR_ARG, "NULL argument");
     const FnDev fd = fn_dev(f);
     require_geometry(m);
-    const double* SF = shfn_table();
-    DevBuf<double> part(RED_BLOCKS + 1);
-    hipLaunchKernelGGL(l2_error_kernel, dim3(RED_BLOCKS), dim3(VBLOCK), 0, 0, m->E, m->maxD, (const int4*)m->geo.p,
-                       (const uint32_t*)m->nl.p, (const uint8_t*)m->cs.p, SF, fd, u, part.p);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(RED2_THREADS), 0, 0, int(RED_BLOCKS),
-                       (const double*)part.p, part.p + RED_BLOCKS);
+    // partials and their sum in a workspace of the mesh, held by one call at a time (the call is
+    // synchronous); the sum goes straight to pinned host memory
+    FemWork& w = m->fem;
+    std::lock_guard<std::mutex> lock(w.mu);
+    if (!w.sum) {
+      w.part.alloc(L2_BLOCKS);
+      HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&w.sum), sizeof(double), hipHostMallocMapped));
+    }
+    const unsigned nb = std::min(blocks_for(m->E), unsigned(L2_BLOCKS));
+    auto* kern = fd.kind == DGH_FN_COS_SUM ? l2_error_kernel<true> : l2_error_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(VBLOCK), 0, 0, m->E, m->maxD, (const int4*)m->geo.p,
+                       (const uint32_t*)m->nl.p, fd, u, w.part.p);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(RED2_THREADS), 0, 0, int(nb), (const double*)w.part.p, w.sum);
     HIP_CHECK(hipGetLastError());
-    double s = 0.0;
-    HIP_CHECK(hipMemcpy(&s, part.p + RED_BLOCKS, sizeof(double), hipMemcpyDeviceToHost));
+    HIP_CHECK(hipStreamSynchronize(nullptr));
+    const double s = *w.sum;
     *err = std::sqrt(s);
   });
 }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <mutex>
 #include <vector>
 
 #include "../host/octree.hpp"
@@ -82,7 +83,6 @@ struct State {
   DevBuf<double> KF64;            // child-0 full stencil rows [18][128] (Laplacian, mass)
   DevBuf<float> KF32;
   std::vector<double> hKF;        // host copy of KF64
-  DevBuf<double> SF;              // shape functions at the 3x3x3 Gauss nodes [144][8][27]
   double lrow[NSTENCIL] = {}, mrow[NSTENCIL] = {};   // max row sums of |L|, |M| per type
   rocblas_handle blas = nullptr;
   // device address of the file-scope scratch array of dgh_matvec_dot_noalloc, per device id
@@ -143,6 +143,15 @@ struct ElasState {
   DevBuf<uint32_t> node_tab;
   DevBuf<int2> texp;
 };
+// Workspace of dgh_l2_error on a mesh, held by one call at a time.
+struct FemWork {
+  std::mutex mu;
+  DevBuf<double> part;
+  double* sum = nullptr;        // pinned host memory
+  ~FemWork() {
+    if (sum) (void)hipHostFree(sum);
+  }
+};
 }  // namespace dgh
 
 using namespace dgh;
@@ -172,9 +181,10 @@ struct dgh_mesh_s {
   DevBuf<uint8_t> bdy;          // [N] boundary flags of the Dirichlet operators (empty: none)
   std::vector<uint8_t> h_bdy;   // host copy (Dirichlet coarsest matrix)
   DevBuf<double> dotp;          // per-tile partials of dgh_matvec_dot
-  DevBuf<int4> geo;             // [E] {anchor x, y, z, level}: element points (dgh_mesh_set_geometry)
+  DevBuf<int4> geo;             // [E] element anchors, level, child, hanging vertices (dgh_mesh_set_geometry)
   DevBuf<uint8_t> hn;           // [E] hanging masks (nodal values)
   ElasState elas;               // dgh_mesh_set_elasticity
+  FemWork fem;
 };
 
 struct dgh_transfer_s {

@@ -86,3 +86,32 @@ def test_factored_elasticity(dev, mesh, dirichlet):
         assert err <= 1e-12
         if dirichlet:
             assert np.array_equal(got[bdy != 0], x[bdy != 0])
+
+
+@pytest.mark.parametrize("fn", [dict(kind=da.FN_COS_SUM, nfreq=1), dict(kind=da.FN_COS_SUM, nfreq=19, a0=1.0, a1=0.5),
+                                dict(kind=da.FN_GAUSSIANS), dict(kind=da.FN_POLY, poly=[1, -2, .5, 3, .25, -1, 2, -.75])])
+@pytest.mark.parametrize("mesh", sorted(MESHES) + ["shuffled"])
+def test_quadrature(dev, mesh, fn):
+    """Load vector and L2 error on meshes of one to many workgroups (partial ones among them), with
+    one and several passes over the frequencies; shuffled: elements in random order, so that a
+    workgroup holds more coordinate intervals than its table takes at once."""
+    L = hierarchy(*MESHES["mid" if mesh == "shuffled" else mesh], 1, seed=6, min_coarse=1).fine
+    if mesh == "shuffled":
+        o = np.random.default_rng(3).permutation(L.n_elem)
+        for name in ("nlist", "child", "hnmask", "lev", "anchor"):
+            setattr(L, name, np.ascontiguousarray(getattr(L, name)[o]))
+    m = da.Mesh(L)
+    m.set_geometry(L.anchor)
+    f = da.function(**fn)
+    b = torch.empty(L.n_node, dtype=torch.float64, device=dev)
+    m.rhs_quadrature(f, b)
+    ref = oracle.rhs_quadrature(L, **fn)
+    got = b.cpu().numpy()
+    # terms of size sum |w f phi|: one is at most the function's maximum times the mass row
+    size = np.linalg.norm(ref) + 1e-3 * np.linalg.norm(oracle.rhs_quadrature(L, kind=da.FN_POLY, poly=[1] + [0] * 7))
+    assert np.linalg.norm(got - ref) <= 1e-12 * size
+    u = np.random.default_rng(4).uniform(-1, 1, L.n_node)
+    e = m.l2_error(f, torch.tensor(u, device=dev))
+    e_ref = oracle.l2_error(L, u, **fn)
+    assert abs(e - e_ref) <= 1e-12 * e_ref
+    assert e == m.l2_error(f, torch.tensor(u, device=dev))   # summed in a fixed order
