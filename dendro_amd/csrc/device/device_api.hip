@@ -592,57 +592,98 @@ static void launch_cg(dgh_mesh m, const double* p, double* w, double* part, hipS
   launch_op<double, OP_CG>(m, p, OpIO<double>{w, nullptr, nullptr, 0.0, part}, st);
 }
 
-// One CG iteration (everything between two stopping tests), on device scalars only:
-// direction update (projected z), the operator with the p.w tile partials, alpha, x and r
-// updates (and the FP32 copy of r), the V-cycle, one pass for all dot products (z kept
-// unprojected, see cg_dots_kernel), the scalars.
-static void cg_iteration(dgh_solver s, hipStream_t st) {
+// z = B r and the dot pass over z, r, w.  x1_ready and the FP32 copy of r: from cg_start_kernel or
+// cg_xr_fused_kernel.
+static void cg_precondition(dgh_solver s, hipStream_t st) {
+  const uint32_t n = s->meshes[s->nlevels - 1]->N;
+  s->zres = precondition_raw(s, s->r.p, st, s->nlevels > 1 && s->prm.nu_pre > 0);
+  if (s->prm.vcycle_prec == DGH_F32)
+    hipLaunchKernelGGL(cg_dots_kernel<float>, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, st, n,
+                       static_cast<const float*>(s->zres), (const double*)s->r.p, (const double*)s->w.p, s->part.p);
+  else
+    hipLaunchKernelGGL(cg_dots_kernel<double>, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, st, n,
+                       static_cast<const double*>(s->zres), (const double*)s->r.p, (const double*)s->w.p, s->part.p);
+}
+
+// Direction, w = A p with the partials of p.w, x and r.
+static void cg_step(dgh_solver s, hipStream_t st) {
   const int top = s->nlevels - 1;
   dgh_mesh m = s->meshes[top];
   const uint32_t n = m->N;
   const bool mixed = (s->prm.vcycle_prec == DGH_F32);
-  const bool pnorm = (s->prm.norm_type == DGH_NORM_PRECONDITIONED);
+  const dim3 gb(cg_blocks(n)), tb(VBLOCK);
   double* S = s->S.p;
   if (mixed)
-    hipLaunchKernelGGL(cg_p_fused_kernel<float>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)S,
-                       static_cast<const float*>(s->zres), s->p.p);
+    hipLaunchKernelGGL(cg_p_fused_kernel<float>, gb, tb, 0, st, n, int(s->prm.null_space), 1, (const double*)s->part.p,
+                       S, static_cast<const float*>(s->zres), s->p.p);
   else
-    hipLaunchKernelGGL(cg_p_fused_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)S,
-                       static_cast<const double*>(s->zres), s->p.p);
-  // alpha from the partials of p.w: the operator's tile partials, or (Dirichlet problem) the
-  // block partials of a separate dot pass
-  int nt = int(m->op.plan.tiles.size());
+    hipLaunchKernelGGL(cg_p_fused_kernel<double>, gb, tb, 0, st, n, int(s->prm.null_space), 0, (const double*)s->part.p,
+                       S, static_cast<const double*>(s->zres), s->p.p);
+  // alpha from the partials of p.w: the operator's tile partials (summed first where they are
+  // many), or (Dirichlet problem) the block partials of a separate dot pass
+  int np = int(m->op.plan.tiles.size());
+  const double* pw = s->ptile.p;
   if (s->dirichlet) {
     launch_dirmv<double>(m, s->p.p, s->w.p, st);
     DotArgs<double> q{};
     q.a[0] = s->p.p;
     q.b[0] = s->w.p;
     hipLaunchKernelGGL(reduce1_kernel<double>, dim3(RED_BLOCKS), dim3(VBLOCK), 0, st, n, q, s->ptile.p);
-    nt = RED_BLOCKS;
+    np = RED_BLOCKS;
   } else {
     launch_cg(m, s->p.p, s->w.p, s->ptile.p, st);
+    if (np > CG_MAX_PART) {
+      hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(RED2_THREADS), 0, st, np, pw, S + S_PROJ);
+      pw = S + S_PROJ;
+      np = 1;
+    }
   }
   const bool x1 = s->nlevels > 1 && s->prm.nu_pre > 0;   // first sweep of the V-cycle fused
-  hipLaunchKernelGGL(cg_alpha_kernel, dim3(1), dim3(RED2_THREADS), 0, st, nt, (const double*)s->ptile.p, S);
   if (mixed)
-    hipLaunchKernelGGL(cg_xr_fused_kernel<float>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)S,
-                       (const double*)s->p.p, (const double*)s->w.p, s->x.p, s->r.p, s->v32[top].b.p,
-                       float(s->om_level[top]), (const float*)s->v32[top].invd.p,
-                       x1 ? s->v32[top].xa.p : s->v32[top].xb.p);
+    hipLaunchKernelGGL(cg_xr_fused_kernel<float>, gb, tb, 0, st, n, np, pw, S, (const double*)s->p.p,
+                       (const double*)s->w.p, s->x.p, s->r.p, s->v32[top].b.p, float(s->om_level[top]),
+                       (const float*)s->v32[top].invd.p, x1 ? s->v32[top].xa.p : s->v32[top].xb.p, s->part_p.p);
   else
-    hipLaunchKernelGGL(cg_xr_fused_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)S,
-                       (const double*)s->p.p, (const double*)s->w.p, s->x.p, s->r.p, (float*)nullptr,
-                       s->om_level[top], (const double*)s->v64[top].invd.p, x1 ? s->v64[top].xa.p : s->v64[top].xb.p);
-  const void* z = precondition_raw(s, s->r.p, st, x1);
-  if (z != s->zres) fail(DGH_ERR_STATE, "V-cycle result buffer changed");
-  if (mixed)
-    hipLaunchKernelGGL(cg_dots_kernel<float>, dim3(DOT_BLOCKS), dim3(VBLOCK), 0, st, n, static_cast<const float*>(z),
-                       (const double*)s->r.p, (const double*)s->w.p, s->part.p);
-  else
-    hipLaunchKernelGGL(cg_dots_kernel<double>, dim3(DOT_BLOCKS), dim3(VBLOCK), 0, st, n, static_cast<const double*>(z),
-                       (const double*)s->r.p, (const double*)s->w.p, s->part.p);
-  hipLaunchKernelGGL(cg_scalar_fused_kernel, dim3(1), dim3(RED2_THREADS), 0, st, (const double*)s->part.p, n,
-                     int(s->prm.null_space), S, int(pnorm), int(mixed));
+    hipLaunchKernelGGL(cg_xr_fused_kernel<double>, gb, tb, 0, st, n, np, pw, S, (const double*)s->p.p,
+                       (const double*)s->w.p, s->x.p, s->r.p, (float*)nullptr, s->om_level[top],
+                       (const double*)s->v64[top].invd.p, x1 ? s->v64[top].xa.p : s->v64[top].xb.p, s->part_p.p);
+}
+
+// The stopping test after an iteration or (init) at the start; dots: on the projected z.
+static void cg_test(dgh_solver s, bool init, bool dots, hipStream_t st) {
+  const uint32_t n = s->meshes[s->nlevels - 1]->N;
+  hipLaunchKernelGGL(cg_test_kernel, dim3(1), dim3(VBLOCK), 0, st, n, int(cg_blocks(n)), (const double*)s->part_p.p,
+                     (const double*)(dots ? s->part.p : nullptr), int(s->prm.null_space), int(init), s->prm.rtol,
+                     s->S.p, s->sig);
+}
+
+// One CG iteration, on device scalars only.  The unpreconditioned norm is known before the V-cycle
+// it would pay for, so there the V-cycle opens the iteration; the preconditioned norm is z's.
+static void cg_iteration(dgh_solver s, hipStream_t st) {
+  if (s->prm.norm_type == DGH_NORM_PRECONDITIONED) {
+    cg_step(s, st);
+    cg_precondition(s, st);
+    cg_test(s, false, true, st);
+  } else {
+    cg_precondition(s, st);
+    cg_step(s, st);
+    cg_test(s, false, false, st);
+  }
+}
+
+// The norm after iteration it (0: the initial one), once the device has written it.
+static double cg_wait(dgh_solver s, int it, hipStream_t st) {
+  const unsigned long long want = static_cast<unsigned long long>(it) + 1ull;
+  for (uint32_t spin = 1; __atomic_load_n(&s->sig->seq, __ATOMIC_ACQUIRE) < want; ++spin) {
+    __builtin_ia32_pause();
+    if (spin % 4096u) continue;
+    const hipError_t q = hipStreamQuery(st);   // an idle or failed stream writes nothing more
+    if (q == hipErrorNotReady) continue;
+    HIP_CHECK(q);
+    if (__atomic_load_n(&s->sig->seq, __ATOMIC_ACQUIRE) < want)
+      fail(DGH_ERR_STATE, "the solve ended without the norm of iteration %d", it);
+  }
+  return s->sig->dp[it & 3];
 }
 
 // Jacobi diagonal of level l (the Dirichlet one, 1 on boundary nodes, for the Dirichlet problem)
@@ -1404,8 +1445,9 @@ int dgh_solver_create(int nlevels, const dgh_mesh* meshes, const dgh_transfer* t
     }
     HIP_CHECK(hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking));
     HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->hS), sizeof(double) * S_NSCAL, hipHostMallocDefault));
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->sig), sizeof(CgSignal), hipHostMallocCoherent));
     s->S.alloc(S_NSCAL);
-    s->part.alloc(size_t(std::max(MAXQ, NDOT)) * RED_BLOCKS);
+    s->part.alloc(size_t(MAXQ) * RED_BLOCKS);
     s->part_p.alloc(MAXQ * RED_BLOCKS);
     // per-level vectors and Jacobi diagonals
     s->v64.resize(nlevels);
@@ -1472,7 +1514,7 @@ int dgh_solver_vcycle(dgh_solver s, const double* r, double* z, void* stream) {
 // PETSc KSPSolve_CG restated (zero initial guess, left preconditioning): see the oracle's
 // or_pcg.  In the FP32-V-cycle mode the preconditioner is inexact and the p-update uses the
 // flexible (Polak-Ribiere) factor z_k.(r_k - r_{k-1}) / z_{k-1}.r_{k-1}.  CG scalars live on
-// the device; the host reads the stopping-test norm once per iteration.
+// the device; the host reads the stopping-test norm of every iteration from pinned memory.
 int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* stats, double* history,
                      int history_len, void* stream) {
   return guarded([&] {
@@ -1501,45 +1543,63 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
       drop_graphs(s);
       s->graph_gen = gen;
     }
-    // r = b (projected), x = 0, p = 0, z = B r, dots
-    hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, b, s->r.p);
-    if (s->prm.null_space) project_mean<double>(s, n, s->r.p, st);
-    hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, s->x.p, 0.0, n);
-    hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, s->p.p, 0.0, n);
+    // r = b (projected), the initial norm
+    s->sig->seq = 0;
+    const double* mean = nullptr;
+    if (s->prm.null_space) {
+      DotArgs<double> d{};
+      d.a[0] = b;
+      reduce<double>(n, d, 1, s->part_p.p, S + S_PROJ, st);
+      mean = S + S_PROJ;
+    }
+    const bool x1 = s->nlevels > 1 && s->prm.nu_pre > 0;
     if (mixed)
-      hipLaunchKernelGGL((convert_kernel<float, double>), dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n,
-                         (const double*)s->r.p, s->v32[top].b.p);
-    s->zres = precondition_raw(s, s->r.p, st);
-    if (mixed)
-      hipLaunchKernelGGL(cg_dots_kernel<float>, dim3(DOT_BLOCKS), dim3(VBLOCK), 0, st, n,
-                         static_cast<const float*>(s->zres), (const double*)s->r.p, (const double*)nullptr, s->part.p);
+      hipLaunchKernelGGL(cg_start_kernel<float>, dim3(cg_blocks(n)), dim3(VBLOCK), 0, st, n, b, mean, s->r.p,
+                         s->v32[top].b.p, float(s->om_level[top]), (const float*)s->v32[top].invd.p,
+                         x1 ? s->v32[top].xa.p : s->v32[top].xb.p, s->part_p.p);
     else
-      hipLaunchKernelGGL(cg_dots_kernel<double>, dim3(DOT_BLOCKS), dim3(VBLOCK), 0, st, n,
-                         static_cast<const double*>(s->zres), (const double*)s->r.p, (const double*)nullptr, s->part.p);
-    hipLaunchKernelGGL(cg_init_fused_kernel, dim3(1), dim3(RED2_THREADS), 0, st, (const double*)s->part.p, n,
-                       int(s->prm.null_space), S, int(pnorm));
-    HIP_CHECK(hipMemcpyAsync(s->hS, S, sizeof(double) * S_NSCAL, hipMemcpyDeviceToHost, st));
-    HIP_CHECK(hipStreamSynchronize(st));
-    const double dp0 = s->hS[S_DP];
-    const double bnorm = std::sqrt(s->hS[S_BB]);
-    double dp = dp0;
-    if (history && history_len > 0) history[0] = dp0;
+      hipLaunchKernelGGL(cg_start_kernel<double>, dim3(cg_blocks(n)), dim3(VBLOCK), 0, st, n, b, mean, s->r.p,
+                         (float*)nullptr, s->om_level[top], (const double*)s->v64[top].invd.p,
+                         x1 ? s->v64[top].xa.p : s->v64[top].xb.p, s->part_p.p);
+    if (pnorm) {
+      hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(RED2_THREADS), 0, st, int(cg_blocks(n)),
+                         (const double*)s->part_p.p, S + S_BB);
+      cg_precondition(s, st);
+      cg_test(s, true, true, st);
+    } else {
+      cg_test(s, true, false, st);
+    }
+    HIP_CHECK(hipGetLastError());
     if (s->prm.use_graph && !s->gexec && !s->coarse_iter) {   // the iterative coarse solve reads back
       HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
       cg_iteration(s, st);
       HIP_CHECK(hipStreamEndCapture(st, &s->graph));
       HIP_CHECK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
     }
-    int it = 0;
-    bool conv = (dp0 == 0.0), bad = false;
-    while (!conv && it < s->prm.max_it) {
+    int queued = 0;
+    auto queue = [&] {
       if (s->gexec)
         HIP_CHECK(hipGraphLaunch(s->gexec, st));
       else
         cg_iteration(s, st);
-      HIP_CHECK(hipMemcpyAsync(&s->hS[S_DP], S + S_DP, sizeof(double), hipMemcpyDeviceToHost, st));
-      HIP_CHECK(hipStreamSynchronize(st));
-      dp = s->hS[S_DP];
+      ++queued;
+    };
+    // While the last two norms put the next one above the tolerance (with a margin of 4), one more
+    // iteration is queued before its norm is read, so the device does not wait for the host (20 us
+    // per iteration, 10% of 630k elements' mixed solve).  DONE stops one queued in vain.
+    const double margin = 4.0;
+    if (s->prm.max_it > 0) queue();
+    const double dp0 = cg_wait(s, 0, st);
+    double dp = dp0, rate = 0.05;   // a V-cycle's usual reduction, until two norms are known
+    if (history && history_len > 0) history[0] = dp0;
+    int it = 0;
+    bool conv = (dp0 == 0.0), bad = false;
+    while (!conv && it < s->prm.max_it) {
+      if (queued == it) queue();
+      if (queued == it + 1 && queued < s->prm.max_it && dp * rate > margin * s->prm.rtol * dp0) queue();
+      const double prev = dp;
+      dp = cg_wait(s, it + 1, st);
+      rate = dp / prev;
       ++it;
       if (history && it < history_len) history[it] = dp;
       if (!std::isfinite(dp)) {
@@ -1548,7 +1608,10 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
       }
       if (dp <= s->prm.rtol * dp0) conv = true;
     }
-    hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)s->x.p, x);
+    if (it > 0)
+      hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, (const double*)s->x.p, x);
+    else
+      hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, x, 0.0, n);
     HIP_CHECK(hipEventRecord(e1, st));
     HIP_CHECK(hipEventSynchronize(e1));
     float ms = 0.f;
@@ -1569,6 +1632,7 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
       reduce<double>(n, q, 1, s->part_p.p, S + S_PROJ, st);
       HIP_CHECK(hipMemcpyAsync(s->hS, S, sizeof(double) * S_NSCAL, hipMemcpyDeviceToHost, st));
       HIP_CHECK(hipStreamSynchronize(st));
+      const double bnorm = std::sqrt(s->hS[S_BB]);
       stats->iterations = it;
       stats->converged = conv ? 1 : 0;
       stats->rnorm0 = dp0;

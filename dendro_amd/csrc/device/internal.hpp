@@ -264,6 +264,7 @@ struct dgh_solver_s {
   DevBuf<double> part;            // reduction partials [MAXQ][RED_BLOCKS]
   DevBuf<double> part_p;          // partials of the null-space projections
   double* hS = nullptr;           // pinned host mirror of S
+  CgSignal* sig = nullptr;        // stopping-test norms, written by the device (pinned host memory)
   DevBuf<double> x, r, z, p, w;   // outer CG vectors (finest, FP64)
   DevBuf<double> ptile;           // per-tile partials of p.w from the operator kernel
   const void* zres = nullptr;     // V-cycle result buffer on the finest level (z, unprojected)
@@ -295,6 +296,7 @@ struct dgh_solver_s {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (hS) (void)hipHostFree(hS);
+    if (sig) (void)hipHostFree(sig);
     if (hcS) (void)hipHostFree(hcS);
     if (st) (void)hipStreamDestroy(st);
   }

@@ -205,71 +205,72 @@ static __global__ void ccg_p_kernel(uint32_t n, const double* __restrict__ S, co
 
 // ---------------------------------------------------------------- CG with device scalars
 // S: RZ = z.r, PW = p.w, DP = stopping-test norm, RATIO = p-update factor, ZZ, ZR, ZW, RR,
-// BB = b.b, ALPHA.
-enum CgScalar { S_RZ = 0, S_PW, S_DP, S_RATIO, S_ZZ, S_ZR, S_ZW, S_RR, S_BB, S_ALPHA, S_PROJ, S_MU, S_NSCAL = 16 };
+// BB = b.b, ALPHA, PROJ (projection sums), MU = mean(z); single right-hand-side solve: RZN = the
+// new z.r until the x update adopts it, ITS = finished iterations, DP0 = initial norm, DONE.
+enum CgScalar { S_RZ = 0, S_PW, S_DP, S_RATIO, S_ZZ, S_ZR, S_ZW, S_RR, S_BB, S_ALPHA, S_PROJ, S_MU, S_RZN, S_ITS,
+                S_DP0, S_DONE, S_NSCAL };
 
-// p = z + ratio p  (VecAYPX)
-static __global__ void cg_p_kernel(uint32_t n, const double* __restrict__ S, const double* __restrict__ z,
-                            double* __restrict__ p) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = z[i] + S[S_RATIO] * p[i];
-}
-
-// a = rz / pw;  x = x + a p;  r = r + (-a) w  (VecAXPY twice)
-static __global__ void cg_xr_kernel(uint32_t n, double* __restrict__ S, const double* __restrict__ p,
-                             const double* __restrict__ w, double* __restrict__ x, double* __restrict__ r) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  const double a = S[S_RZ] / S[S_PW];
-  if (i == 0) S[S_ALPHA] = a;
-  if (i < n) {
-    x[i] = x[i] + a * p[i];
-    r[i] = r[i] + (-a) * w[i];
-  }
-}
+// What the device tells the host about the stopping test, in pinned host memory: the norm after
+// iteration i in dp[i % 4] (i = 0: the initial one), then seq = i + 1.  The host queues at most one
+// iteration ahead of the norms it has read, so four slots are never overwritten unread.
+struct CgSignal {
+  double dp[4];
+  unsigned long long seq;
+};
 
 // ---------------------------------------------------------------- fused CG iteration
 // The preconditioned residual z stays unprojected (FP32 in the mixed solver); its constant
 // null-space component mu = mean(z) is applied where z is used: in the direction update
-// (p' = (z - mu) + beta p, inside the operator kernel) and in the dot products, which come
-// from one pass over z, r, w as
+// (p' = (z - mu) + beta p) and in the dot products, which come from one pass over z, r, w as
 //   z'.z' = z.z - n mu^2,  z'.r = z.r - mu sum(r),  z'.w = z.w - mu sum(w).
-constexpr int NDOT = 7;   // sum z, z.z, z.r, z.w, r.r, sum r, sum w
-enum CgDot { D_SZ = 0, D_ZZ, D_ZR, D_ZW, D_RR, D_SR, D_SW };
-constexpr int DOT_BLOCKS = 1024;  // workgroups of the dot pass (one partial each)
-constexpr int DOT_UNROLL = 2;     // elements per thread and step of the dot pass
-static_assert(NDOT * DOT_BLOCKS <= (MAXQ > NDOT ? MAXQ : NDOT) * RED_BLOCKS, "partials fit the buffer");
+// No kernel of the iteration runs on one workgroup but the stopping test's: the direction update
+// sums the dot pass's partials in every workgroup, the x update those of p.w (at most
+// CG_MAX_PART).  The single-workgroup kernels these replace took 4 us each, of which the sums
+// themselves are about one.
+constexpr int NDOT = 6;   // sum z, z.z, z.r, z.w, sum r, sum w
+enum CgDot { D_SZ = 0, D_ZZ, D_ZR, D_ZW, D_SR, D_SW };
+constexpr int DOT_BLOCKS = 256;      // workgroups of the dot pass (one partial each)
+constexpr int DOT_THREADS = 1024;
+constexpr int CG_UNROLL = 2;         // elements per thread and step of the passes over the vectors
+constexpr int CG_BLOCKS = 2048;      // most workgroups of the direction and x updates (one resident round)
+constexpr int CG_MAX_PART = 2048;    // most partials of p.w every workgroup of the x update sums
+static_assert(NDOT * DOT_BLOCKS <= MAXQ * RED_BLOCKS && CG_BLOCKS <= MAXQ * RED_BLOCKS, "partials fit the buffers");
 
-// Stage 1 of the dots: block partials part[q * DOT_BLOCKS + block] (w == nullptr: z.w and
-// sum w are zero).
+// Workgroups of the direction and x updates of n values.
+inline unsigned cg_blocks(uint32_t n) {
+  const unsigned b = unsigned((n + VBLOCK * CG_UNROLL - 1) / (VBLOCK * CG_UNROLL));
+  return b < 1u ? 1u : b > unsigned(CG_BLOCKS) ? unsigned(CG_BLOCKS) : b;
+}
+
+// Stage 1 of the dots: block partials part[q * DOT_BLOCKS + block].
 template <class TZ>
-__global__ void __launch_bounds__(VBLOCK)
+__global__ void __launch_bounds__(DOT_THREADS)
 cg_dots_kernel(uint32_t n, const TZ* __restrict__ z, const double* __restrict__ r, const double* __restrict__ w,
                double* __restrict__ part) {
-  double s[NDOT] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  // DOT_UNROLL strided elements per step, loaded together
-  constexpr uint32_t STRIDE = DOT_BLOCKS * VBLOCK;
-  for (uint32_t i0 = blockIdx.x * VBLOCK + threadIdx.x; i0 < n; i0 += DOT_UNROLL * STRIDE) {
-    double zi[DOT_UNROLL], ri[DOT_UNROLL], wi[DOT_UNROLL];
+  double s[NDOT] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  // CG_UNROLL strided elements per step, loaded together
+  constexpr uint32_t STRIDE = DOT_BLOCKS * DOT_THREADS;
+  for (uint32_t i0 = blockIdx.x * DOT_THREADS + threadIdx.x; i0 < n; i0 += CG_UNROLL * STRIDE) {
+    double zi[CG_UNROLL], ri[CG_UNROLL], wi[CG_UNROLL];
 #pragma unroll
-    for (int u = 0; u < DOT_UNROLL; ++u) {
+    for (int u = 0; u < CG_UNROLL; ++u) {
       const uint32_t i = i0 + u * STRIDE;
       const bool in = i < n;
       zi[u] = in ? double(z[i]) : 0.0;
       ri[u] = in ? r[i] : 0.0;
-      wi[u] = (in && w) ? w[i] : 0.0;
+      wi[u] = in ? w[i] : 0.0;
     }
 #pragma unroll
-    for (int u = 0; u < DOT_UNROLL; ++u) {
+    for (int u = 0; u < CG_UNROLL; ++u) {
       s[D_SZ] += zi[u];
       s[D_ZZ] += zi[u] * zi[u];
       s[D_ZR] += zi[u] * ri[u];
       s[D_ZW] += zi[u] * wi[u];
-      s[D_RR] += ri[u] * ri[u];
       s[D_SR] += ri[u];
       s[D_SW] += wi[u];
     }
   }
-  __shared__ double red[NDOT][VBLOCK / 64];
+  __shared__ double red[NDOT][DOT_THREADS / 64];
 #pragma unroll
   for (int q = 0; q < NDOT; ++q) {
     const double v = wave_sum(s[q]);
@@ -278,141 +279,207 @@ cg_dots_kernel(uint32_t n, const TZ* __restrict__ z, const double* __restrict__ 
   __syncthreads();
   if (threadIdx.x < NDOT) {
     double t = 0.0;
-    for (int k = 0; k < VBLOCK / 64; ++k) t += red[threadIdx.x][k];
+    for (int k = 0; k < DOT_THREADS / 64; ++k) t += red[threadIdx.x][k];
     part[threadIdx.x * DOT_BLOCKS + blockIdx.x] = t;
   }
 }
 
-// Sums the NDOT x DOT_BLOCKS partials in a fixed order (one RED2_THREADS-thread workgroup:
-// DOT_BLOCKS / RED2_THREADS partials of every quantity per thread, all loads in flight).
-static_assert(DOT_BLOCKS % RED2_THREADS == 0, "whole partials per thread");
+// Sums the NDOT x DOT_BLOCKS partials in a fixed order (workgroups of VBLOCK = DOT_BLOCKS threads).
+static_assert(DOT_BLOCKS == VBLOCK, "one partial of each quantity per thread");
 __device__ __forceinline__ void cg_sum_dots(const double* __restrict__ part, double* out) {
-  constexpr int PPT = DOT_BLOCKS / RED2_THREADS;
-  __shared__ double red[NDOT][RED2_THREADS / 64];
+  __shared__ double red[NDOT][VBLOCK / 64];
   double v[NDOT];
-  double pv[NDOT][PPT];
 #pragma unroll
-  for (int q = 0; q < NDOT; ++q)
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) pv[q][k] = part[q * DOT_BLOCKS + k * RED2_THREADS + threadIdx.x];
-#pragma unroll
-  for (int q = 0; q < NDOT; ++q) {
-    v[q] = pv[q][0];
-#pragma unroll
-    for (int k = 1; k < PPT; ++k) v[q] += pv[q][k];
-  }
+  for (int q = 0; q < NDOT; ++q) v[q] = part[q * DOT_BLOCKS + threadIdx.x];
 #pragma unroll
   for (int q = 0; q < NDOT; ++q) {
     v[q] = wave_sum(v[q]);
     if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = v[q];
   }
   __syncthreads();
+#pragma unroll
   for (int q = 0; q < NDOT; ++q) {
     double t = 0.0;
-    for (int k = 0; k < RED2_THREADS / 64; ++k) t += red[q][k];
+#pragma unroll
+    for (int k = 0; k < VBLOCK / 64; ++k) t += red[q][k];
     out[q] = t;
   }
 }
 
-// Projected dots into S (mu = 0 without a null space).
-__device__ __forceinline__ void cg_projected(const double* d, uint32_t n, int null_space, double* __restrict__ S) {
-  const double mu = null_space ? d[D_SZ] / double(n) : 0.0;
-  S[S_MU] = mu;
-  S[S_ZZ] = d[D_ZZ] - double(n) * mu * mu;
-  S[S_ZR] = d[D_ZR] - mu * d[D_SR];
-  S[S_ZW] = d[D_ZW] - mu * d[D_SW];
-  S[S_RR] = d[D_RR];
-}
-
-// after z = B r: projected dots, dp, the next p-update factor, rz (grid: one workgroup of
-// RED2_THREADS)
-static __global__ void __launch_bounds__(RED2_THREADS)
-cg_scalar_fused_kernel(const double* __restrict__ part, uint32_t n, int null_space, double* __restrict__ S,
-                       int precond_norm, int flexible) {
-  double d[NDOT];
-  cg_sum_dots(part, d);
-  if (threadIdx.x != 0) return;
-  cg_projected(d, n, null_space, S);
-  const double dp = sqrt(precond_norm ? S[S_ZZ] : S[S_RR]);
-  const double ratio = flexible ? (-S[S_ALPHA] * S[S_ZW]) / S[S_RZ] : S[S_ZR] / S[S_RZ];
-  S[S_DP] = dp;
-  S[S_RATIO] = ratio;
-  S[S_RZ] = S[S_ZR];
-}
-
-// before the first iteration (r = b projected, p = 0): rz, dp0, bb, ratio = 0
-static __global__ void __launch_bounds__(RED2_THREADS)
-cg_init_fused_kernel(const double* __restrict__ part, uint32_t n, int null_space, double* __restrict__ S,
-                     int precond_norm) {
-  double d[NDOT];
-  cg_sum_dots(part, d);
-  if (threadIdx.x != 0) return;
-  cg_projected(d, n, null_space, S);
-  S[S_BB] = d[D_RR];
-  S[S_RZ] = S[S_ZR];
-  S[S_DP] = sqrt(precond_norm ? S[S_ZZ] : S[S_BB]);
-  S[S_RATIO] = 0.0;
-}
-
-// p = (z - mu) + beta p  (the projected z with VecAYPX)
-template <class TZ>
-__global__ void cg_p_fused_kernel(uint32_t n, const double* __restrict__ S, const TZ* __restrict__ z,
-                                  double* __restrict__ p) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (double(z[i]) - S[S_MU]) + S[S_RATIO] * p[i];
-}
-
-// p.w = the sum of the operator's tile partials (the order of sum_partials_kernel), and
-// alpha = rz / p.w, into S (grid: one workgroup of RED2_THREADS)
-static __global__ void __launch_bounds__(RED2_THREADS)
-cg_alpha_kernel(int ntiles, const double* __restrict__ part, double* __restrict__ S) {
-  __shared__ double red[RED2_THREADS / 64];
+// part[0] + ... + part[m-1] in the order of sum_partials_kernel (workgroups of VBLOCK threads),
+// the same in every thread.
+static_assert(VBLOCK == RED2_THREADS, "the order of sum_partials_kernel");
+__device__ __forceinline__ double cg_sum_partials(int m, const double* __restrict__ part) {
+  __shared__ double red[VBLOCK / 64];
   double v = 0.0;
-  for (int k = threadIdx.x; k < ntiles; k += RED2_THREADS) v += part[k];
+  for (int k = threadIdx.x; k < m; k += VBLOCK) v += part[k];
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int k = 0; k < VBLOCK / 64; ++k) t += red[k];
+  return t;
+}
+
+// Start of a solve: r = b - sum[0] / n (sum: the projection of a constant null space, or nullptr),
+// the V-cycle's right-hand side and first sweep (see cg_xr_fused_kernel) and block partials of r.r.
+template <class TV>
+__global__ void __launch_bounds__(VBLOCK)
+cg_start_kernel(uint32_t n, const double* __restrict__ b, const double* __restrict__ sum, double* __restrict__ r,
+                float* __restrict__ r32, TV omega, const TV* __restrict__ invd, TV* __restrict__ x1,
+                double* __restrict__ part) {
+  double rr = 0.0;
+  for (uint32_t i = blockIdx.x * VBLOCK + threadIdx.x; i < n; i += gridDim.x * VBLOCK) {
+    const double ri = sum ? b[i] - sum[0] / double(n) : b[i];
+    r[i] = ri;
+    if (r32) r32[i] = float(ri);
+    x1[i] = TV(0) + omega * (TV(ri) * invd[i]);
+    rr += ri * ri;
+  }
+  __shared__ double red[VBLOCK / 64];
+  rr = wave_sum(rr);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rr;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    double pw = 0.0;
-    for (int k = 0; k < RED2_THREADS / 64; ++k) pw += red[k];
-    S[S_PW] = pw;
-    S[S_ALPHA] = S[S_RZ] / pw;
+    double t = 0.0;
+    for (int k = 0; k < VBLOCK / 64; ++k) t += red[k];
+    part[blockIdx.x] = t;
   }
 }
 
-// x = x + alpha p;  r = r + (-alpha) w;  and the V-cycle's first smoothing sweep from zero,
-// x1 = omega (r invd), in the V-cycle's precision TV (mixed: also the FP32 copy of r, r32)
+// After z = B r and the dot pass: the projected dots, the p-update factor (0 in the first
+// iteration; flexible: Polak-Ribiere) and p = (z - mu) + ratio p.
+template <class TZ>
+__global__ void __launch_bounds__(VBLOCK)
+cg_p_fused_kernel(uint32_t n, int null_space, int flexible, const double* __restrict__ part, double* __restrict__ S,
+                  const TZ* __restrict__ z, double* __restrict__ p) {
+  const uint32_t stride = gridDim.x * VBLOCK;
+  uint32_t i0 = blockIdx.x * VBLOCK + threadIdx.x;
+  double zi[CG_UNROLL], pi[CG_UNROLL];
+  auto fetch = [&](uint32_t j) {   // the first values are in flight while the partials are summed
+#pragma unroll
+    for (int u = 0; u < CG_UNROLL; ++u) {
+      const uint32_t i = min(j + u * stride, n - 1u);
+      zi[u] = double(z[i]);
+      pi[u] = p[i];
+    }
+  };
+  fetch(i0);
+  const bool first = S[S_ITS] == 0.0;
+  const double rz = S[S_RZ], alpha = S[S_ALPHA];
+  double d[NDOT];
+  cg_sum_dots(part, d);
+  const double mu = null_space ? d[D_SZ] / double(n) : 0.0;
+  const double zr = d[D_ZR] - mu * d[D_SR];
+  const double zw = d[D_ZW] - mu * d[D_SW];
+  const double ratio = flexible ? (-alpha * zw) / rz : zr / rz;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[S_MU] = mu;
+    S[S_ZR] = zr;
+    S[S_ZW] = zw;
+    S[S_RATIO] = first ? 0.0 : ratio;
+    S[S_RZN] = zr;   // S_RZ itself is still read by the other workgroups
+  }
+  for (; i0 < n; i0 += CG_UNROLL * stride) {
+#pragma unroll
+    for (int u = 0; u < CG_UNROLL; ++u) {
+      const uint32_t i = i0 + u * stride;
+      if (i < n) p[i] = first ? zi[u] - mu : (zi[u] - mu) + ratio * pi[u];
+    }
+    fetch(i0 + CG_UNROLL * stride);
+  }
+}
+
+// alpha = rz / p.w (p.w the sum of npart partials), x = x + alpha p (x = alpha p in the first
+// iteration), r = r + (-alpha) w, the V-cycle's first smoothing sweep from zero,
+// x1 = omega (r invd), in the V-cycle's precision TV (mixed: also the FP32 copy of r, r32), and
+// block partials of r.r -> rrpart.  Nothing moves once the stopping test holds (DONE): the host may
+// have queued this iteration before it knew.
 template <class TV>
 __global__ void __launch_bounds__(VBLOCK)
-cg_xr_fused_kernel(uint32_t n, const double* __restrict__ S, const double* __restrict__ p,
-                   const double* __restrict__ w, double* __restrict__ x, double* __restrict__ r,
-                   float* __restrict__ r32, TV omega, const TV* __restrict__ invd, TV* __restrict__ x1) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double a = S[S_ALPHA];
-  x[i] = x[i] + a * p[i];
-  const double ri = r[i] + (-a) * w[i];
-  r[i] = ri;
-  if (r32) r32[i] = float(ri);
-  x1[i] = TV(0) + omega * (TV(ri) * invd[i]);
+cg_xr_fused_kernel(uint32_t n, int npart, const double* __restrict__ part, double* __restrict__ S,
+                   const double* __restrict__ p, const double* __restrict__ w, double* __restrict__ x,
+                   double* __restrict__ r, float* __restrict__ r32, TV omega, const TV* __restrict__ invd,
+                   TV* __restrict__ x1, double* __restrict__ rrpart) {
+  const uint32_t stride = gridDim.x * VBLOCK;
+  uint32_t i0 = blockIdx.x * VBLOCK + threadIdx.x;
+  double pi[CG_UNROLL], wi[CG_UNROLL], xi[CG_UNROLL], ri[CG_UNROLL];
+  TV di[CG_UNROLL];
+  auto fetch = [&](uint32_t j) {   // the first values are in flight while the partials are summed
+#pragma unroll
+    for (int u = 0; u < CG_UNROLL; ++u) {
+      const uint32_t i = min(j + u * stride, n - 1u);
+      pi[u] = p[i];
+      wi[u] = w[i];
+      xi[u] = x[i];
+      ri[u] = r[i];
+      di[u] = invd[i];
+    }
+  };
+  fetch(i0);
+  const bool done = S[S_DONE] != 0.0, first = S[S_ITS] == 0.0;
+  const double rz = S[S_RZN];
+  const double pw = cg_sum_partials(npart, part);
+  const double a = rz / pw;
+  if (done) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[S_PW] = pw;
+    S[S_ALPHA] = a;
+    S[S_RZ] = rz;
+  }
+  double rr = 0.0;
+  for (; i0 < n; i0 += CG_UNROLL * stride) {
+#pragma unroll
+    for (int u = 0; u < CG_UNROLL; ++u) {
+      const uint32_t i = i0 + u * stride;
+      if (i < n) {
+        x[i] = first ? a * pi[u] : xi[u] + a * pi[u];
+        const double rn = ri[u] + (-a) * wi[u];
+        r[i] = rn;
+        if (r32) r32[i] = float(rn);
+        x1[i] = TV(0) + omega * (TV(rn) * di[u]);
+        rr += rn * rn;
+      }
+    }
+    fetch(i0 + CG_UNROLL * stride);
+  }
+  __shared__ double red[VBLOCK / 64];
+  rr = wave_sum(rr);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rr;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int k = 0; k < VBLOCK / 64; ++k) t += red[k];
+    rrpart[blockIdx.x] = t;
+  }
 }
 
-// after z = B r and the dots: dp, the next p-update factor, rz
-static __global__ void cg_scalar_kernel(double* __restrict__ S, int precond_norm, int flexible) {
-  if (threadIdx.x != 0) return;
-  const double dp = sqrt(precond_norm ? S[S_ZZ] : S[S_RR]);
-  const double ratio = flexible ? (-S[S_ALPHA] * S[S_ZW]) / S[S_RZ] : S[S_ZR] / S[S_RZ];
+// Stopping test (one workgroup): the norm of r (npart partials of r.r) or, dots given, of the
+// projected z; init: the initial norm, iteration count 0.  Sets DP, DONE and tells the host.
+static __global__ void __launch_bounds__(VBLOCK)
+cg_test_kernel(uint32_t n, int npart, const double* __restrict__ rrpart, const double* __restrict__ dots,
+               int null_space, int init, double rtol, double* __restrict__ S, CgSignal* sig) {
+  const bool done = !init && S[S_DONE] != 0.0;
+  const double its = init ? 0.0 : S[S_ITS] + 1.0, dp0 = S[S_DP0];
+  double v;
+  if (dots) {
+    double d[NDOT];
+    cg_sum_dots(dots, d);
+    const double mu = null_space ? d[D_SZ] / double(n) : 0.0;
+    v = d[D_ZZ] - double(n) * mu * mu;
+  } else {
+    v = cg_sum_partials(npart, rrpart);
+    if (init && threadIdx.x == 0) S[S_BB] = v;
+  }
+  if (threadIdx.x != 0 || done) return;
+  const double dp = sqrt(v);
   S[S_DP] = dp;
-  S[S_RATIO] = ratio;
-  S[S_RZ] = S[S_ZR];
-}
-
-// before the first iteration: rz, dp0, ratio = 0 (p starts at zero)
-static __global__ void cg_init_kernel(double* __restrict__ S, int precond_norm) {
-  if (threadIdx.x != 0) return;
-  S[S_RZ] = S[S_ZR];
-  S[S_DP] = sqrt(precond_norm ? S[S_ZZ] : S[S_BB]);
-  S[S_RATIO] = 0.0;
+  S[S_ITS] = its;
+  if (init) S[S_DP0] = dp;
+  S[S_DONE] = (init ? dp == 0.0 : !(dp > rtol * dp0)) ? 1.0 : 0.0;
+  __hip_atomic_store(&sig->dp[int(its) & 3], dp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&sig->seq, static_cast<unsigned long long>(its) + 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <class T>
