@@ -153,6 +153,41 @@ static void launch_smooth(dgh_mesh m, const T* x, const T* b, const T* invd, T o
   launch_op<T, OP_SMOOTH>(m, x, OpIO<T>{x_out, b, invd, omega}, st);
 }
 
+// Whether two sweeps of the mesh run in one launch.
+template <class T>
+static bool op_paired(const dgh_mesh m) {
+  return op_factored(m) && !m->pair.plan.tiles.empty() && (sizeof(T) == 4 || m->E <= PAIR_MAX_ELEMS64);
+}
+
+// x = the iterate after one sweep of x, y and r as PairMode says
+template <class T, int MODE>
+static void launch_pair(dgh_mesh m, const T* x, const PairIO<T>& io, hipStream_t st) {
+  const DevTiles& d = m->pair;
+  const int nt = int(d.plan.tiles.size());
+  const unsigned grid = unsigned(NXCD * ((nt + NXCD - 1) / NXCD));
+  const size_t lds = sizeof(T) == 8 ? d.lds64 : d.lds32;
+  const T *kap, *mas;
+  if constexpr (sizeof(T) == 8) {
+    kap = d.rk64.p;
+    mas = d.rm64.p;
+  } else {
+    kap = d.rk32.p;
+    mas = d.rm32.p;
+  }
+  const double u1 = m->lap_fac * m->hFac / 2.0, u2 = m->mass_fac * m->hFac * m->hFac * m->hFac / 8.0;
+#define DGH_PAIR_LAUNCH(MASS, UNI)                                                                                   \
+  hipLaunchKernelGGL((tile_pair_kernel<T, MASS, MODE, UNI>), dim3(grid), dim3(PAIR_BLOCK), lds, st, d.tiles.p,         \
+                     d.node_tab.p, x, d.lid.p, d.texp.p, nt, d.pitch, kap, mas, io, u1, u2, m->maxD)
+  if (!kap)
+    DGH_PAIR_LAUNCH(true, true);
+  else if (!mas)
+    DGH_PAIR_LAUNCH(false, false);
+  else
+    DGH_PAIR_LAUNCH(true, false);
+#undef DGH_PAIR_LAUNCH
+  HIP_CHECK(hipGetLastError());
+}
+
 // c = R f; with x1 given, also x1 = omega (c * invd) (the first sweep on the coarse level)
 // Boundary flags of a transfer's two meshes when both carry them (Dirichlet problem): the
 // transfers then drop every entry that touches a boundary node (the suppressed DOFs of
@@ -310,6 +345,8 @@ static std::vector<uint16_t> pack_records(const TilePlan& plan) {
   return p;
 }
 
+static void upload_pitched(DevTiles& d);
+
 // (Re)builds a tiling with the largest tile size <= T whose LDS need (lds(d)) fits; with
 // budget > 0 tiles also end before their owned plus touched nodes exceed the budget, and with
 // block > 0 (single right-hand-side operator) the owned nodes get the fixed capacity
@@ -334,16 +371,7 @@ void build_devtiles(dgh_mesh m, DevTiles& d, uint32_t T, size_t (*lds)(const Dev
   const std::vector<uint16_t> packed = pack_records(d.plan);
   d.lid.upload(packed.data(), packed.size());
   if (block > 0) {   // single right-hand-side kernels: a fixed pitch, padded with each tile's last node
-    d.pitch = d.plan.max_touch;
-    std::vector<uint32_t> tab(d.plan.tiles.size() * size_t(d.pitch));
-    for (size_t t = 0; t < d.plan.tiles.size(); ++t) {
-      const TileRec& tr = d.plan.tiles[t];
-      const uint32_t* src = d.plan.node_tab.data() + tr.node_off;
-      uint32_t* dst = tab.data() + t * d.pitch;
-      std::copy(src, src + tr.n_touch, dst);
-      std::fill(dst + tr.n_touch, dst + d.pitch, src[tr.n_touch - 1]);
-    }
-    d.node_tab.upload(tab.data(), tab.size());
+    upload_pitched(d);
   } else {
     d.node_tab.upload(d.plan.node_tab.data(), d.plan.node_tab.size());
   }
@@ -351,6 +379,44 @@ void build_devtiles(dgh_mesh m, DevTiles& d, uint32_t T, size_t (*lds)(const Dev
 }
 
 static size_t op_lds_f64(const DevTiles& d) { return d.lds64; }
+
+// node_tab at a fixed pitch, padded with each tile's last node.
+static void upload_pitched(DevTiles& d) {
+  d.pitch = d.plan.max_touch;
+  std::vector<uint32_t> tab(d.plan.tiles.size() * size_t(d.pitch));
+  for (size_t t = 0; t < d.plan.tiles.size(); ++t) {
+    const TileRec& tr = d.plan.tiles[t];
+    const uint32_t* src = d.plan.node_tab.data() + tr.node_off;
+    uint32_t* dst = tab.data() + t * d.pitch;
+    std::copy(src, src + tr.n_touch, dst);
+    std::fill(dst + tr.n_touch, dst + d.pitch, src[tr.n_touch - 1]);
+  }
+  d.node_tab.upload(tab.data(), tab.size());
+}
+
+// Two-sweep tiles of a mesh that a V-cycle smooths (once per mesh).
+static void build_pair(dgh_mesh m) {
+  if (m->pair_tried) return;
+  m->pair_tried = true;
+  if (m->E > PAIR_MAX_ELEMS) return;
+  DevTiles& d = m->pair;
+  for (uint32_t T = std::max(32u, m->E / 256u);; T /= 2) {   // one tile per CU; E/128 and E/512 within 2%
+    build_pair_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), T, d.plan);
+    if (d.plan.max_touch <= uint32_t(PAIR_XC * PAIR_BLOCK) && d.plan.max_own <= uint32_t(PAIR_OC * PAIR_BLOCK)) break;
+    if (T < 16) {   // too dense a neighbourhood: single sweeps
+      d.plan = TilePlan();
+      return;
+    }
+  }
+  d.block = PAIR_BLOCK;
+  d.lds64 = uint32_t(tile_lds_bytes<double>(PAIR_BLOCK, d.plan.max_touch));
+  d.lds32 = uint32_t(tile_lds_bytes<float>(PAIR_BLOCK, d.plan.max_touch));
+  d.tiles.upload(d.plan.tiles.data(), d.plan.tiles.size());
+  const std::vector<uint16_t> packed = pack_records(d.plan);
+  d.lid.upload(packed.data(), packed.size());
+  upload_pitched(d);
+  upload_coefs(m, d);
+}
 
 // Node budget of a single right-hand-side tile for a block size: the LDS share that lets the
 // wave limit (32 wavefronts per CU) rather than LDS bound the workgroups per CU, less a
@@ -539,11 +605,24 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
   if (!x1_ready)
     hipLaunchKernelGGL(smooth_first_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, om, b,
                        (const T*)V.invd.p, xc);
-  for (int it = 1; it < s->prm.nu_pre; ++it) {
-    sweep(xc, xn);
+  const bool paired = !split && op_paired<T>(m);
+  auto sweeps = [&](int n_sweeps) {
+    int it = 0;
+    for (; paired && it + 2 <= n_sweeps; it += 2) {
+      launch_pair<T, PAIR_SMOOTH>(m, xc, PairIO<T>{xn, nullptr, b, V.invd.p, om}, st);
+      std::swap(xc, xn);
+    }
+    for (; it < n_sweeps; ++it) {
+      sweep(xc, xn);
+      std::swap(xc, xn);
+    }
+  };
+  const bool pair_resid = paired && s->prm.nu_pre % 2 == 0;   // the last of nu_pre - 1 sweeps and the residual
+  sweeps(s->prm.nu_pre - 1 - (pair_resid ? 1 : 0));
+  if (pair_resid) {
+    launch_pair<T, PAIR_RESID>(m, xc, PairIO<T>{xn, V.r.p, b, V.invd.p, om}, st);
     std::swap(xc, xn);
-  }
-  if (split) {
+  } else if (split) {
     apply(xc);
     hipLaunchKernelGGL(resid_vec_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, b, (const T*)V.r.p, V.r.p);
   } else {
@@ -556,10 +635,7 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
     launch_restrict<T>(s->transfers[l - 1], V.r.p, C.b.p, st);
   T* xcoarse = vcycle<T>(s, l - 1, C.b.p, st, l - 1 > 0 && s->prm.nu_pre > 0);
   launch_prolong<T>(s->transfers[l - 1], xcoarse, xc, xc, st);
-  for (int it = 0; it < s->prm.nu_post; ++it) {
-    sweep(xc, xn);
-    std::swap(xc, xn);
-  }
+  sweeps(s->prm.nu_post);
   return xc;
 }
 
@@ -1126,6 +1202,7 @@ int dgh_mesh_set_coefficients(dgh_mesh m, const double* kappa, const double* mas
     if (mass) m->h_mass.assign(mass, mass + m->E);
     upload_coefs(m, m->op);
     if (!m->mop.plan.tiles.empty()) upload_coefs(m, m->mop);
+    if (!m->pair.plan.tiles.empty()) upload_coefs(m, m->pair);
     ++m->coef_gen;
   });
 }
@@ -1449,6 +1526,9 @@ int dgh_solver_create(int nlevels, const dgh_mesh* meshes, const dgh_transfer* t
     s->S.alloc(S_NSCAL);
     s->part.alloc(size_t(MAXQ) * RED_BLOCKS);
     s->part_p.alloc(MAXQ * RED_BLOCKS);
+    if (!s->dirichlet)
+      for (int l = 1; l < nlevels; ++l)
+        if (params->coarse_op == DGH_COARSE_JAC2 || l == nlevels - 1) build_pair(meshes[l]);
     // per-level vectors and Jacobi diagonals
     s->v64.resize(nlevels);
     if (params->vcycle_prec == DGH_F32) s->v32.resize(nlevels);

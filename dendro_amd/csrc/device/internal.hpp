@@ -71,6 +71,14 @@ constexpr size_t CLASS_ROWS_MIN_TILES = 1024;
 // 1024-thread tiles, from LARGE_MESH_ELEMS up of at most 8192 elements.
 constexpr uint32_t MID_MESH_ELEMS = 1200000;
 constexpr uint32_t LARGE_MESH_ELEMS = 4000000;
+// Largest mesh smoothed two sweeps per launch (build_pair).  The first sweep of a tile takes 7 times
+// its elements' records (a single sweep 1.5 to 2), which a launch of a small mesh has room for: V-cycle
+// with the levels up to 60k elements paired / single, FP64: finest 11k elements 86.1 / 96.7 us, 64k 107.2 /
+// 110.5, 297k 147.8 / 148.4, where its level of 37k gains nothing; pairing levels of 64k and 100k
+// elements too 113.4 and 156.2.  FP32, whose records cost half: mixed PCG of 631k elements 1941 us
+// single, 1924 with the level of 10k paired, 1900 with that of 41k too.
+constexpr uint32_t PAIR_MAX_ELEMS = 60000;
+constexpr uint32_t PAIR_MAX_ELEMS64 = 20000;
 // Largest coarsest level solved with a dense inverse (n^2 doubles on the host and the device).
 constexpr int COARSE_DENSE_LIMIT = 40000;
 
@@ -173,6 +181,8 @@ struct dgh_mesh_s {
   DevTiles op;
   int block = 512;              // threads per operator workgroup (256, 512 or 1024)
   DevTiles mop;
+  DevTiles pair;                // two sweeps per launch (build_pair; no tiles: the mesh takes single ones)
+  bool pair_tried = false;
   uint32_t mtile = 0;           // batched tile size (0: default)
   int mvariant = 6;             // batched FP32 products (multi_api.hip): 1 matrix cores, others vector ALUs
   uint64_t gen = 0;             // bumped whenever device tilings or coefficients are rebuilt

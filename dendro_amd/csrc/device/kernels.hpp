@@ -720,6 +720,141 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
   }
 }
 
+// Two applications of the operator in one launch, for meshes whose single sweeps are a chain of
+// latencies: a sweep x' = x + omega (invd (b - A x)), then PAIR_SMOOTH: another one, y = x'';
+// PAIR_RESID: y = x' and r = b - A x'.  A tile (build_pair_tiles) updates all nodes of its own
+// records in the first sweep, so neighbouring tiles repeat the sweep on each other's border nodes
+// instead of exchanging them through memory and a launch.  A single sweep of a small mesh takes 4.5
+// to 5 us in a chain of dependent launches, most of it the launch and two hops to memory; the second
+// sweep here adds about 3: mixed PCG of 37k elements 1258 -> 1090 us.
+enum PairMode { PAIR_SMOOTH = 0, PAIR_RESID = 1 };
+template <class T>
+struct PairIO {
+  T* y;
+  T* r;            // PAIR_RESID
+  const T* b;
+  const T* invd;
+  T omega;
+};
+constexpr int PAIR_BLOCK = 512;
+constexpr int PAIR_XC = 4;   // touched and first-sweep nodes per thread, at most
+constexpr int PAIR_OC = 3;
+
+template <class T, bool MASS, int MODE, bool UNI>
+__global__ void __launch_bounds__(PAIR_BLOCK)
+tile_pair_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ node_tab, const T* __restrict__ x,
+                 const uint16_t* __restrict__ lid, const int2* __restrict__ texp, int ntiles, uint32_t pitch,
+                 const T* __restrict__ kappa, const T* __restrict__ mass, PairIO<T> io, double u1, double u2,
+                 uint32_t maxD) {
+  constexpr int BLOCK = PAIR_BLOCK, NW = BLOCK / 64;
+  constexpr uint32_t XS = tile_xs_off<T, BLOCK>();
+  static_assert(PAIR_OC * BLOCK <= int(op_own_cap(BLOCK)), "the first sweep's sums fit");
+  const lds_ptr<fx_acc_t<T>> acc = lds_at<fx_acc_t<T>>(0);
+  const lds_ptr<T> xs = lds_at<T>(XS);
+  const lds_ptr<uint32_t> s_xhi = lds_at<uint32_t>(tile_xhi_off<T, BLOCK>());
+  const int t = xcd_tile(blockIdx.x, ntiles);
+  if (t >= ntiles) return;
+  const TileRec rec = tiles[t];
+  const uint32_t* nodes = node_tab + size_t(t) * pitch;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t w0 = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x - lane)));
+  RecF<T> R;
+  auto load = [&](RecF<T>& r, uint32_t r0) {
+    load_rec_fact<T, MASS, UNI>(r, rec.elem_off + min(r0 + lane, rec.n_elem - 1u), lid, kappa, mass);
+  };
+  // slots past the end are clamped to the last node, as in tile_op_kernel
+  uint32_t nid[PAIR_XC];
+  const uint32_t last = pitch - 1u;
+#pragma unroll
+  for (int q = 0; q < PAIR_XC; ++q) nid[q] = nodes[min(threadIdx.x + uint32_t(q * BLOCK), last)];
+  load(R, w0);
+  T v[PAIR_XC], ob[PAIR_OC], od[PAIR_OC];
+#pragma unroll
+  for (int q = 0; q < PAIR_XC; ++q) v[q] = x[nid[q]];
+#pragma unroll
+  for (int q = 0; q < PAIR_OC; ++q) {
+    ob[q] = io.b[nid[q]];
+    od[q] = io.invd[nid[q]];
+  }
+  uint32_t xhi = 0;
+  auto take = [&](T val) {   // FP32 bits order as |x| does, converted by max_x
+    if constexpr (sizeof(T) == 8)
+      xhi = max(xhi, uint32_t(uint64_t(__double_as_longlong(val)) >> 32) & 0x7fffffffu);
+    else
+      xhi = max(xhi, __float_as_uint(val) & 0x7fffffffu);
+  };
+  auto wave_max = [&] {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) xhi = max(xhi, uint32_t(__shfl_xor(int(xhi), off)));
+    if (lane == 0) s_xhi[threadIdx.x >> 6] = xhi;
+  };
+  auto max_x = [&] {   // high word of the tile's max |x|
+#pragma unroll
+    for (int w = 0; w < NW; ++w) xhi = max(xhi, s_xhi[w]);
+    if constexpr (sizeof(T) == 4)
+      xhi = uint32_t(uint64_t(__double_as_longlong(double(__uint_as_float(xhi)))) >> 32);
+  };
+#pragma unroll
+  for (int q = 0; q < PAIR_XC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i < rec.n_touch) xs[i] = v[q];
+    take(v[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < PAIR_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i < rec.n_own) acc[i] = 0;
+  }
+  wave_max();
+  __syncthreads();
+  max_x();
+  bool finite = (xhi >> 20) < 0x7ffu;
+  int es = fx_scale<T>(texp[t], fx_ex<T>(xhi));
+  auto sweep = [&](uint32_t n_elem, uint32_t n_own) {
+    const uint32_t own_bytes = n_own * uint32_t(sizeof(T));
+    for (uint32_t r0 = w0; r0 < n_elem; r0 += BLOCK) {
+      RecF<T> Rn;
+      // the last round loads the first records again, for the next sweep
+      load(Rn, r0 + BLOCK < n_elem ? r0 + BLOCK : w0);
+      eval_fact<T, MASS, XS, UNI>(R, r0 + lane < n_elem ? own_bytes : 0u, es, u1, u2, maxD);
+      R = Rn;
+    }
+  };
+  sweep(rec.n_elem, rec.n_own);
+  __syncthreads();
+  xhi = 0;
+#pragma unroll
+  for (int q = 0; q < PAIR_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i < rec.n_own) {
+      const T a = finite ? T(fx_value<T>(acc[i], es)) : T(__builtin_nan(""));
+      const T xn = xs[i] + io.omega * ((ob[q] - a) * od[q]);
+      xs[i] = xn;
+      acc[i] = 0;
+      take(xn);
+    }
+  }
+  wave_max();
+  __syncthreads();
+  max_x();
+  finite = (xhi >> 20) < 0x7ffu;
+  es = fx_scale<T>(texp[t], fx_ex<T>(xhi));
+  sweep(rec.n_elem2, rec.n_own2);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PAIR_OC; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q * BLOCK);
+    if (i >= rec.n_own2) break;
+    const T a = finite ? T(fx_value<T>(acc[i], es)) : T(__builtin_nan(""));
+    if (MODE == PAIR_SMOOTH) {
+      io.y[nid[q]] = xs[i] + io.omega * ((ob[q] - a) * od[q]);
+    } else {
+      io.y[nid[q]] = xs[i];
+      io.r[nid[q]] = ob[q] - a;
+    }
+  }
+}
+
 // f_out[j] = f_in[j] + sum_k W[s][pos][k] c[cnl[k]] for every fine node j (prolongation
 // P = R^T): the coarse shape functions of the coarse element holding node j.
 template <class T>

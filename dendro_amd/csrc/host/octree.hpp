@@ -51,7 +51,9 @@ struct TileRec {
   uint32_t node_off;   // first entry of the tile's node table
   uint32_t n_touch;    // nodes touched by the records (owned first)
   uint32_t n_own;      // nodes owned (stored) by the tile
-  uint32_t pad[3];
+  uint32_t n_elem2;    // two-sweep tiles: records of the second sweep (they come first),
+  uint32_t n_own2;     // and nodes the tile stores (n_own: nodes the first sweep updates)
+  uint32_t pad;
 };
 struct TilePlan {
   uint32_t tile_elems = 0;          // element cap per tile
@@ -71,6 +73,13 @@ struct TilePlan {
 // (the owned-node sums then sit in a fixed-size LDS region ahead of the staged x).
 void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                  const uint8_t* lev, uint32_t T, TilePlan& plan, uint32_t budget = 0, uint32_t own_cap = 0);
+// Tiles of T consecutive elements for two sweeps in one launch (budget and own_cap unused).  The
+// tile's second sweep needs what a tile of build_tiles holds: the nodes it owns (n_own2, first in
+// its node list) and the records touching them (n_elem2, its first records).  Its first sweep
+// updates every node of those records (n_own), which takes all records touching them (n_elem), and
+// reads the nodes of those (n_touch).
+void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                      const uint8_t* lev, uint32_t T, TilePlan& plan);
 // Tile boundaries alone: bounds[t] = first element of tile t, bounds.back() = E.
 void tile_bounds(uint32_t E, uint32_t N, const uint32_t* nl, uint32_t T, uint32_t budget,
                  std::vector<uint32_t>& bounds, uint32_t own_cap = 0);

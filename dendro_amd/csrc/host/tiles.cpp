@@ -124,6 +124,93 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
   build(bounds);
 }
 
+// Child-0 type of every element's mirrored hanging mask.
+static std::vector<uint8_t> element_types(uint32_t E, const uint8_t* child, const uint8_t* hn) {
+  std::vector<int8_t> type_of(8 * 256);
+  for (int c = 0; c < 8; ++c)
+    for (int h = 0; h < 256; ++h) type_of[c * 256 + h] = int8_t(etype_of(0, mirror_mask(uint8_t(h), c)));
+  std::vector<uint8_t> tp(E);
+  for (uint32_t e = 0; e < E; ++e) {
+    const int t0 = type_of[child[e] * 256 + hn[e]];
+    if (t0 < 0) fail(DGH_ERR_MESH, "element %u: mirrored hanging mask is not a child-0 type", e);
+    tp[e] = uint8_t(t0);
+  }
+  return tp;
+}
+
+// Orders a tile's records (of one sweep).  Classes: child-0 type, then level (uniform coefficients
+// read one element matrix per (type, level) class); a counting sort keeps the Morton order inside a
+// class.  cls_end (1024 entries) and sorted are scratch.
+static void order_records(uint32_t* recs, size_t n, const uint8_t* tp, const uint8_t* lev,
+                          std::vector<uint32_t>& cls_end, std::vector<uint32_t>& sorted) {
+  auto cls = [&](uint32_t e) { return (uint32_t(tp[e]) << 5) | lev[e]; };
+  std::fill(cls_end.begin(), cls_end.end(), 0u);
+  for (size_t i = 0; i < n; ++i) ++cls_end[cls(recs[i])];
+  uint32_t at = 0;
+  for (uint32_t& c : cls_end) {
+    const uint32_t m = c;
+    c = at;
+    at += m;
+  }
+  sorted.resize(n);
+  for (size_t i = 0; i < n; ++i) sorted[cls_end[cls(recs[i])]++] = recs[i];
+  // Inside each class, deal the Morton-ordered records round-robin over the class's
+  // wavefronts: the 64 lanes of a wavefront then hold elements about n/64 apart, so
+  // siblings (which share the parent-centre node after the mirror permutation) do
+  // not collide on one LDS address in the same atomic instruction.
+  size_t q = 0;
+  for (size_t a = 0; a < sorted.size();) {
+    const size_t b = cls_end[cls(sorted[a])], W = (b - a + 63) / 64;
+    for (size_t w = 0; w < W; ++w)
+      for (size_t i = a + w; i < b; i += W) recs[q++] = sorted[i];
+    a = b;
+  }
+}
+
+// Joins the per-tile records, node lists and ids into the plan.
+static void concatenate(const std::vector<std::vector<uint32_t>>& t_rec, const std::vector<std::vector<uint32_t>>& t_nodes,
+                        const std::vector<std::vector<uint16_t>>& t_lid, const std::vector<uint8_t>& tp,
+                        const uint8_t* lev, TilePlan& plan) {
+  const uint32_t ntiles = uint32_t(plan.tiles.size());
+  size_t R = 0, NT = 0;
+  for (uint32_t t = 0; t < ntiles; ++t) {
+    plan.tiles[t].elem_off = uint32_t(R);
+    plan.tiles[t].node_off = uint32_t(NT);
+    R += t_rec[t].size();
+    NT += t_nodes[t].size();
+    plan.max_touch = std::max(plan.max_touch, plan.tiles[t].n_touch);
+    plan.max_own = std::max(plan.max_own, plan.tiles[t].n_own);
+    plan.max_elem = std::max(plan.max_elem, plan.tiles[t].n_elem);
+    plan.max_slots = std::max(plan.max_slots, plan.tiles[t].n_own + plan.tiles[t].n_touch);
+  }
+  if (R > 0xffffffffu || NT > 0xffffffffu) fail(DGH_ERR_ARG, "mesh too large for 32-bit tile offsets");
+  plan.rec_elem.resize(R);
+  plan.meta.resize(R);
+  plan.lid.resize(R * 8);
+  plan.node_tab.resize(NT);
+  for (uint32_t t = 0; t < ntiles; ++t) {
+    const size_t ro = plan.tiles[t].elem_off, no = plan.tiles[t].node_off;
+    std::copy(t_rec[t].begin(), t_rec[t].end(), plan.rec_elem.begin() + ro);
+    std::copy(t_lid[t].begin(), t_lid[t].end(), plan.lid.begin() + ro * 8);
+    std::copy(t_nodes[t].begin(), t_nodes[t].end(), plan.node_tab.begin() + no);
+    for (size_t r = 0; r < t_rec[t].size(); ++r) {
+      const uint32_t e = t_rec[t][r];
+      plan.meta[ro + r] = uint16_t(tp[e] | (uint16_t(lev[e]) << 5));
+    }
+  }
+}
+
+// Runs f(worker, tile) for every tile on a few threads.
+template <class F>
+static void for_tiles(uint32_t ntiles, F f) {
+  unsigned nt = std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
+  nt = std::min(nt, std::max(1u, ntiles / 16u));   // a worker's start costs as much as a dozen small tiles
+  std::vector<std::thread> th;
+  for (unsigned w = 0; w < nt; ++w)
+    th.emplace_back([&f, w, nt, ntiles] { f(w, nt, ntiles); });
+  for (auto& x : th) x.join();
+}
+
 static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                               const uint8_t* lev, const std::vector<uint32_t>& bounds, TilePlan& plan) {
   const uint32_t ntiles = uint32_t(bounds.size() - 1);
@@ -165,26 +252,13 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
     std::vector<uint32_t> fillp(own_cnt.begin(), own_cnt.end() - 1);
     for (uint32_t n = 0; n < N; ++n) owned[fillp[owner[n]]++] = n;
   }
-  // element class t' (child-0 type of the mirrored mask), by child and mask
-  std::vector<int8_t> type_of(8 * 256);
-  for (int c = 0; c < 8; ++c)
-    for (int h = 0; h < 256; ++h) type_of[c * 256 + h] = int8_t(etype_of(0, mirror_mask(uint8_t(h), c)));
-  std::vector<uint8_t> tp(E);
-  for (uint32_t e = 0; e < E; ++e) {
-    const int t0 = type_of[child[e] * 256 + hn[e]];
-    if (t0 < 0) fail(DGH_ERR_MESH, "element %u: mirrored hanging mask is not a child-0 type", e);
-    tp[e] = uint8_t(t0);
-  }
+  const std::vector<uint8_t> tp = element_types(E, child, hn);   // child-0 type t'
   // per-tile records, built in parallel (each worker keeps a dense node -> local id map)
   plan.tiles.resize(ntiles);
   std::vector<std::vector<uint32_t>> t_rec(ntiles), t_nodes(ntiles);
   std::vector<std::vector<uint16_t>> t_lid(ntiles);
-  unsigned nt = std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
-  nt = std::min(nt, std::max(1u, ntiles / 16u));   // a worker's start costs as much as a dozen small tiles
-  std::vector<std::thread> th;
-  std::vector<int> err(nt, 0);
-  for (unsigned w = 0; w < nt; ++w) {
-    th.emplace_back([&, w] {
+  std::vector<int> err(16, 0);
+  for_tiles(ntiles, [&](unsigned w, unsigned nt, uint32_t) {
       std::vector<int32_t> lid_of(N, -1);
       std::vector<uint32_t> cls_end(1024), sorted;
       for (uint32_t t = w; t < ntiles; t += nt) {
@@ -193,30 +267,7 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
         recs.resize(e1 - e0);
         std::iota(recs.begin(), recs.end(), e0);
         recs.insert(recs.end(), halo[t].begin(), halo[t].end());
-        // classes: child-0 type, then level (uniform coefficients read one element matrix
-        // per (type, level) class); a counting sort keeps the Morton order inside a class
-        auto cls = [&](uint32_t e) { return (uint32_t(tp[e]) << 5) | lev[e]; };
-        std::fill(cls_end.begin(), cls_end.end(), 0u);
-        for (uint32_t e : recs) ++cls_end[cls(e)];
-        uint32_t at = 0;
-        for (uint32_t& c : cls_end) {
-          const uint32_t n = c;
-          c = at;
-          at += n;
-        }
-        sorted.resize(recs.size());
-        for (uint32_t e : recs) sorted[cls_end[cls(e)]++] = e;
-        // Inside each class, deal the Morton-ordered records round-robin over the class's
-        // wavefronts: the 64 lanes of a wavefront then hold elements about n/64 apart, so
-        // siblings (which share the parent-centre node after the mirror permutation) do
-        // not collide on one LDS address in the same atomic instruction.
-        size_t q = 0;
-        for (size_t a = 0; a < sorted.size();) {
-          const size_t b = cls_end[cls(sorted[a])], W = (b - a + 63) / 64;
-          for (size_t w2 = 0; w2 < W; ++w2)
-            for (size_t i = a + w2; i < b; i += W) recs[q++] = sorted[i];
-          a = b;
-        }
+        order_records(recs.data(), recs.size(), tp.data(), lev, cls_end, sorted);
         auto& nodes = t_nodes[t];
         nodes.assign(owned.begin() + own_cnt[t], owned.begin() + own_cnt[t + 1]);
         for (size_t i = 0; i < nodes.size(); ++i) lid_of[nodes[i]] = int32_t(i);
@@ -249,38 +300,88 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
         plan.tiles[t].n_touch = uint32_t(nodes.size());
         plan.tiles[t].n_elem = uint32_t(recs.size());
       }
-    });
-  }
-  for (auto& x : th) x.join();
+  });
   for (int e : err)
     if (e) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
-  // concatenate
-  size_t R = 0, NT = 0;
-  for (uint32_t t = 0; t < ntiles; ++t) {
-    plan.tiles[t].elem_off = uint32_t(R);
-    plan.tiles[t].node_off = uint32_t(NT);
-    R += t_rec[t].size();
-    NT += t_nodes[t].size();
-    plan.max_touch = std::max(plan.max_touch, plan.tiles[t].n_touch);
-    plan.max_own = std::max(plan.max_own, plan.tiles[t].n_own);
-    plan.max_elem = std::max(plan.max_elem, plan.tiles[t].n_elem);
-    plan.max_slots = std::max(plan.max_slots, plan.tiles[t].n_own + plan.tiles[t].n_touch);
+  concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
+}
+
+void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                      const uint8_t* lev, uint32_t T, TilePlan& plan) {
+  plan = TilePlan();
+  plan.tile_elems = T;
+  const uint32_t ntiles = (E + T - 1) / T;
+  plan.tiles.resize(ntiles);
+  const std::vector<uint8_t> tp = element_types(E, child, hn);
+  // elements touching each node (CSR, ascending): the first one's tile owns the node
+  std::vector<uint32_t> ptr(size_t(N) + 1, 0), adj(size_t(E) * 8);
+  for (size_t i = 0; i < size_t(E) * 8; ++i) ptr[nl[i] + 1]++;
+  for (uint32_t n = 0; n < N; ++n) ptr[n + 1] += ptr[n];
+  {
+    std::vector<uint32_t> fill(ptr.begin(), ptr.end() - 1);
+    for (uint32_t e = 0; e < E; ++e)
+      for (int k = 0; k < 8; ++k) adj[fill[nl[size_t(e) * 8 + k]]++] = e;
   }
-  if (R > 0xffffffffu || NT > 0xffffffffu) fail(DGH_ERR_ARG, "mesh too large for 32-bit tile offsets");
-  plan.rec_elem.resize(R);
-  plan.meta.resize(R);
-  plan.lid.resize(R * 8);
-  plan.node_tab.resize(NT);
-  for (uint32_t t = 0; t < ntiles; ++t) {
-    const size_t ro = plan.tiles[t].elem_off, no = plan.tiles[t].node_off;
-    std::copy(t_rec[t].begin(), t_rec[t].end(), plan.rec_elem.begin() + ro);
-    std::copy(t_lid[t].begin(), t_lid[t].end(), plan.lid.begin() + ro * 8);
-    std::copy(t_nodes[t].begin(), t_nodes[t].end(), plan.node_tab.begin() + no);
-    for (size_t r = 0; r < t_rec[t].size(); ++r) {
-      const uint32_t e = t_rec[t][r];
-      plan.meta[ro + r] = uint16_t(tp[e] | (uint16_t(lev[e]) << 5));
+  std::vector<std::vector<uint32_t>> t_rec(ntiles), t_nodes(ntiles);
+  std::vector<std::vector<uint16_t>> t_lid(ntiles);
+  std::vector<int> err(16, 0);
+  for_tiles(ntiles, [&](unsigned w, unsigned nt, uint32_t) {
+    std::vector<int32_t> lid_of(N, -1);
+    std::vector<uint32_t> emark(E, 0), cls_end(1024), sorted;
+    for (uint32_t t = w; t < ntiles; t += nt) {
+      const uint32_t e0 = t * T, e1 = std::min(E, e0 + T);
+      auto& recs = t_rec[t];
+      auto& nodes = t_nodes[t];
+      auto add_elem = [&](uint32_t e) {
+        if (emark[e] == t + 1) return;
+        emark[e] = t + 1;
+        recs.push_back(e);
+      };
+      // lists the nodes of recs[from, ...) not listed yet, ascending; owned: only those of tile t
+      auto add_nodes = [&](size_t from, bool owned) {
+        const size_t n0 = nodes.size();
+        for (size_t r = from; r < recs.size(); ++r)
+          for (int k = 0; k < 8; ++k) {
+            const uint32_t n = nl[size_t(recs[r]) * 8 + k];
+            if (lid_of[n] != -1 || (owned && adj[ptr[n]] / T != t)) continue;
+            lid_of[n] = -2;
+            nodes.push_back(n);
+          }
+        std::sort(nodes.begin() + n0, nodes.end());
+        for (size_t i = n0; i < nodes.size(); ++i) lid_of[nodes[i]] = int32_t(i);
+      };
+      auto add_elems_of = [&](size_t from) {
+        for (size_t i = from; i < nodes.size(); ++i)
+          for (uint32_t p = ptr[nodes[i]]; p < ptr[nodes[i] + 1]; ++p) add_elem(adj[p]);
+      };
+      for (uint32_t e = e0; e < e1; ++e) add_elem(e);
+      add_nodes(0, true);
+      const size_t n_out = nodes.size();
+      add_elems_of(0);
+      const size_t r2 = recs.size();
+      add_nodes(0, false);
+      const size_t n1 = nodes.size();
+      add_elems_of(n_out);
+      add_nodes(r2, false);
+      order_records(recs.data(), r2, tp.data(), lev, cls_end, sorted);
+      order_records(recs.data() + r2, recs.size() - r2, tp.data(), lev, cls_end, sorted);
+      if (nodes.size() > 65535) err[w] = 1;
+      auto& lids = t_lid[t];
+      lids.resize(recs.size() * 8);
+      for (size_t r = 0; r < recs.size(); ++r)
+        for (int k = 0; k < 8; ++k) lids[r * 8 + k] = uint16_t(lid_of[nl[size_t(recs[r]) * 8 + (k ^ child[recs[r]])]]);
+      for (uint32_t n : nodes) lid_of[n] = -1;
+      TileRec& tr = plan.tiles[t];
+      tr.n_own = uint32_t(n1);
+      tr.n_touch = uint32_t(nodes.size());
+      tr.n_elem = uint32_t(recs.size());
+      tr.n_own2 = uint32_t(n_out);
+      tr.n_elem2 = uint32_t(r2);
     }
-  }
+  });
+  for (int e : err)
+    if (e) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
+  concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
 }  // namespace dgh
