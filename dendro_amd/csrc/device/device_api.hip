@@ -188,6 +188,24 @@ static void launch_pair(dgh_mesh m, const T* x, const PairIO<T>& io, hipStream_t
   HIP_CHECK(hipGetLastError());
 }
 
+// f(slots per thread) for a gather of pitch columns by a workgroup of that many threads.
+template <class F>
+static void gather_slots(uint32_t pitch, uint32_t threads, F f) {
+  const uint32_t ns = (pitch + threads - 1) / threads;
+  if (ns <= 1)
+    f(std::integral_constant<int, 1>());
+  else if (ns <= 2)
+    f(std::integral_constant<int, 2>());
+  else if (ns <= 3)
+    f(std::integral_constant<int, 3>());
+  else if (ns <= 4)
+    f(std::integral_constant<int, 4>());
+  else if (ns <= 6)
+    f(std::integral_constant<int, 6>());
+  else
+    f(std::integral_constant<int, 8>());
+}
+
 // c = R f; with x1 given, also x1 = omega (c * invd) (the first sweep on the coarse level)
 // Boundary flags of a transfer's two meshes when both carry them (Dirichlet problem): the
 // transfers then drop every entry that touches a boundary node (the suppressed DOFs of
@@ -205,12 +223,23 @@ static void launch_restrict(dgh_transfer t, const T* f, T* c, hipStream_t st, T 
   const uint32_t nc = t->coarse->N;
   if (!nc) return;
   const uint8_t *bc = tbdy_c(t), *bf = tbdy_f(t);
-  if (t->ent.p)
-    hipLaunchKernelGGL((restrict_kernel<T, true>), dim3(blocks_for(size_t(nc) * RLANES)), dim3(VBLOCK), 0, st, nc,
-                       t->rowptr.p, t->ent.p, (const float*)nullptr, f, c, omega, invd, x1, bc, bf);
-  else
-    hipLaunchKernelGGL((restrict_kernel<T, false>), dim3(blocks_for(size_t(nc) * RLANES)), dim3(VBLOCK), 0, st, nc,
+  if (t->rpitch) {
+    auto launch = [&](auto lanes) {
+      const uint32_t rows = RT_BLOCK / lanes.value;
+      gather_slots(t->rpitch, RT_BLOCK, [&](auto ns) {
+        hipLaunchKernelGGL((restrict_tile_kernel<T, ns.value, lanes.value>), dim3((nc + rows - 1) / rows), dim3(RT_BLOCK),
+                           (t->rpitch + 1) * sizeof(T), st, nc, t->rpitch, t->rlist.p, t->rowptr.p, t->rent.p, f, c,
+                           omega, invd, x1, bc, bf);
+      });
+    };
+    if (nc < RT_LARGE)
+      launch(std::integral_constant<int, RT_LANES_SMALL>());
+    else
+      launch(std::integral_constant<int, RT_LANES_LARGE>());
+  } else {
+    hipLaunchKernelGGL(restrict_kernel<T>, dim3(blocks_for(size_t(nc) * RLANES)), dim3(VBLOCK), 0, st, nc,
                        t->rowptr.p, t->col.p, t->w.p, f, c, omega, invd, x1, bc, bf);
+  }
   HIP_CHECK(hipGetLastError());
 }
 
@@ -218,8 +247,16 @@ template <class T>
 static void launch_prolong(dgh_transfer t, const T* c, const T* f_in, T* f_out, hipStream_t st) {
   const uint32_t nf = t->fine->N;
   if (!nf) return;
-  hipLaunchKernelGGL(prolong_kernel<T>, dim3(blocks_for(nf)), dim3(VBLOCK), 0, st, nf, t->celem.p,
-                     t->pos.p, t->coarse->nl.p, t->coarse->cs.p, Wtab<T>(), c, f_in, f_out, tbdy_c(t), tbdy_f(t));
+  if (t->ppitch) {
+    const dim3 grid((nf + PT_ROWS - 1) / PT_ROWS), block(PT_ROWS);
+    gather_slots(t->ppitch, block.x, [&](auto ns) {
+      hipLaunchKernelGGL((prolong_tile_kernel<T, ns.value>), grid, block, (t->ppitch + 1) * sizeof(T), st, nf, t->ppitch,
+                         t->plist.p, reinterpret_cast<const uint4*>(t->pent.p), c, f_in, f_out, tbdy_c(t), tbdy_f(t));
+    });
+  } else {
+    hipLaunchKernelGGL(prolong_kernel<T>, dim3(blocks_for(nf)), dim3(VBLOCK), 0, st, nf, t->celem.p,
+                       t->pos.p, t->coarse->nl.p, t->coarse->cs.p, Wtab<T>(), c, f_in, f_out, tbdy_c(t), tbdy_f(t));
+  }
   HIP_CHECK(hipGetLastError());
 }
 
@@ -449,6 +486,41 @@ static void default_tiling(uint32_t E, uint32_t& T, int& block) {
   } else {
     T = std::max(std::min(192u, std::max(64u, E / 256u)), E / 512u);
   }
+}
+
+// The LDS forms of both transfers, where their blocks and weights fit (GATHER_MAX columns; every mesh
+// tried has at most a quarter).  W: transfer weights; rowptr, col, w: R = P^T.
+static void plan_transfer(dgh_transfer t, const double* W, const std::vector<uint32_t>& rowptr,
+                          const std::vector<uint32_t>& col, const std::vector<float>& w) {
+  static_assert(GATHER_MAX + 1 <= 8 * PT_ROWS && GATHER_MAX + 1 <= 8 * RT_BLOCK, "at most 8 slots per thread");
+  const uint32_t nf = t->fine->N, nc = t->coarse->N;
+  GatherPlan r;
+  const uint32_t rows = RT_BLOCK / (nc < RT_LARGE ? RT_LANES_SMALL : RT_LANES_LARGE);
+  if (build_gather(nc, rowptr.data(), col.data(), w.data(), rows, r)) {
+    t->rpitch = r.pitch;
+    t->rlist.upload(r.list.data(), r.list.size());
+    t->rent.upload(r.ent.data(), r.ent.size());
+  }
+  std::vector<uint32_t> prow(size_t(nf) + 1, 0), pcol(col.size());   // P, entries in vertex order
+  std::vector<float> pw(col.size());
+  uint32_t q = 0;
+  for (uint32_t j = 0; j < nf; ++j) {
+    const uint32_t ce = t->h_celem[j];
+    const double* wj = W + (size_t(t->coarse->h_cs[ce]) * 27 + t->h_pos[j]) * 8;
+    for (int k = 0; k < 8; ++k)
+      if (wj[k] != 0.0) {
+        pcol[q] = t->coarse->h_nl[size_t(ce) * 8 + k];
+        pw[q++] = float(wj[k]);
+      }
+    prow[j + 1] = q;
+  }
+  GatherPlan p;
+  if (!build_gather(nf, prow.data(), pcol.data(), pw.data(), PT_ROWS, p)) return;
+  std::vector<uint16_t> e8(size_t(nf) * 8, uint16_t(p.pitch));   // unused entries: the zero slot
+  for (uint32_t j = 0; j < nf; ++j) std::copy(p.ent.begin() + prow[j], p.ent.begin() + prow[j + 1], e8.begin() + size_t(j) * 8);
+  t->ppitch = p.pitch;
+  t->plist.upload(p.list.data(), p.list.size());
+  t->pent.upload(e8.data(), e8.size());
 }
 
 // (Re)builds the single right-hand-side tiling with tiles of at most T elements within the
@@ -1384,16 +1456,7 @@ int dgh_transfer_create(dgh_mesh coarse, dgh_mesh fine, const uint32_t* coarse_e
     t->rowptr.upload(rowptr.data(), rowptr.size());
     t->col.upload(col.data(), col.size());
     t->w.upload(wv.data(), wv.size());
-    // packed entries (half the index traffic of the restriction) when every weight is a
-    // multiple of 1/32 in (0, 1] and the fine nodes fit in 27 bits
-    bool packable = nf <= RP_COL + 1u;
-    std::vector<uint32_t> ent(col.size());
-    for (size_t q = 0; q < col.size() && packable; ++q) {
-      const double k = double(wv[q]) * 32.0;
-      packable = (k == std::floor(k) && k >= 1.0 && k <= 32.0);
-      ent[q] = (uint32_t(k - 1.0) << RP_SHIFT) | col[q];
-    }
-    if (packable) t->ent.upload(ent.data(), ent.size());
+    plan_transfer(t.get(), W.data(), rowptr, col, wv);
     *out = t.release();
   });
 }

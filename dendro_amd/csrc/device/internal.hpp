@@ -203,7 +203,10 @@ struct dgh_transfer_s {
   DevBuf<uint8_t> pos;          // [N_f] position code inside it
   DevBuf<uint32_t> rowptr, col; // R = P^T in CSR (rows: coarse nodes)
   DevBuf<float> w;              // exact dyadic weights
-  DevBuf<uint32_t> ent;         // packed (32 w - 1) << 27 | col, when every entry fits
+  // both directions through LDS (build_gather); pitch 0: not planned, the general kernels run
+  uint32_t ppitch = 0, rpitch = 0;
+  DevBuf<uint32_t> plist, rlist;
+  DevBuf<uint16_t> pent, rent;  // prolongation: [N_f][8] entries; restriction: one per entry of R
   std::vector<uint32_t> h_celem; // host copies of celem and pos (Jacobian3 coarsest assembly)
   std::vector<uint8_t> h_pos;
   DevBuf<double> j3v64, j3w64;  // fine-level scratch of dgh_matvec_jac3

@@ -896,11 +896,7 @@ prolong_kernel(uint32_t nf, const uint32_t* __restrict__ celem, const uint8_t* _
 constexpr int RLANES = 4;
 // With x1 given, also the coarse level's first smoothing sweep from a zero guess:
 // x1 = omega (c * invd), as smooth_first_kernel forms it.
-// PACKED: one 32-bit word per entry, (32 w - 1) << 27 | fine node (every weight is a
-// multiple of 1/32 in (0, 1]); otherwise col and w arrays.
-constexpr int RP_SHIFT = 27;
-constexpr uint32_t RP_COL = (1u << RP_SHIFT) - 1u;
-template <class T, bool PACKED = false>
+template <class T>
 __global__ void __launch_bounds__(256)
 restrict_kernel(uint32_t nc, const uint32_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
                 const float* __restrict__ w, const T* __restrict__ f, T* __restrict__ c, T omega = T(0),
@@ -921,22 +917,19 @@ restrict_kernel(uint32_t nc, const uint32_t* __restrict__ rowptr, const uint32_t
       for (int u = 0; u < RU; ++u) {
         const uint32_t p = p0 + u * RLANES;
         e[u] = p < p1 ? col[p] : 0u;
-        wv[u] = (!PACKED && p < p1) ? T(w[p]) : T(0);
+        wv[u] = p < p1 ? T(w[p]) : T(0);
       }
 #pragma unroll
-      for (int u = 0; u < RU; ++u) fv[u] = p0 + u * RLANES < p1 ? f[PACKED ? (e[u] & RP_COL) : e[u]] : T(0);
+      for (int u = 0; u < RU; ++u) fv[u] = p0 + u * RLANES < p1 ? f[e[u]] : T(0);
       if (fbdy) {   // Dirichlet: no entry from a boundary fine node
 #pragma unroll
         for (int u = 0; u < RU; ++u)
-          if (p0 + u * RLANES < p1 && fbdy[PACKED ? (e[u] & RP_COL) : e[u]]) fv[u] = T(0);
+          if (p0 + u * RLANES < p1 && fbdy[e[u]]) fv[u] = T(0);
       }
 #pragma unroll
       for (int u = 0; u < RU; ++u) {
         if (p0 + u * RLANES >= p1) break;
-        if (PACKED)
-          acc += T(float((e[u] >> RP_SHIFT) + 1u) * 0.03125f) * fv[u];
-        else
-          acc += wv[u] * fv[u];
+        acc += wv[u] * fv[u];
       }
     }
   }
@@ -946,6 +939,117 @@ restrict_kernel(uint32_t nc, const uint32_t* __restrict__ rowptr, const uint32_t
     if (cbdy && cbdy[i]) acc = T(0);   // Dirichlet: no entry into a boundary coarse node
     c[i] = acc;
     if (x1) x1[i] = T(0) + omega * (acc * invd[i]);
+  }
+}
+
+// ---------------------------------------------------------------- transfers through LDS
+// Both transfers as sparse products whose workgroups gather the distinct columns of their rows once
+// into LDS (build_gather).  The forms above chase three dependent loads (a row's place, its columns,
+// their values) and issue up to 12 scattered loads per fine node, 40% of them for zero weights; here
+// the column lists and the rows' entries (2 bytes each) arrive together, then the values, and the
+// products read LDS.  NS: column slots per thread.  The zero slot past the list takes unused
+// entries, so whole rows are read without a count.
+constexpr uint32_t GE_ID = (1u << GATHER_BITS) - 1u;
+template <class T>
+__device__ __forceinline__ T gather_weight(uint32_t e) {
+  return T(float((e >> GATHER_BITS) + 1u) * 0.03125f);
+}
+// stages the values of the block's columns (0 where zero flags one), and the zero slot
+template <class T, int NS>
+__device__ __forceinline__ void gather_stage(T* xs, uint32_t pitch, const uint32_t* __restrict__ list,
+                                             const T* __restrict__ x, const uint8_t* __restrict__ zero) {
+  uint32_t id[NS];
+  T v[NS];
+#pragma unroll
+  for (int q = 0; q < NS; ++q) id[q] = list[min(threadIdx.x + uint32_t(q) * blockDim.x, pitch - 1u)];
+#pragma unroll
+  for (int q = 0; q < NS; ++q) v[q] = x[id[q]];
+  if (zero) {
+#pragma unroll
+    for (int q = 0; q < NS; ++q) v[q] = zero[id[q]] ? T(0) : v[q];
+  }
+#pragma unroll
+  for (int q = 0; q < NS; ++q) {
+    const uint32_t i = threadIdx.x + uint32_t(q) * blockDim.x;
+    if (i < pitch) xs[i] = v[q];
+  }
+  if (threadIdx.x == 0) xs[pitch] = T(0);
+}
+
+// f_out = f_in + P c: a thread per fine node, its up to 8 entries in 16 bytes.
+constexpr int PT_ROWS = 256;
+template <class T, int NS>
+__global__ void __launch_bounds__(PT_ROWS)
+prolong_tile_kernel(uint32_t nf, uint32_t pitch, const uint32_t* __restrict__ list, const uint4* __restrict__ ent,
+                    const T* __restrict__ c, const T* __restrict__ f_in, T* __restrict__ f_out,
+                    const uint8_t* __restrict__ cbdy, const uint8_t* __restrict__ fbdy) {
+  extern __shared__ __align__(16) unsigned char gather_lds[];
+  T* xs = reinterpret_cast<T*>(gather_lds);
+  const uint32_t j = blockIdx.x * PT_ROWS + threadIdx.x, jc = min(j, nf - 1u);
+  const uint4 e4 = ent[jc];
+  const T f = f_in ? f_in[jc] : T(0);
+  gather_stage<T, NS>(xs, pitch, list + size_t(blockIdx.x) * pitch, c, cbdy);
+  const bool out0 = fbdy && fbdy[jc];   // Dirichlet: no entry into a boundary fine node
+  __syncthreads();
+  if (j >= nf) return;
+  const uint32_t e[4] = {e4.x, e4.y, e4.z, e4.w};
+  T acc = T(0);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t ek = (e[k >> 1] >> (16 * (k & 1))) & 0xffffu;
+    acc += gather_weight<T>(ek) * xs[ek & GE_ID];
+  }
+  f_out[j] = f + (out0 ? T(0) : acc);
+}
+
+// c = P^T f and x1 (see restrict_kernel): RT_LANES lanes per coarse node, 8 where the launch does not
+// fill the device, 2 from RT_LARGE coarse nodes on, where fewer workgroups and shuffles count.  Both
+// transfers in turn, FP32 / FP64 us, 461k fine and 135k coarse nodes: 2 lanes 8.5 / 10.4, 4 lanes 9.1 /
+// 12.1, 8 lanes 10.5 / 13.3, the general kernels 11.3 / 14.6; 5.5M and 2.1M: 70 / 89, 104 / 124, 127 /
+// 152 and 95 / 137.  FP64 V-cycle of 11k elements: 81.9 us with 8 lanes, 86.9 with the general kernels.
+constexpr int RT_BLOCK = 256, RT_LANES_SMALL = 8, RT_LANES_LARGE = 2;
+constexpr uint32_t RT_LARGE = 80000;
+template <class T, int NS, int RT_LANES>
+__global__ void __launch_bounds__(RT_BLOCK)
+restrict_tile_kernel(uint32_t nc, uint32_t pitch, const uint32_t* __restrict__ list,
+                     const uint32_t* __restrict__ rowptr, const uint16_t* __restrict__ ent, const T* __restrict__ f,
+                     T* __restrict__ c, T omega, const T* __restrict__ invd, T* __restrict__ x1,
+                     const uint8_t* __restrict__ cbdy, const uint8_t* __restrict__ fbdy) {
+  extern __shared__ __align__(16) unsigned char gather_lds[];
+  T* xs = reinterpret_cast<T*>(gather_lds);
+  constexpr uint32_t RT_ROWS = RT_BLOCK / RT_LANES;
+  const uint32_t i = blockIdx.x * RT_ROWS + threadIdx.x / RT_LANES, lane = threadIdx.x % RT_LANES;
+  const uint32_t ic = min(i, nc - 1u);
+  const uint32_t p0 = rowptr[ic] + lane, p1 = rowptr[ic + 1];
+  const T dv = x1 ? invd[ic] : T(0);
+  gather_stage<T, NS>(xs, pitch, list + size_t(blockIdx.x) * pitch, f, fbdy);
+  constexpr int RU = 32 / RT_LANES;   // a row of up to 32 entries in one step
+  uint32_t e[RU];
+#pragma unroll
+  for (int u = 0; u < RU; ++u) e[u] = p0 + u * RT_LANES < p1 ? uint32_t(ent[p0 + u * RT_LANES]) : pitch;
+  __syncthreads();
+  constexpr int NA = RT_LANES < RLANES ? RLANES / RT_LANES : 1;   // partial sums per lane, in restrict_kernel's order
+  T part[NA];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) part[a] = T(0);
+#pragma unroll
+  for (int u = 0; u < RU; ++u) part[u % NA] += gather_weight<T>(e[u]) * xs[e[u] & GE_ID];
+  for (uint32_t p = p0 + RU * RT_LANES; p < p1; p += NA * RT_LANES)
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+      if (p + a * RT_LANES < p1) {
+        const uint32_t ep = ent[p + a * RT_LANES];
+        part[a] += gather_weight<T>(ep) * xs[ep & GE_ID];
+      }
+  T acc = part[0];
+#pragma unroll
+  for (int a = 1; a < NA; ++a) acc += part[a];
+#pragma unroll
+  for (int off = RT_LANES / 2; off > 0; off >>= 1) acc += __shfl_down(acc, off, RT_LANES);
+  if (i < nc && lane == 0) {
+    if (cbdy && cbdy[i]) acc = T(0);
+    c[i] = acc;
+    if (x1) x1[i] = T(0) + omega * (acc * dv);
   }
 }
 

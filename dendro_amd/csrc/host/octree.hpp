@@ -80,6 +80,19 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
 // reads the nodes of those (n_touch).
 void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                       const uint8_t* lev, uint32_t T, TilePlan& plan);
+// Blocks of B consecutive rows of a sparse matrix (CSR, weights multiples of 1/32 in (0, 1]) for
+// kernels that gather each block's distinct columns once: list holds block b's columns, ascending,
+// at [b * pitch, ...), padded with its last one, and ent, per CSR entry, (32 w - 1) << 11 | index in
+// its block's list.  False if a block has more than GATHER_MAX columns or a weight does not fit.
+constexpr uint32_t GATHER_BITS = 11;
+constexpr uint32_t GATHER_MAX = (1u << GATHER_BITS) - 1u;   // one index stays free for a zero slot
+struct GatherPlan {
+  uint32_t pitch = 0;
+  std::vector<uint32_t> list;
+  std::vector<uint16_t> ent;
+};
+bool build_gather(uint32_t nrows, const uint32_t* rowptr, const uint32_t* col, const float* w, uint32_t B,
+                  GatherPlan& plan);
 // Tile boundaries alone: bounds[t] = first element of tile t, bounds.back() = E.
 void tile_bounds(uint32_t E, uint32_t N, const uint32_t* nl, uint32_t T, uint32_t budget,
                  std::vector<uint32_t>& bounds, uint32_t own_cap = 0);

@@ -384,4 +384,56 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
+bool build_gather(uint32_t nrows, const uint32_t* rowptr, const uint32_t* col, const float* w, uint32_t B,
+                  GatherPlan& plan) {
+  const uint32_t nb = (nrows + B - 1) / B;
+  std::vector<std::vector<uint32_t>> cols(nb);
+  plan.ent.resize(rowptr[nrows]);
+  std::vector<int> bad(16, 0);
+  for_tiles(nb, [&](unsigned wk, unsigned nt, uint32_t) {
+    // the block's columns in an open-addressed table of twice the most it may hold
+    constexpr uint32_t HS = 2u << GATHER_BITS;
+    std::vector<uint32_t> key(HS), owner(HS, 0xffffffffu), slot(HS);
+    uint32_t b = wk;
+    auto find = [&](uint32_t c) {
+      uint32_t h = (c * 2654435761u) >> (31 - GATHER_BITS);
+      while (owner[h] == b && key[h] != c) h = (h + 1) & (HS - 1);
+      return h;
+    };
+    for (; b < nb && !bad[wk]; b += nt) {
+      const uint32_t q0 = rowptr[b * B], q1 = rowptr[std::min(nrows, (b + 1) * B)];
+      auto& l = cols[b];
+      for (uint32_t q = q0; q < q1 && l.size() <= GATHER_MAX; ++q) {
+        const uint32_t h = find(col[q]);
+        if (owner[h] == b) continue;
+        owner[h] = b;
+        key[h] = col[q];
+        l.push_back(col[q]);
+      }
+      if (l.size() > GATHER_MAX) {
+        bad[wk] = 1;
+        break;
+      }
+      std::sort(l.begin(), l.end());
+      for (size_t i = 0; i < l.size(); ++i) slot[find(l[i])] = uint32_t(i);
+      for (uint32_t q = q0; q < q1; ++q) {
+        const double k = double(w[q]) * 32.0;
+        if (!(k >= 1.0 && k <= 32.0 && k == double(int(k)))) bad[wk] = 1;
+        plan.ent[q] = uint16_t((uint32_t(k - 1.0) << GATHER_BITS) | slot[find(col[q])]);
+      }
+    }
+  });
+  for (int e : bad)
+    if (e) return false;
+  plan.pitch = 1;
+  for (const auto& l : cols) plan.pitch = std::max(plan.pitch, uint32_t(l.size()));
+  plan.list.assign(size_t(nb) * plan.pitch, 0u);
+  for (uint32_t b = 0; b < nb; ++b) {
+    uint32_t* dst = plan.list.data() + size_t(b) * plan.pitch;
+    std::copy(cols[b].begin(), cols[b].end(), dst);
+    if (!cols[b].empty()) std::fill(dst + cols[b].size(), dst + plan.pitch, cols[b].back());
+  }
+  return true;
+}
+
 }  // namespace dgh
