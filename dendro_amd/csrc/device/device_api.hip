@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <thread>
 #include <vector>
 
 #include "internal.hpp"
@@ -224,18 +225,18 @@ static void launch_restrict(dgh_transfer t, const T* f, T* c, hipStream_t st, T 
   if (!nc) return;
   const uint8_t *bc = tbdy_c(t), *bf = tbdy_f(t);
   if (t->rpitch) {
-    auto launch = [&](auto lanes) {
-      const uint32_t rows = RT_BLOCK / lanes.value;
-      gather_slots(t->rpitch, RT_BLOCK, [&](auto ns) {
-        hipLaunchKernelGGL((restrict_tile_kernel<T, ns.value, lanes.value>), dim3((nc + rows - 1) / rows), dim3(RT_BLOCK),
-                           (t->rpitch + 1) * sizeof(T), st, nc, t->rpitch, t->rlist.p, t->rowptr.p, t->rent.p, f, c,
-                           omega, invd, x1, bc, bf);
+    auto launch = [&](auto lanes, auto rows) {
+      const uint32_t threads = lanes.value * rows.value;
+      gather_slots(t->rpitch, threads, [&](auto ns) {
+        hipLaunchKernelGGL((restrict_tile_kernel<T, ns.value, lanes.value, rows.value>),
+                           dim3((nc + rows.value - 1) / rows.value), dim3(threads), (t->rpitch + 1) * sizeof(T), st, nc,
+                           t->rpitch, t->rlist.p, t->rowptr.p, t->rent.p, f, c, omega, invd, x1, bc, bf);
       });
     };
     if (nc < RT_LARGE)
-      launch(std::integral_constant<int, RT_LANES_SMALL>());
+      launch(std::integral_constant<int, sizeof(T) == 8 ? 8 : 4>(), std::integral_constant<int, RT_ROWS_SMALL>());
     else
-      launch(std::integral_constant<int, RT_LANES_LARGE>());
+      launch(std::integral_constant<int, 2>(), std::integral_constant<int, RT_ROWS_LARGE>());
   } else {
     hipLaunchKernelGGL(restrict_kernel<T>, dim3(blocks_for(size_t(nc) * RLANES)), dim3(VBLOCK), 0, st, nc,
                        t->rowptr.p, t->col.p, t->w.p, f, c, omega, invd, x1, bc, bf);
@@ -431,28 +432,36 @@ static void upload_pitched(DevTiles& d) {
   d.node_tab.upload(tab.data(), tab.size());
 }
 
-// Two-sweep tiles of a mesh that a V-cycle smooths (once per mesh).
-static void build_pair(dgh_mesh m) {
-  if (m->pair_tried) return;
-  m->pair_tried = true;
-  if (m->E > PAIR_MAX_ELEMS) return;
-  DevTiles& d = m->pair;
-  for (uint32_t T = std::max(32u, m->E / 256u);; T /= 2) {   // one tile per CU; E/128 and E/512 within 2%
-    build_pair_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), T, d.plan);
-    if (d.plan.max_touch <= uint32_t(PAIR_XC * PAIR_BLOCK) && d.plan.max_own <= uint32_t(PAIR_OC * PAIR_BLOCK)) break;
-    if (T < 16) {   // too dense a neighbourhood: single sweeps
-      d.plan = TilePlan();
-      return;
-    }
+// Two-sweep tiles of the meshes a V-cycle smooths (once per mesh; the meshes are planned at the same time).
+static void build_pairs(const std::vector<dgh_mesh>& meshes) {
+  std::vector<std::thread> th;
+  for (dgh_mesh m : meshes)
+    th.emplace_back([m] {
+      try {
+        for (uint32_t T = std::max(32u, m->E / 256u);; T /= 2) {   // one tile per CU; E/128 and E/512 within 2%
+          TilePlan& p = m->pair.plan;
+          build_pair_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), T, p);
+          if (p.max_touch <= uint32_t(PAIR_XC * PAIR_BLOCK) && p.max_own <= uint32_t(PAIR_OC * PAIR_BLOCK)) return;
+          if (T < 16) break;   // too dense a neighbourhood
+        }
+      } catch (...) {
+      }
+      m->pair.plan = TilePlan();   // single sweeps
+    });
+  for (auto& t : th) t.join();
+  for (dgh_mesh m : meshes) {
+    m->pair_tried = true;
+    DevTiles& d = m->pair;
+    if (d.plan.tiles.empty()) continue;
+    d.block = PAIR_BLOCK;
+    d.lds64 = uint32_t(tile_lds_bytes<double>(PAIR_BLOCK, d.plan.max_touch));
+    d.lds32 = uint32_t(tile_lds_bytes<float>(PAIR_BLOCK, d.plan.max_touch));
+    d.tiles.upload(d.plan.tiles.data(), d.plan.tiles.size());
+    const std::vector<uint16_t> packed = pack_records(d.plan);
+    d.lid.upload(packed.data(), packed.size());
+    upload_pitched(d);
+    upload_coefs(m, d);
   }
-  d.block = PAIR_BLOCK;
-  d.lds64 = uint32_t(tile_lds_bytes<double>(PAIR_BLOCK, d.plan.max_touch));
-  d.lds32 = uint32_t(tile_lds_bytes<float>(PAIR_BLOCK, d.plan.max_touch));
-  d.tiles.upload(d.plan.tiles.data(), d.plan.tiles.size());
-  const std::vector<uint16_t> packed = pack_records(d.plan);
-  d.lid.upload(packed.data(), packed.size());
-  upload_pitched(d);
-  upload_coefs(m, d);
 }
 
 // Node budget of a single right-hand-side tile for a block size: the LDS share that lets the
@@ -492,10 +501,10 @@ static void default_tiling(uint32_t E, uint32_t& T, int& block) {
 // tried has at most a quarter).  W: transfer weights; rowptr, col, w: R = P^T.
 static void plan_transfer(dgh_transfer t, const double* W, const std::vector<uint32_t>& rowptr,
                           const std::vector<uint32_t>& col, const std::vector<float>& w) {
-  static_assert(GATHER_MAX + 1 <= 8 * PT_ROWS && GATHER_MAX + 1 <= 8 * RT_BLOCK, "at most 8 slots per thread");
+  static_assert(GATHER_MAX + 1 <= 8 * PT_ROWS && GATHER_MAX + 1 <= 8 * 256, "at most 8 slots per thread");
   const uint32_t nf = t->fine->N, nc = t->coarse->N;
   GatherPlan r;
-  const uint32_t rows = RT_BLOCK / (nc < RT_LARGE ? RT_LANES_SMALL : RT_LANES_LARGE);
+  const uint32_t rows = nc < RT_LARGE ? RT_ROWS_SMALL : RT_ROWS_LARGE;
   if (build_gather(nc, rowptr.data(), col.data(), w.data(), rows, r)) {
     t->rpitch = r.pitch;
     t->rlist.upload(r.list.data(), r.list.size());
@@ -819,18 +828,22 @@ static void cg_iteration(dgh_solver s, hipStream_t st) {
   }
 }
 
-// The norm after iteration it (0: the initial one), once the device has written it.
-static double cg_wait(dgh_solver s, int it, hipStream_t st) {
+// Waits until the device has told the norms after iteration it (0: the initial ones).
+void cg_wait_seq(const unsigned long long* seq, int it, hipStream_t st) {
   const unsigned long long want = static_cast<unsigned long long>(it) + 1ull;
-  for (uint32_t spin = 1; __atomic_load_n(&s->sig->seq, __ATOMIC_ACQUIRE) < want; ++spin) {
+  for (uint32_t spin = 1; __atomic_load_n(seq, __ATOMIC_ACQUIRE) < want; ++spin) {
     __builtin_ia32_pause();
     if (spin % 4096u) continue;
     const hipError_t q = hipStreamQuery(st);   // an idle or failed stream writes nothing more
     if (q == hipErrorNotReady) continue;
     HIP_CHECK(q);
-    if (__atomic_load_n(&s->sig->seq, __ATOMIC_ACQUIRE) < want)
+    if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) < want)
       fail(DGH_ERR_STATE, "the solve ended without the norm of iteration %d", it);
   }
+}
+
+static double cg_wait(dgh_solver s, int it, hipStream_t st) {
+  cg_wait_seq(&s->sig->seq, it, st);
   return s->sig->dp[it & 3];
 }
 
@@ -1589,9 +1602,13 @@ int dgh_solver_create(int nlevels, const dgh_mesh* meshes, const dgh_transfer* t
     s->S.alloc(S_NSCAL);
     s->part.alloc(size_t(MAXQ) * RED_BLOCKS);
     s->part_p.alloc(MAXQ * RED_BLOCKS);
-    if (!s->dirichlet)
-      for (int l = 1; l < nlevels; ++l)
-        if (params->coarse_op == DGH_COARSE_JAC2 || l == nlevels - 1) build_pair(meshes[l]);
+    std::vector<dgh_mesh> paired;
+    for (int l = 1; l < nlevels && !s->dirichlet; ++l)
+      if (!meshes[l]->pair_tried && (params->coarse_op == DGH_COARSE_JAC2 || l == nlevels - 1) &&
+          meshes[l]->E <= (params->vcycle_prec == DGH_F32 ? PAIR_MAX_ELEMS : PAIR_MAX_ELEMS64) &&
+          std::find(paired.begin(), paired.end(), meshes[l]) == paired.end())
+        paired.push_back(meshes[l]);
+    build_pairs(paired);
     // per-level vectors and Jacobi diagonals
     s->v64.resize(nlevels);
     if (params->vcycle_prec == DGH_F32) s->v32.resize(nlevels);
@@ -1727,19 +1744,17 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
         cg_iteration(s, st);
       ++queued;
     };
-    // While the last two norms put the next one above the tolerance (with a margin of 4), one more
-    // iteration is queued before its norm is read, so the device does not wait for the host (20 us
-    // per iteration, 10% of 630k elements' mixed solve).  DONE stops one queued in vain.
-    const double margin = 4.0;
+    // DONE stops an iteration that was queued ahead in vain (10% of a mixed solve of 630k elements was the
+    // device waiting)
     if (s->prm.max_it > 0) queue();
     const double dp0 = cg_wait(s, 0, st);
-    double dp = dp0, rate = 0.05;   // a V-cycle's usual reduction, until two norms are known
+    double dp = dp0, rate = CG_USUAL_RATE;
     if (history && history_len > 0) history[0] = dp0;
     int it = 0;
     bool conv = (dp0 == 0.0), bad = false;
     while (!conv && it < s->prm.max_it) {
       if (queued == it) queue();
-      if (queued == it + 1 && queued < s->prm.max_it && dp * rate > margin * s->prm.rtol * dp0) queue();
+      if (queued == it + 1 && queued < s->prm.max_it && dp * rate > CG_AHEAD_MARGIN * s->prm.rtol * dp0) queue();
       const double prev = dp;
       dp = cg_wait(s, it + 1, st);
       rate = dp / prev;

@@ -71,7 +71,7 @@ constexpr size_t CLASS_ROWS_MIN_TILES = 1024;
 // 1024-thread tiles, from LARGE_MESH_ELEMS up of at most 8192 elements.
 constexpr uint32_t MID_MESH_ELEMS = 1200000;
 constexpr uint32_t LARGE_MESH_ELEMS = 4000000;
-// Largest mesh smoothed two sweeps per launch (build_pair).  The first sweep of a tile takes 7 times
+// Largest mesh smoothed two sweeps per launch (build_pairs).  The first sweep of a tile takes 7 times
 // its elements' records (a single sweep 1.5 to 2), which a launch of a small mesh has room for: V-cycle
 // with the levels up to 60k elements paired / single, FP64: finest 11k elements 86.1 / 96.7 us, 64k 107.2 /
 // 110.5, 297k 147.8 / 148.4, where its level of 37k gains nothing; pairing levels of 64k and 100k
@@ -181,7 +181,7 @@ struct dgh_mesh_s {
   DevTiles op;
   int block = 512;              // threads per operator workgroup (256, 512 or 1024)
   DevTiles mop;
-  DevTiles pair;                // two sweeps per launch (build_pair; no tiles: the mesh takes single ones)
+  DevTiles pair;                // two sweeps per launch (build_pairs; no tiles: the mesh takes single ones)
   bool pair_tried = false;
   uint32_t mtile = 0;           // batched tile size (0: default)
   int mvariant = 6;             // batched FP32 products (multi_api.hip): 1 matrix cores, others vector ALUs
@@ -252,6 +252,16 @@ struct LearnState {
 
 }  // namespace dgh
 
+namespace dgh {
+struct CgSignalMulti;
+// Queued ahead: while the last norms put the next one above the tolerance by this factor, a solve
+// queues one more iteration before it reads the norm of the last, so the device does not wait for the
+// host (20 us per iteration).
+constexpr double CG_AHEAD_MARGIN = 4.0;
+constexpr double CG_USUAL_RATE = 0.05;   // a V-cycle's reduction, until two norms are known
+void cg_wait_seq(const unsigned long long* seq, int it, hipStream_t st);
+}  // namespace dgh
+
 struct dgh_solver_s {
   int nlevels = 0;
   std::vector<dgh_mesh> meshes;
@@ -292,8 +302,8 @@ struct dgh_solver_s {
   DevBuf<double> mS;                   // per-column CG scalars
   DevBuf<double> mpart, mpart_p;       // column reduction partials
   DevBuf<double> mptile;               // CG mode of the FP64 batched product: [tiles][k] partials of p.w
-  DevBuf<double> mdense;               // split partial sums of the batched coarse solve
   double* hmS = nullptr;
+  CgSignalMulti* msig = nullptr;       // the columns' norms, written by the device (pinned host memory)
   hipGraph_t mgraph = nullptr;
   hipGraphExec_t mgexec = nullptr;
   std::vector<double> om_level;        // Richardson scale per level (1 where learned weights sit in invd)
@@ -306,6 +316,7 @@ struct dgh_solver_s {
     if (mgexec) (void)hipGraphExecDestroy(mgexec);
     if (mgraph) (void)hipGraphDestroy(mgraph);
     if (hmS) (void)hipHostFree(hmS);
+    if (msig) (void)hipHostFree(msig);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (hS) (void)hipHostFree(hS);

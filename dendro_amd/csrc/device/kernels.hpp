@@ -1002,22 +1002,23 @@ prolong_tile_kernel(uint32_t nf, uint32_t pitch, const uint32_t* __restrict__ li
   f_out[j] = f + (out0 ? T(0) : acc);
 }
 
-// c = P^T f and x1 (see restrict_kernel): RT_LANES lanes per coarse node, 8 where the launch does not
-// fill the device, 2 from RT_LARGE coarse nodes on, where fewer workgroups and shuffles count.  Both
-// transfers in turn, FP32 / FP64 us, 461k fine and 135k coarse nodes: 2 lanes 8.5 / 10.4, 4 lanes 9.1 /
-// 12.1, 8 lanes 10.5 / 13.3, the general kernels 11.3 / 14.6; 5.5M and 2.1M: 70 / 89, 104 / 124, 127 /
-// 152 and 95 / 137.  FP64 V-cycle of 11k elements: 81.9 us with 8 lanes, 86.9 with the general kernels.
-constexpr int RT_BLOCK = 256, RT_LANES_SMALL = 8, RT_LANES_LARGE = 2;
+// c = P^T f and x1 (see restrict_kernel): RT_LANES lanes for each of RT_ROWS coarse nodes.  Where the
+// launch does not fill the device 64 rows, FP64 with 8 lanes (FP64 V-cycle 149.6 -> 147.7 us, of 11k
+// elements 84.2 -> 81.9), FP32 with the 4 of restrict_kernel, whose sums it keeps; from RT_LARGE coarse
+// nodes on 128 rows with 2 lanes and two partial sums each, the same sums: there fewer workgroups and
+// shuffles count.  Both transfers in turn, FP32 / FP64 us, 461k fine and 135k coarse nodes: 2 lanes 8.5
+// / 10.4, 4 lanes 9.1 / 12.1, 8 lanes 10.5 / 13.3, the general kernels 11.3 / 14.6; 5.5M and 2.1M: 70 /
+// 89, 104 / 124, 127 / 152 and 95 / 137.
+constexpr uint32_t RT_ROWS_SMALL = 64, RT_ROWS_LARGE = 128;
 constexpr uint32_t RT_LARGE = 80000;
-template <class T, int NS, int RT_LANES>
-__global__ void __launch_bounds__(RT_BLOCK)
+template <class T, int NS, int RT_LANES, int RT_ROWS>
+__global__ void __launch_bounds__(RT_LANES * RT_ROWS)
 restrict_tile_kernel(uint32_t nc, uint32_t pitch, const uint32_t* __restrict__ list,
                      const uint32_t* __restrict__ rowptr, const uint16_t* __restrict__ ent, const T* __restrict__ f,
                      T* __restrict__ c, T omega, const T* __restrict__ invd, T* __restrict__ x1,
                      const uint8_t* __restrict__ cbdy, const uint8_t* __restrict__ fbdy) {
   extern __shared__ __align__(16) unsigned char gather_lds[];
   T* xs = reinterpret_cast<T*>(gather_lds);
-  constexpr uint32_t RT_ROWS = RT_BLOCK / RT_LANES;
   const uint32_t i = blockIdx.x * RT_ROWS + threadIdx.x / RT_LANES, lane = threadIdx.x % RT_LANES;
   const uint32_t ic = min(i, nc - 1u);
   const uint32_t p0 = rowptr[ic] + lane, p1 = rowptr[ic + 1];

@@ -482,152 +482,163 @@ __global__ void smooth_first_multi_kernel(uint32_t n, int k, T omega, const T* _
   x[i] = T(0) + omega * (b[i] * invd[i / k]);
 }
 
-// c[i][j] = sum_p w_p f[col_p][j]: lanes run over the right-hand sides of a row.
+// c[i][j] = sum_p w_p f[col_p][j], and with x1 given the coarse level's first sweep from zero, x1 =
+// omega (c invd): RM_LANES x k / VEC threads per row, each summing every RM_LANES-th entry of VEC
+// columns (16-byte loads, RU entries in flight), combined in a fixed order.  One thread per column
+// walking the row four entries at a time was a chain of up to 13 loads.  16 columns: 84k fine nodes 12.4
+// -> 6.5 us, 26k 9.5 -> 4.9, 8.9k 8.9 -> 4.7, and the sweep's own launch (5 us) saved.
+constexpr int RM_LANES = 4;
 template <class T>
 static __global__ void __launch_bounds__(256)
 restrict_multi_kernel(uint32_t nc, int k, const uint32_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
-                      const float* __restrict__ w, const T* __restrict__ f, T* __restrict__ c) {
-  const size_t gid = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t i = gid / k;
-  const int j = int(gid % k);
-  if (i >= nc) return;
-  T acc = T(0);
-  const uint32_t p1 = rowptr[i + 1];
-  // four entries per step: their column and weight loads, then their f loads, go out
-  // together (the sum still runs over the row in order)
-  constexpr int RU = 4;
-  for (uint32_t p0 = rowptr[i]; p0 < p1; p0 += RU) {
-    uint32_t cc[RU];
-    T wv[RU], fv[RU];
+                      const float* __restrict__ w, const T* __restrict__ f, T* __restrict__ c, T omega,
+                      const T* __restrict__ invd, T* __restrict__ x1) {
+  using V = vec16_t<T>;
+  constexpr int VEC = 16 / int(sizeof(T));
+  // lane l of a row's RM_LANES are adjacent threads, so they combine by shuffles
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t l = gid % RM_LANES, item = gid / RM_LANES, kv = uint32_t(k / VEC);
+  const uint32_t i = item / kv, j = (item % kv) * VEC;
+  const bool in = i < nc;
+  V acc = {};
+  if (in) {
+    const uint32_t p1 = rowptr[i + 1];
+    constexpr int RU = 8;
+    for (uint32_t p0 = rowptr[i] + l; p0 < p1; p0 += RU * RM_LANES) {
+      uint32_t cc[RU];
+      T wv[RU];
+      V fv[RU];
 #pragma unroll
-    for (int u = 0; u < RU; ++u) {
-      const bool in = p0 + u < p1;
-      cc[u] = in ? col[p0 + u] : 0u;
-      wv[u] = in ? T(w[p0 + u]) : T(0);
+      for (int u = 0; u < RU; ++u) {
+        const uint32_t p = p0 + u * RM_LANES;
+        cc[u] = p < p1 ? col[p] : 0u;
+        wv[u] = p < p1 ? T(w[p]) : T(0);
+      }
+#pragma unroll
+      for (int u = 0; u < RU; ++u)
+        fv[u] = p0 + u * RM_LANES < p1 ? *reinterpret_cast<const V*>(f + size_t(cc[u]) * k + j) : V{};
+#pragma unroll
+      for (int u = 0; u < RU; ++u) acc += wv[u] * fv[u];
     }
-#pragma unroll
-    for (int u = 0; u < RU; ++u) fv[u] = p0 + u < p1 ? f[size_t(cc[u]) * k + j] : T(0);
-#pragma unroll
-    for (int u = 0; u < RU; ++u)
-      if (p0 + u < p1) acc += wv[u] * fv[u];
   }
-  c[i * k + j] = acc;
+#pragma unroll
+  for (int off = RM_LANES / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[e] += __shfl_down(acc[e], off, RM_LANES);
+  if (!in || l != 0) return;
+  *reinterpret_cast<V*>(c + size_t(i) * k + j) = acc;
+  if (x1) *reinterpret_cast<V*>(x1 + size_t(i) * k + j) = omega * (acc * invd[i]);
 }
 
-// f_out[j][q] = f_in[j][q] + sum_m W[s][pos_j][m] c[cnl[m]][q]
+// f_out[j][q] = f_in[j][q] + sum_m W[s][pos_j][m] c[cnl[m]][q], VEC columns per thread
 template <class T>
 static __global__ void __launch_bounds__(256)
 prolong_multi_kernel(uint32_t nf, int k, const uint32_t* __restrict__ celem, const uint8_t* __restrict__ pos,
                      const uint32_t* __restrict__ cnl, const uint8_t* __restrict__ cs,
                      const T* __restrict__ W, const T* __restrict__ c, const T* __restrict__ f_in,
                      T* __restrict__ f_out) {
-  const size_t gid = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t j = gid / k;
-  const int q = int(gid % k);
+  using V = vec16_t<T>;
+  constexpr int VEC = 16 / int(sizeof(T));
+  const uint32_t kv = uint32_t(k / VEC);
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t j = gid / kv;
   if (j >= nf) return;
+  const size_t q = size_t(gid % kv) * VEC, at = size_t(j) * k + q;
   const uint32_t ce = celem[j];
   const T* wv = W + (size_t(cs[ce]) * 27 + pos[j]) * 8;
   // the coarse values are loaded whatever the weights: they then wait on the vertex ids only
   const uint4 a = reinterpret_cast<const uint4*>(cnl)[2 * size_t(ce)];
   const uint4 b = reinterpret_cast<const uint4*>(cnl)[2 * size_t(ce) + 1];
   const uint32_t idx[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  T cv[8];
+  V cv[8];
 #pragma unroll
-  for (int m = 0; m < 8; ++m) cv[m] = c[size_t(idx[m]) * k + q];
-  T acc = T(0);
+  for (int m = 0; m < 8; ++m) cv[m] = *reinterpret_cast<const V*>(c + size_t(idx[m]) * k + q);
+  V fv = {};
+  if (f_in) fv = *reinterpret_cast<const V*>(f_in + at);
+  V acc = {};
 #pragma unroll
   for (int m = 0; m < 8; ++m) {
     const T wk = wv[m];
-    acc += (wk != T(0)) ? wk * cv[m] : T(0);
+    if (wk != T(0)) acc += wk * cv[m];
   }
-  f_out[gid] = (f_in ? f_in[gid] : T(0)) + acc;
+  *reinterpret_cast<V*>(f_out + at) = fv + acc;
 }
 
-// X = Ainv B for the dense coarsest inverse (row pitch ld) and k right-hand sides ([n][k]),
-// split over DM_SPLIT column ranges of Ainv (enough workgroups to fill the chip):
-// part[s][i][j] = sum over m in range s of Ainv[i][m] B[m][j] (FP64), then
-// dense_multi_sum_kernel adds the ranges in order.  A workgroup computes DM_ROWS rows x 32
-// columns of one range, a thread a 4 x 4 block of them (rows 4 tr .. 4 tr + 3, columns
-// 4 tc .. 4 tc + 3) from one 16-byte LDS read of each operand per m; Ainv (transposed into
-// LDS, rows padded by 4 values) and B pass through LDS in chunks of DM_CH columns of Ainv,
-// the next chunk in flight in registers meanwhile.
-constexpr int DM_ROWS = 128, DM_CH = 32, DM_SPLIT = 16;
-template <class T>
-__global__ void __launch_bounds__(256)
-dense_multi_kernel(int n, int ld, int k, const T* __restrict__ Ainv, const T* __restrict__ B,
-                   double* __restrict__ part) {
-  static_assert(DM_ROWS == 4 * 32 && MAXK == 4 * 8, "256 threads of 4 x 4 blocks cover DM_ROWS x MAXK");
-  using V = vec16_t<T>;
-  static_assert(sizeof(V) == 4 * sizeof(T), "4-value vectors");
-  __shared__ __align__(16) T sa[DM_CH][DM_ROWS + 4];
-  __shared__ __align__(16) T sb[DM_CH][MAXK];
-  const int row0 = blockIdx.x * DM_ROWS;
-  const int per = (n + DM_SPLIT - 1) / DM_SPLIT;
-  const int mlo = blockIdx.y * per, mhi = min(n, mlo + per);
-  const int tr = threadIdx.x >> 3, tc = threadIdx.x & 7;
-  double acc[4][4];
+// X = Ainv B for the dense coarsest inverse (row pitch ld, FP32) and k right-hand sides ([n][k]) on the
+// matrix cores: FP64 products and sums of the FP32 values (v_mfma_f64_16x16x4).  A workgroup forms 16
+// rows of X, its DM_WAVES wavefronts sharing the columns of Ainv; their sums meet in LDS in a fixed
+// order.  In a step a lane loads 4 adjacent values of a row of Ainv (row lane % 16, columns 4 (lane /
+// 16) ...) and the same 4 rows of B, so the four products of a step take any order of the columns.
+// Result register r of a lane is row lane / 16 + 4 r, column lane % 16.
+// The vector ALUs' form (4 x 4 blocks per thread, 16 partial sums in memory and a kernel to add them)
+// took 33 + 5 us for 2634 rows and 16 columns, this one 12 (22 without the next step's loads in flight);
+// reading the matrix takes about 5, its conversions and products about 7 on the 165 CUs that have rows.
+constexpr int DM_WAVES = 16, DM_UNROLL = 2;
+typedef double mfma_d4 __attribute__((ext_vector_type(4)));
+template <int NT>   // 16-column groups of B
+__global__ void __launch_bounds__(DM_WAVES * 64)
+dense_multi_kernel(int n, int ld, int k, const float* __restrict__ Ainv, const float* __restrict__ B,
+                   float* __restrict__ X) {
+  __shared__ double red[DM_WAVES][16 * 16];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lr = lane & 15, lk = (lane >> 4) * 4;
+  const int row0 = blockIdx.x * 16;
+  const float* Ar = Ainv + size_t(min(row0 + lr, n - 1)) * ld;
+  mfma_d4 acc[NT];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  // the next chunk's values are loaded into registers while the current chunk is used
-  constexpr int NA = DM_ROWS * DM_CH / 256, NB = DM_CH * MAXK / 256;
-  T ra[NA], rb[NB];
+  for (int t = 0; t < NT; ++t) acc[t] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+  float4 an[DM_UNROLL];
+  float bn[DM_UNROLL][NT][4];
   auto fetch = [&](int m0) {
 #pragma unroll
-    for (int q = 0; q < NA; ++q) {   // coalesced along the rows of Ainv
-      const int i = threadIdx.x + q * 256, r = i / DM_CH, m = i % DM_CH;
-      ra[q] = (row0 + r < n && m0 + m < mhi) ? Ainv[size_t(row0 + r) * ld + m0 + m] : T(0);
-    }
+    for (int u = 0; u < DM_UNROLL; ++u) {
+      // columns past the end: the row's padding is zero and so are B's values; ld is a multiple of 8
+      const int m = m0 + u * DM_WAVES * 16 + lk;
+      an[u] = m < n ? *reinterpret_cast<const float4*>(Ar + m) : float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int i = threadIdx.x + q * 256, m = i / MAXK, j = i % MAXK;
-      rb[q] = (j < k && m0 + m < mhi) ? B[size_t(m0 + m) * k + j] : T(0);
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          bn[u][t][e] = (m + e < n && t * 16 + lr < k) ? B[size_t(m + e) * k + t * 16 + lr] : 0.f;
     }
   };
-  if (mlo < mhi) fetch(mlo);
-  for (int m0 = mlo; m0 < mhi; m0 += DM_CH) {
+  fetch(wv * 16);
+  for (int m0 = wv * 16; m0 < n; m0 += DM_UNROLL * DM_WAVES * 16) {
+    float av[DM_UNROLL][4], bv[DM_UNROLL][NT][4];
 #pragma unroll
-    for (int q = 0; q < NA; ++q) {
-      const int i = threadIdx.x + q * 256;
-      sa[i % DM_CH][i / DM_CH] = ra[q];
+    for (int u = 0; u < DM_UNROLL; ++u) {
+      av[u][0] = an[u].x;
+      av[u][1] = an[u].y;
+      av[u][2] = an[u].z;
+      av[u][3] = an[u].w;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[u][t][e] = bn[u][t][e];
     }
+    fetch(m0 + DM_UNROLL * DM_WAVES * 16);   // in flight during the products
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int i = threadIdx.x + q * 256;
-      sb[i / MAXK][i % MAXK] = rb[q];
-    }
-    __syncthreads();
-    if (m0 + DM_CH < mhi) fetch(m0 + DM_CH);
-#pragma unroll 4
-    for (int m = 0; m < DM_CH; ++m) {
-      const V a = *reinterpret_cast<const V*>(&sa[m][4 * tr]);
-      const V b = *reinterpret_cast<const V*>(&sb[m][4 * tc]);
+    for (int u = 0; u < DM_UNROLL; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] += double(a[u]) * double(b[v]);
-    }
-    __syncthreads();
+        for (int t = 0; t < NT; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(double(av[u][e]), double(bv[u][t][e]), acc[t], 0, 0, 0);
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = row0 + 4 * tr + u;
-    if (r >= n) break;
+  for (int t = 0; t < NT; ++t) {
+    if (t) __syncthreads();
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (4 * tc + v < k) part[(size_t(blockIdx.y) * n + r) * k + 4 * tc + v] = acc[u][v];
+    for (int r = 0; r < 4; ++r) red[wv][((lane >> 4) + 4 * r) * 16 + lr] = acc[t][r];
+    __syncthreads();
+    if (threadIdx.x < 256) {
+      const int i = row0 + int(threadIdx.x >> 4), j = t * 16 + int(threadIdx.x & 15);
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < DM_WAVES; ++w) s += red[w][threadIdx.x];
+      if (i < n && j < k) X[size_t(i) * k + j] = float(s);
+    }
   }
-}
-
-template <class T>
-__global__ void __launch_bounds__(256)
-dense_multi_sum_kernel(int n, int k, const double* __restrict__ part, T* __restrict__ X) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(n) * k) return;
-  double s = 0.0;
-  for (int q = 0; q < DM_SPLIT; ++q) s += part[size_t(q) * n * k + i];
-  X[i] = T(s);
 }
 
 // ---------------------------------------------------------------- column reductions
@@ -699,7 +710,8 @@ __global__ void subtract_mean_multi_kernel(uint32_t n, int k, const double* __re
 // ---------------------------------------------------------------- batched CG
 // Scalars per right-hand side j: SM[q * MAXK + j] with q a CgScalar, plus SM_DP0 (initial
 // norm) and SM_ACT (1 while the column iterates).  A converged column is frozen: its
-// step length is zero, so its iterate stays the one that met the test.
+// step length is zero, so its iterate stays the one that met the test (also in an iteration that the
+// host queued before it knew).
 enum { SM_DP0 = S_NSCAL, SM_ACT, SM_NSCAL };
 
 static __global__ void cg_p_multi_kernel(uint32_t n, int k, const double* __restrict__ S, const double* __restrict__ z,
@@ -746,29 +758,58 @@ static __global__ void convert_sub_mean_multi_kernel(uint32_t n, int k, const fl
   z[i] = sum ? zi - double(sum[i % k] / double(n)) : zi;
 }
 
-static __global__ void cg_scalar_multi_kernel(int k, double* __restrict__ S, int precond_norm, int flexible, double rtol) {
-  const int j = threadIdx.x;
-  if (j >= k) return;
-  if (S[SM_ACT * MAXK + j] == 0.0) return;
-  const double dp = sqrt(precond_norm ? S[S_ZZ * MAXK + j] : S[S_RR * MAXK + j]);
-  const double ratio = flexible ? (-S[S_ALPHA * MAXK + j] * S[S_ZW * MAXK + j]) / S[S_RZ * MAXK + j]
-                                : S[S_ZR * MAXK + j] / S[S_RZ * MAXK + j];
-  S[S_DP * MAXK + j] = dp;
-  S[S_RATIO * MAXK + j] = ratio;
-  S[S_RZ * MAXK + j] = S[S_ZR * MAXK + j];
-  if (!(dp > rtol * S[SM_DP0 * MAXK + j])) S[SM_ACT * MAXK + j] = 0.0;
+// Tells the host about the columns after iteration its (one wavefront, lane j: column j; see CgSignal).
+struct CgSignalMulti {
+  double dp[4][MAXK];
+  unsigned int act[4];   // bit j: column j still iterates
+  unsigned long long seq;
+};
+__device__ __forceinline__ void cg_tell(int k, int its, double dp, bool act, CgSignalMulti* sig) {
+  const int j = threadIdx.x, slot = its & 3;
+  const unsigned int mask = static_cast<unsigned int>(__ballot(act));
+  if (j < k) __hip_atomic_store(&sig->dp[slot][j], dp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  if (j == 0) {
+    __hip_atomic_store(&sig->act[slot], mask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&sig->seq, static_cast<unsigned long long>(its) + 1ull, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
-static __global__ void cg_init_multi_kernel(int k, double* __restrict__ S, int precond_norm, double rtol) {
+static __global__ void __launch_bounds__(64)
+cg_scalar_multi_kernel(int k, double* __restrict__ S, int precond_norm, int flexible, double rtol, CgSignalMulti* sig) {
   const int j = threadIdx.x;
-  if (j >= k) return;
-  S[S_RZ * MAXK + j] = S[S_ZR * MAXK + j];
-  const double dp = sqrt(precond_norm ? S[S_ZZ * MAXK + j] : S[S_BB * MAXK + j]);
-  S[S_DP * MAXK + j] = dp;
-  S[SM_DP0 * MAXK + j] = dp;
-  S[S_RATIO * MAXK + j] = 0.0;
-  S[SM_ACT * MAXK + j] = dp > 0.0 ? 1.0 : 0.0;
-  (void)rtol;
+  const int its = int(S[S_ITS * MAXK]) + 1;
+  bool act = j < k && S[SM_ACT * MAXK + j] != 0.0;
+  double dp = 0.0;
+  if (act) {
+    dp = sqrt(precond_norm ? S[S_ZZ * MAXK + j] : S[S_RR * MAXK + j]);
+    const double ratio = flexible ? (-S[S_ALPHA * MAXK + j] * S[S_ZW * MAXK + j]) / S[S_RZ * MAXK + j]
+                                  : S[S_ZR * MAXK + j] / S[S_RZ * MAXK + j];
+    S[S_DP * MAXK + j] = dp;
+    S[S_RATIO * MAXK + j] = ratio;
+    S[S_RZ * MAXK + j] = S[S_ZR * MAXK + j];
+    act = dp > rtol * S[SM_DP0 * MAXK + j];
+    if (!act) S[SM_ACT * MAXK + j] = 0.0;
+  }
+  cg_tell(k, its, dp, act, sig);
+  if (j == 0) S[S_ITS * MAXK] = double(its);
+}
+
+static __global__ void __launch_bounds__(64)
+cg_init_multi_kernel(int k, double* __restrict__ S, int precond_norm, CgSignalMulti* sig) {
+  const int j = threadIdx.x;
+  double dp = 0.0;
+  if (j < k) {
+    S[S_RZ * MAXK + j] = S[S_ZR * MAXK + j];
+    dp = sqrt(precond_norm ? S[S_ZZ * MAXK + j] : S[S_BB * MAXK + j]);
+    S[S_DP * MAXK + j] = dp;
+    S[SM_DP0 * MAXK + j] = dp;
+    S[S_RATIO * MAXK + j] = 0.0;
+    S[SM_ACT * MAXK + j] = dp > 0.0 ? 1.0 : 0.0;
+  }
+  cg_tell(k, 0, dp, dp > 0.0, sig);
+  if (j == 0) S[S_ITS * MAXK] = 0.0;
 }
 
 }  // namespace dgh

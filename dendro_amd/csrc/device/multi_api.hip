@@ -132,18 +132,20 @@ static void launch_multi(dgh_mesh m, const MultiIO<T>& io, hipStream_t st) {
   HIP_CHECK(hipGetLastError());
 }
 
+// c = R f; with x1 given also x1 = omega (c invd)
 template <class T>
-static void restrict_multi(dgh_transfer t, int k, const T* f, T* c, hipStream_t st) {
+static void restrict_multi(dgh_transfer t, int k, const T* f, T* c, hipStream_t st, T omega = T(0),
+                           const T* invd = nullptr, T* x1 = nullptr) {
   const uint32_t nc = t->coarse->N;
-  hipLaunchKernelGGL(restrict_multi_kernel<T>, dim3(blocks_for(size_t(nc) * k)), dim3(256), 0, st, nc, k,
-                     t->rowptr.p, t->col.p, t->w.p, f, c);
+  hipLaunchKernelGGL(restrict_multi_kernel<T>, dim3(blocks_for(size_t(nc) * (k * sizeof(T) / 16) * RM_LANES)), dim3(256), 0,
+                     st, nc, k, t->rowptr.p, t->col.p, t->w.p, f, c, omega, invd, x1);
   HIP_CHECK(hipGetLastError());
 }
 
 template <class T>
 static void prolong_multi(dgh_transfer t, int k, const T* c, const T* f_in, T* f_out, hipStream_t st) {
   const uint32_t nf = t->fine->N;
-  hipLaunchKernelGGL(prolong_multi_kernel<T>, dim3(blocks_for(size_t(nf) * k)), dim3(256), 0, st, nf, k,
+  hipLaunchKernelGGL(prolong_multi_kernel<T>, dim3(blocks_for(size_t(nf) * (k * sizeof(T) / 16))), dim3(256), 0, st, nf, k,
                      t->celem.p, t->pos.p, t->coarse->nl.p, t->coarse->cs.p, Wtab<T>(), c, f_in, f_out);
   HIP_CHECK(hipGetLastError());
 }
@@ -178,10 +180,11 @@ float* mvcycle(dgh_solver s, int l, int k, const float* b, hipStream_t st, bool 
       project_mean_multi<float>(s, uint32_t(n), k, V.r.p, st);
       bb = V.r.p;
     }
-    hipLaunchKernelGGL(dense_multi_kernel<float>, dim3((n + DM_ROWS - 1) / DM_ROWS, DM_SPLIT), dim3(256), 0, st, n,
-                       s->ldc, k, (const float*)s->Ainv32.p, bb, s->mdense.p);
-    hipLaunchKernelGGL(dense_multi_sum_kernel<float>, dim3(blocks_for(size_t(n) * k)), dim3(256), 0, st, n, k,
-                       (const double*)s->mdense.p, V.xa.p);
+    const dim3 gd((n + 15) / 16), bd(DM_WAVES * 64);
+    if (k <= 16)
+      hipLaunchKernelGGL(dense_multi_kernel<1>, gd, bd, 0, st, n, s->ldc, k, (const float*)s->Ainv32.p, bb, V.xa.p);
+    else
+      hipLaunchKernelGGL(dense_multi_kernel<2>, gd, bd, 0, st, n, s->ldc, k, (const float*)s->Ainv32.p, bb, V.xa.p);
     HIP_CHECK(hipGetLastError());
     return V.xa.p;
   }
@@ -199,8 +202,13 @@ float* mvcycle(dgh_solver s, int l, int k, const float* b, hipStream_t st, bool 
     std::swap(xc, xn);
   }
   launch_multi<float, OP_RESID>(m, MultiIO<float>{xc, V.r.p, b, nullptr, 0.f, k}, st);
-  restrict_multi<float>(s->transfers[l - 1], k, V.r.p, s->m32[l - 1].b.p, st);
-  const float* xcoarse = mvcycle(s, l - 1, k, s->m32[l - 1].b.p, st);
+  auto& C = s->m32[l - 1];
+  const bool x1 = l - 1 > 0;   // the restriction writes the coarse level's first sweep too
+  if (x1)
+    restrict_multi<float>(s->transfers[l - 1], k, V.r.p, C.b.p, st, float(s->om_level[l - 1]), s->v32[l - 1].invd.p, C.xa.p);
+  else
+    restrict_multi<float>(s->transfers[l - 1], k, V.r.p, C.b.p, st);
+  const float* xcoarse = mvcycle(s, l - 1, k, C.b.p, st, x1);
   prolong_multi<float>(s->transfers[l - 1], k, xcoarse, xc, xc, st);
   for (int it = 0; it < s->prm.nu_post; ++it) {
     launch_multi<float, OP_SMOOTH>(m, MultiIO<float>{xc, xn, b, invd, om, k}, st);
@@ -256,7 +264,7 @@ static void mcg_iteration(dgh_solver s, int k, hipStream_t st) {
   e.a[2] = s->mz.p; e.b[2] = s->mw.p;    // ZW (flexible update: the V-cycle runs in FP32)
   e.a[3] = pnorm ? nullptr : s->mr.p; e.b[3] = s->mr.p;   // RR
   reduce_multi<double>(n, k, e, 4, s->mpart.p, S + S_ZZ * MAXK, st);
-  hipLaunchKernelGGL(cg_scalar_multi_kernel, dim3(1), dim3(MAXK), 0, st, k, S, int(pnorm), 1, s->prm.rtol);
+  hipLaunchKernelGGL(cg_scalar_multi_kernel, dim3(1), dim3(64), 0, st, k, S, int(pnorm), 1, s->prm.rtol, s->msig);
 }
 
 // Sizes the batched buffers of a solver for k columns (FP32 per-level vectors, FP64 outer
@@ -340,12 +348,12 @@ void ensure_multi_buffers(dgh_solver s, int k) {
   s->mz.alloc(nk);
   s->mp.alloc(nk);
   s->mw.alloc(nk);
-  s->mdense.alloc(size_t(DM_SPLIT) * s->nc * k);
   if (!s->mS.p) {
     s->mS.alloc(size_t(SM_NSCAL) * MAXK);
     s->mpart.alloc(size_t(MAXQ) * RED_BLOCKS_M * MAXK);
     s->mpart_p.alloc(size_t(MAXQ) * RED_BLOCKS_M * MAXK);
     HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->hmS), sizeof(double) * SM_NSCAL * MAXK, hipHostMallocDefault));
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->msig), sizeof(CgSignalMulti), hipHostMallocCoherent));
   }
   HIP_CHECK(hipStreamSynchronize(s->st));
   s->mk = k;
@@ -482,41 +490,54 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
     DotArgs<double> bb{};
     bb.a[0] = s->mr.p; bb.b[0] = s->mr.p;
     reduce_multi<double>(n, k, bb, 1, s->mpart_p.p, S + S_BB * MAXK, st);
-    hipLaunchKernelGGL(cg_init_multi_kernel, dim3(1), dim3(MAXK), 0, st, k, S, int(pnorm), s->prm.rtol);
-    HIP_CHECK(hipMemcpyAsync(s->hmS, S, sizeof(double) * SM_NSCAL * MAXK, hipMemcpyDeviceToHost, st));
-    HIP_CHECK(hipStreamSynchronize(st));
-    std::vector<double> bnorm(k), dp0(k);
-    std::vector<int> its(k, 0), conv(k, 0);
-    for (int j = 0; j < k; ++j) {
-      bnorm[j] = std::sqrt(s->hmS[S_BB * MAXK + j]);
-      dp0[j] = s->hmS[SM_DP0 * MAXK + j];
-      conv[j] = s->hmS[SM_ACT * MAXK + j] == 0.0;
-    }
+    s->msig->seq = 0;
+    hipLaunchKernelGGL(cg_init_multi_kernel, dim3(1), dim3(64), 0, st, k, S, int(pnorm), s->msig);
+    HIP_CHECK(hipGetLastError());
     if (s->prm.use_graph && !s->mgexec) {
       HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
       mcg_iteration(s, k, st);
       HIP_CHECK(hipStreamEndCapture(st, &s->mgraph));
       HIP_CHECK(hipGraphInstantiate(&s->mgexec, s->mgraph, nullptr, nullptr, 0));
     }
-    int it = 0;
+    int it = 0, queued = 0;
     bool bad = false;
-    auto all_done = [&] { return std::all_of(conv.begin(), conv.end(), [](int c) { return c != 0; }); };
-    while (!all_done() && it < s->prm.max_it) {
+    auto queue = [&] {
       if (s->mgexec)
         HIP_CHECK(hipGraphLaunch(s->mgexec, st));
       else
         mcg_iteration(s, k, st);
-      HIP_CHECK(hipMemcpyAsync(s->hmS, S, sizeof(double) * SM_NSCAL * MAXK, hipMemcpyDeviceToHost, st));
-      HIP_CHECK(hipStreamSynchronize(st));
-      ++it;
+      ++queued;
+    };
+    // the columns still iterating after iteration q, and the largest of their norms relative to dp0
+    std::vector<double> dp0(k);
+    std::vector<int> its(k, 0);
+    unsigned int act = 0;
+    double worst = 0.0;
+    auto wait = [&](int q) {
+      cg_wait_seq(&s->msig->seq, q, st);
+      const double* dp = s->msig->dp[q & 3];
+      const unsigned int before = act;
+      act = s->msig->act[q & 3];
+      worst = 0.0;
       for (int j = 0; j < k; ++j) {
-        if (conv[j]) continue;
-        const double dp = s->hmS[S_DP * MAXK + j];
-        its[j] = it;
-        if (!std::isfinite(dp)) bad = true;
-        if (s->hmS[SM_ACT * MAXK + j] == 0.0) conv[j] = 1;
+        if (q == 0) {
+          dp0[j] = dp[j];
+        } else if ((before >> j) & 1u) {
+          its[j] = q;
+          if (!std::isfinite(dp[j])) bad = true;
+        }
+        if ((act >> j) & 1u) worst = std::max(worst, dp[j] / dp0[j]);
       }
-      if (bad) break;
+    };
+    if (s->prm.max_it > 0) queue();
+    wait(0);
+    double rate = CG_USUAL_RATE;
+    while (act && !bad && it < s->prm.max_it) {
+      if (queued == it) queue();
+      if (queued == it + 1 && queued < s->prm.max_it && worst * rate > CG_AHEAD_MARGIN * s->prm.rtol) queue();
+      const double prev = worst;
+      wait(++it);
+      rate = worst / prev;
     }
     hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, uint32_t(nk), (const double*)s->mx.p, X);
     HIP_CHECK(hipEventRecord(e1, st));
@@ -535,10 +556,11 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
       HIP_CHECK(hipStreamSynchronize(st));
       for (int j = 0; j < k; ++j) {
         stats[j].iterations = its[j];
-        stats[j].converged = conv[j];
+        stats[j].converged = ((act >> j) & 1u) ? 0 : 1;
         stats[j].rnorm0 = dp0[j];
         stats[j].rnorm = s->hmS[S_DP * MAXK + j];
-        stats[j].rel_true = bnorm[j] > 0 ? std::sqrt(s->hmS[S_PROJ * MAXK + j]) / bnorm[j] : 0.0;
+        const double bnorm = std::sqrt(s->hmS[S_BB * MAXK + j]);
+        stats[j].rel_true = bnorm > 0 ? std::sqrt(s->hmS[S_PROJ * MAXK + j]) / bnorm : 0.0;
         stats[j].seconds = ms * 1e-3;
       }
     }

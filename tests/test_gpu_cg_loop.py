@@ -90,3 +90,37 @@ def test_many_and_few_partials(problem):
         tiles.append(info["n_tiles"])
         assert st.iterations == ref[0].iterations and rel_err(x, ref[2]) <= 1e-8
     assert tiles[0] > 2048 > 512 > tiles[1]
+
+
+@pytest.mark.parametrize("k", [8, 24])
+@pytest.mark.parametrize("norm", [da.NORM_UNPRECONDITIONED, da.NORM_PRECONDITIONED])
+@pytest.mark.parametrize("rtol,max_it", [(1e-8, 100), (0.3, 100), (1e-8, 2), (1e-8, 0)])
+def test_batched_loop(problem, norm, rtol, max_it, k):
+    """Columns of different difficulty (smooth, rough, zero) against single solves with the same FP32
+    V-cycle: equal iterations, and solutions that agree to what their residuals leave open."""
+    h, coefs, _, b = problem
+    ms = []
+    for l in range(h.n):
+        m = da.Mesh(h.levels[l])
+        m.set_coefficients(*coefs[l])
+        ms.append(m)
+    ts = [da.Transfer(ms[l - 1], ms[l], *h.transfers[l - 1]) for l in range(1, h.n)]
+    rng = np.random.default_rng(19)
+    B = rng.uniform(-1, 1, (h.fine.n_node, k))
+    B[:, 1] = 1.0
+    B[:, 3] = 0.0
+    for graph in (0, 1):
+        s = da.Solver(ms, ts, da.default_params(omega=2.0 / 3.0, nu_pre=2, nu_post=2, rtol=rtol, max_it=max_it,
+                                                norm_type=norm, use_graph=graph, vcycle_prec=da.F32))
+        Bt = torch.tensor(B, dtype=torch.float64, device="cuda:0")
+        X, Y = torch.full_like(Bt, float("nan")), torch.empty_like(Bt)
+        st = s.solve_multi(Bt, X, k)
+        s.solve_multi(Bt, Y, k)
+        assert torch.equal(X, Y)
+        assert st[3].iterations == 0 and st[3].converged and not X[:, 3].any()
+        for j in (0, 1, k - 1):
+            bt, x = Bt[:, j].contiguous(), torch.empty_like(Bt[:, 0])
+            one, _ = s.solve(bt, x)
+            assert st[j].iterations == one.iterations and st[j].converged == one.converged
+            if max_it:
+                assert rel_err(X[:, j].cpu().numpy(), x.cpu().numpy()) <= max(1e-4, 10 * rtol if rtol < 0.1 else 0.0)
