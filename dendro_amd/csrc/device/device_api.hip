@@ -96,6 +96,7 @@ static void launch_op_b(dgh_mesh m, const T* x, const OpIO<T>& io, hipStream_t s
       return;
     }
   }
+  if constexpr (MODE != OP_SMOOTH0) {
 #define DGH_OP_LAUNCH(MASS, UNI, LANE, COMB)                                                                   \
   hipLaunchKernelGGL((tile_op_kernel<T, T, MASS, MODE, BLOCK, UNI, LANE, COMB>), dim3(grid), dim3(BLOCK), lds, st, \
                      m->op.tiles.p, m->op.node_tab.p, x, m->op.lid.p, m->op.texp.p, nt, m->op.pitch, kap, mas, io,  \
@@ -120,6 +121,7 @@ static void launch_op_b(dgh_mesh m, const T* x, const OpIO<T>& io, hipStream_t s
   }
 #undef DGH_OP_LAUNCH
   HIP_CHECK(hipGetLastError());
+  }
 }
 
 template <class T, int MODE>
@@ -648,9 +650,10 @@ static void coarse_apply(dgh_solver s, const T* b, T* x, hipStream_t st) {
 // holding the result (one of the level's two iterate buffers).  The first sweep from zero,
 // x = omega (b * invd), needs no operator: with x1_ready the kernel that produced b has
 // already written it into the level's first iterate buffer (the restriction does so for
-// every level below the top).
+// every level below the top).  out: where the last post-smoothing sweep writes, if there is one; it
+// must not overlap b.
 template <class T>
-static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready = false) {
+static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready = false, T* out = nullptr) {
   auto& VV = vecs<T>(s);
   auto& V = VV[l];
   if (l == 0) {
@@ -683,23 +686,34 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
     hipLaunchKernelGGL(smooth_vec_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, xi, b, (const T*)V.r.p,
                        (const T*)V.invd.p, om, xo);
   };
-  if (!x1_ready)
+  // the first sweep rides in the second one's gather where there is one that gathers so (FP64, 512
+  // threads; its 72 registers would leave one workgroup of 1024 threads per CU), its own launch
+  // elsewhere: 2 us of the 143 of an FP64 V-cycle of 297k elements
+  int pre = s->prm.nu_pre - 1;   // sweeps from a nonzero guess
+  if (sizeof(T) == 8 && !x1_ready && pre > 0 && !split && op_factored(m) && !op_paired<T>(m) && m->block == 512) {
+    launch_op_b<T, OP_SMOOTH0, 512>(m, nullptr, OpIO<T>{xn, b, V.invd.p, om}, st);
+    std::swap(xc, xn);
+    --pre;
+  } else if (!x1_ready) {
     hipLaunchKernelGGL(smooth_first_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, om, b,
                        (const T*)V.invd.p, xc);
+  }
   const bool paired = !split && op_paired<T>(m);
-  auto sweeps = [&](int n_sweeps) {
+  auto sweeps = [&](int n_sweeps, T* last) {   // last: where the last of them writes (nullptr: as the others)
     int it = 0;
     for (; paired && it + 2 <= n_sweeps; it += 2) {
+      if (last && it + 2 == n_sweeps) xn = last;
       launch_pair<T, PAIR_SMOOTH>(m, xc, PairIO<T>{xn, nullptr, b, V.invd.p, om}, st);
       std::swap(xc, xn);
     }
     for (; it < n_sweeps; ++it) {
+      if (last && it + 1 == n_sweeps) xn = last;
       sweep(xc, xn);
       std::swap(xc, xn);
     }
   };
   const bool pair_resid = paired && s->prm.nu_pre % 2 == 0;   // the last of nu_pre - 1 sweeps and the residual
-  sweeps(s->prm.nu_pre - 1 - (pair_resid ? 1 : 0));
+  sweeps(pre - (pair_resid ? 1 : 0), nullptr);
   if (pair_resid) {
     launch_pair<T, PAIR_RESID>(m, xc, PairIO<T>{xn, V.r.p, b, V.invd.p, om}, st);
     std::swap(xc, xn);
@@ -716,7 +730,7 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
     launch_restrict<T>(s->transfers[l - 1], V.r.p, C.b.p, st);
   T* xcoarse = vcycle<T>(s, l - 1, C.b.p, st, l - 1 > 0 && s->prm.nu_pre > 0);
   launch_prolong<T>(s->transfers[l - 1], xcoarse, xc, xc, st);
-  sweeps(s->prm.nu_post);
+  sweeps(s->prm.nu_post, out);
   return xc;
 }
 
@@ -730,8 +744,11 @@ static void precondition(dgh_solver s, const double* r, double* z, hipStream_t s
     const float* res = vcycle<float>(s, top, V.b.p, st);
     hipLaunchKernelGGL((convert_kernel<double, float>), dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, res, z);
   } else {
-    const double* res = vcycle<double>(s, top, r, st);
-    hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, res, z);
+    // the last sweep writes z itself, unless z overlaps r (then, or without a sweep, a copy does: 3 us of
+    // 147 at 297k elements)
+    const bool apart = z + n <= r || r + n <= z;
+    const double* res = vcycle<double>(s, top, r, st, false, apart ? z : nullptr);
+    if (res != z) hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, res, z);
   }
   if (s->prm.null_space) project_mean<double>(s, n, z, st);
 }

@@ -49,7 +49,9 @@ __device__ __forceinline__ void elem_factors(uint32_t lev, uint32_t maxD, double
 // CG: y = A x and the tile's partial sum of x.y (the CG product p.Ap).
 // OP_DIRMV: the Dirichlet-masked MatVec (examples/src/backend/omgJac.C:859-1056): x of
 // boundary nodes is staged as 0 (their columns drop out) and their rows return x itself.
-enum OpMode { OP_MATVEC = 0, OP_DIAG = 1, OP_RESID = 2, OP_SMOOTH = 3, OP_CG = 4, OP_DIRMV = 5 };
+// OP_SMOOTH0: OP_SMOOTH of x = omega (b * invd), the first sweep from a zero guess, formed as it is
+// gathered (x unused).
+enum OpMode { OP_MATVEC = 0, OP_DIAG = 1, OP_RESID = 2, OP_SMOOTH = 3, OP_CG = 4, OP_DIRMV = 5, OP_SMOOTH0 = 6 };
 
 template <class T>
 struct OpIO {
@@ -607,7 +609,8 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
   // store phase waits on no global load.  FP64 loads them before the last barrier instead (held
   // from the gather on, they would take the kernel past the 64 VGPRs of eight wavefronts per
   // SIMD).  Lanes past the owned nodes load the first node's.
-  constexpr bool RS = MODE == OP_RESID || MODE == OP_SMOOTH;
+  constexpr bool SM = MODE == OP_SMOOTH || MODE == OP_SMOOTH0;
+  constexpr bool RS = MODE == OP_RESID || SM;
   constexpr bool EARLY = RS && sizeof(T) == 4;
   T own_b[OP_OC], own_d[OP_OC];
   auto load_own = [&] {
@@ -616,7 +619,7 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
     for (int q = 0; q < OP_OC; ++q) {
       const uint32_t n = threadIdx.x + uint32_t(q * BLOCK) < n_own ? nid[q] : n0;
       own_b[q] = io.b[n];
-      if (MODE == OP_SMOOTH) own_d[q] = io.invd[n];
+      if (SM) own_d[q] = io.invd[n];
     }
   };
   uint32_t own_bdy = 0;   // DIRMV: boundary flags of this thread's owned nodes, one bit each
@@ -624,7 +627,8 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
   if (MODE != OP_DIAG) {
     T v[OP_XC];
 #pragma unroll
-    for (int q = 0; q < OP_XC; ++q) v[q] = x[nid[q]];
+    for (int q = 0; q < OP_XC; ++q)
+      v[q] = MODE == OP_SMOOTH0 ? T(0) + io.omega * (io.b[nid[q]] * io.invd[nid[q]]) : x[nid[q]];
     if (MODE == OP_DIRMV) {   // flags loaded beside x (both wait on the node ids only)
       uint8_t bf[OP_XC];
 #pragma unroll
@@ -698,7 +702,7 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
       io.y[n] = (own_bdy >> q) & 1u ? x[n] : v;
     } else if (MODE == OP_RESID) {
       io.y[n] = own_b[q] - v;
-    } else if (MODE == OP_SMOOTH) {
+    } else if (SM) {
       io.y[n] = xs[i] + io.omega * ((own_b[q] - v) * own_d[q]);   // owned nodes lead the staged x
     } else {
       io.y[n] = v;

@@ -54,6 +54,9 @@ def test_vcycle_of_pairs(mesh, coef):
                 e = rel_err(z.cpu().numpy(), ref)
                 print(f"{mesh} {coef} scale {scale} nu {pre},{post} prec {prec}: {e:.2e}")
                 assert e <= tol
+                same = rt.clone()   # in place: the result may not be written while r is still read
+                s.vcycle(same, same)
+                assert torch.equal(same, z)
 
     check(1.0)
     for l, m in enumerate(ms):
