@@ -1614,6 +1614,7 @@ int dgh_solver_create(int nlevels, const dgh_mesh* meshes, const dgh_transfer* t
       s->bdy_gen.push_back(meshes[l]->bdy_gen);
     }
     HIP_CHECK(hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking));
+    for (int q = 0; q < 3; ++q) HIP_CHECK(hipEventCreateWithFlags(&s->ev[q], q < 2 ? hipEventDefault : hipEventDisableTiming));
     HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->hS), sizeof(double) * S_NSCAL, hipHostMallocDefault));
     HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&s->sig), sizeof(CgSignal), hipHostMallocCoherent));
     s->S.alloc(S_NSCAL);
@@ -1704,10 +1705,7 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
     const uint32_t n = m->N;
     const bool pnorm = (s->prm.norm_type == DGH_NORM_PRECONDITIONED);
     double* S = s->S.p;
-    hipEvent_t e0, e1, eu;
-    HIP_CHECK(hipEventCreate(&e0));
-    HIP_CHECK(hipEventCreate(&e1));
-    HIP_CHECK(hipEventCreateWithFlags(&eu, hipEventDisableTiming));
+    const hipEvent_t e0 = s->ev[0], e1 = s->ev[1], eu = s->ev[2];
     HIP_CHECK(hipEventRecord(eu, ust));          // b is ready on the caller's stream
     HIP_CHECK(hipStreamWaitEvent(st, eu, 0));
     HIP_CHECK(hipEventRecord(e0, st));
@@ -1726,8 +1724,8 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
     if (s->prm.null_space) {
       DotArgs<double> d{};
       d.a[0] = b;
-      reduce<double>(n, d, 1, s->part_p.p, S + S_PROJ, st);
-      mean = S + S_PROJ;
+      reduce<double>(n, d, 1, s->part_p.p, S + S_BSUM, st);
+      mean = S + S_BSUM;
     }
     const bool x1 = s->nlevels > 1 && s->prm.nu_pre > 0;
     if (mixed)
@@ -1788,25 +1786,29 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
     else
       hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, x, 0.0, n);
     HIP_CHECK(hipEventRecord(e1, st));
-    HIP_CHECK(hipEventSynchronize(e1));
-    float ms = 0.f;
-    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
     if (stats) {
       // true residual ||b - A x|| / ||b|| in FP64 (b projected when constants are the null space)
-      hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, b, s->w.p);
-      if (s->prm.null_space) project_mean<double>(s, n, s->w.p, st);
+      const double* rhs = b;
+      if (mean) {
+        hipLaunchKernelGGL(mean_free_kernel, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, 1, b, mean, s->w.p);
+        rhs = s->w.p;
+      }
       if (s->dirichlet) {
         launch_dirmv<double>(m, x, s->z.p, st);
         hipLaunchKernelGGL(resid_vec_kernel<double>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n,
-                           (const double*)s->w.p, (const double*)s->z.p, s->z.p);
+                           rhs, (const double*)s->z.p, s->z.p);
       } else {
-        launch_resid<double>(m, x, s->w.p, s->z.p, st);
+        launch_resid<double>(m, x, rhs, s->z.p, st);
       }
       DotArgs<double> q{};
       q.a[0] = s->z.p; q.b[0] = s->z.p;
       reduce<double>(n, q, 1, s->part_p.p, S + S_PROJ, st);
       HIP_CHECK(hipMemcpyAsync(s->hS, S, sizeof(double) * S_NSCAL, hipMemcpyDeviceToHost, st));
-      HIP_CHECK(hipStreamSynchronize(st));
+    }
+    HIP_CHECK(hipStreamSynchronize(st));
+    if (stats) {
+      float ms = 0.f;
+      HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
       const double bnorm = std::sqrt(s->hS[S_BB]);
       stats->iterations = it;
       stats->converged = conv ? 1 : 0;
@@ -1815,10 +1817,6 @@ int dgh_solver_solve(dgh_solver s, const double* b, double* x, dgh_solve_stats* 
       stats->rel_true = bnorm > 0 ? std::sqrt(s->hS[S_PROJ]) / bnorm : 0.0;
       stats->seconds = ms * 1e-3;
     }
-    HIP_CHECK(hipStreamSynchronize(st));
-    HIP_CHECK(hipEventDestroy(e0));
-    HIP_CHECK(hipEventDestroy(e1));
-    HIP_CHECK(hipEventDestroy(eu));
     if (bad) fail(DGH_ERR_DIVERGED, "CG breakdown: non-finite residual at iteration %d", it);
   });
 }

@@ -292,6 +292,7 @@ struct dgh_solver_s {
   DevBuf<double> ptile;           // per-tile partials of p.w from the operator kernel
   const void* zres = nullptr;     // V-cycle result buffer on the finest level (z, unprojected)
   hipStream_t st = nullptr;
+  hipEvent_t ev[3] = {};          // start and end of a solve, the caller's stream
   hipGraph_t graph = nullptr;     // one CG iteration
   hipGraphExec_t gexec = nullptr;
   uint64_t graph_gen = 0;         // mesh_generation() when the graphs were captured
@@ -322,6 +323,8 @@ struct dgh_solver_s {
     if (hS) (void)hipHostFree(hS);
     if (sig) (void)hipHostFree(sig);
     if (hcS) (void)hipHostFree(hcS);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
     if (st) (void)hipStreamDestroy(st);
   }
 };

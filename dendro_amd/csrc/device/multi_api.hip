@@ -471,15 +471,20 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
     const size_t nk = size_t(n) * k;
     const bool pnorm = (s->prm.norm_type == DGH_NORM_PRECONDITIONED);
     double* S = s->mS.p;
-    hipEvent_t e0, e1, eu;
-    HIP_CHECK(hipEventCreate(&e0));
-    HIP_CHECK(hipEventCreate(&e1));
-    HIP_CHECK(hipEventCreateWithFlags(&eu, hipEventDisableTiming));
+    const hipEvent_t e0 = s->ev[0], e1 = s->ev[1], eu = s->ev[2];
     HIP_CHECK(hipEventRecord(eu, ust));
     HIP_CHECK(hipStreamWaitEvent(st, eu, 0));
     HIP_CHECK(hipEventRecord(e0, st));
-    hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, uint32_t(nk), B, s->mr.p);
-    if (s->prm.null_space) project_mean_multi<double>(s, n, k, s->mr.p, st);
+    const double* mean = nullptr;   // sums of the right-hand sides with a constant null space
+    if (s->prm.null_space) {
+      DotArgs<double> q{};
+      q.a[0] = B;
+      reduce_multi<double>(n, k, q, 1, s->mpart_p.p, S + S_BSUM * MAXK, st);
+      mean = S + S_BSUM * MAXK;
+      hipLaunchKernelGGL(mean_free_kernel, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, n, k, B, mean, s->mr.p);
+    } else {
+      hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, uint32_t(nk), B, s->mr.p);
+    }
     hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, s->mx.p, 0.0, uint32_t(nk));
     hipLaunchKernelGGL(fill_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, s->mp.p, 0.0, uint32_t(nk));
     mprecondition(s, k, s->mr.p, s->mz.p, st);
@@ -541,19 +546,23 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
     }
     hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, uint32_t(nk), (const double*)s->mx.p, X);
     HIP_CHECK(hipEventRecord(e1, st));
-    HIP_CHECK(hipEventSynchronize(e1));
-    float ms = 0.f;
-    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
     if (stats) {
       // true residuals ||b_j - A x_j|| / ||b_j|| in FP64
-      hipLaunchKernelGGL(copy_kernel<double>, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, uint32_t(nk), B, s->mw.p);
-      if (s->prm.null_space) project_mean_multi<double>(s, n, k, s->mw.p, st);
-      launch_multi<double, OP_RESID>(m, MultiIO<double>{X, s->mz.p, s->mw.p, nullptr, 0.0, k}, st);
+      const double* rhs = B;
+      if (mean) {
+        hipLaunchKernelGGL(mean_free_kernel, dim3(blocks_for(nk)), dim3(VBLOCK), 0, st, n, k, B, mean, s->mw.p);
+        rhs = s->mw.p;
+      }
+      launch_multi<double, OP_RESID>(m, MultiIO<double>{X, s->mz.p, rhs, nullptr, 0.0, k}, st);
       DotArgs<double> q{};
       q.a[0] = s->mz.p; q.b[0] = s->mz.p;
       reduce_multi<double>(n, k, q, 1, s->mpart_p.p, S + S_PROJ * MAXK, st);
       HIP_CHECK(hipMemcpyAsync(s->hmS, S, sizeof(double) * SM_NSCAL * MAXK, hipMemcpyDeviceToHost, st));
-      HIP_CHECK(hipStreamSynchronize(st));
+    }
+    HIP_CHECK(hipStreamSynchronize(st));
+    if (stats) {
+      float ms = 0.f;
+      HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
       for (int j = 0; j < k; ++j) {
         stats[j].iterations = its[j];
         stats[j].converged = ((act >> j) & 1u) ? 0 : 1;
@@ -564,10 +573,6 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
         stats[j].seconds = ms * 1e-3;
       }
     }
-    HIP_CHECK(hipStreamSynchronize(st));
-    HIP_CHECK(hipEventDestroy(e0));
-    HIP_CHECK(hipEventDestroy(e1));
-    HIP_CHECK(hipEventDestroy(eu));
     if (bad) fail(DGH_ERR_DIVERGED, "CG breakdown: non-finite residual at iteration %d", it);
   });
 }

@@ -132,6 +132,13 @@ __global__ void subtract_mean_kernel(uint32_t n, const double* __restrict__ sum,
   if (i < n) v[i] = v[i] - T(sum[0] / double(n));
 }
 
+// w[n][j] = b[n][j] - sum[j] / n for k columns
+static __global__ void mean_free_kernel(uint32_t n, int k, const double* __restrict__ b, const double* __restrict__ sum,
+                                        double* __restrict__ w) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < size_t(n) * k) w[i] = b[i] - sum[i % k] / double(n);
+}
+
 // ---------------------------------------------------------------- coarsest-level CG
 // Jacobi-preconditioned CG for coarsest levels too large for the dense inverse, FP64, with
 // its scalars on the device: the iterations run in chunks without host synchronisation;
@@ -206,9 +213,10 @@ static __global__ void ccg_p_kernel(uint32_t n, const double* __restrict__ S, co
 // ---------------------------------------------------------------- CG with device scalars
 // S: RZ = z.r, PW = p.w, DP = stopping-test norm, RATIO = p-update factor, ZZ, ZR, ZW, RR,
 // BB = b.b, ALPHA, PROJ (projection sums), MU = mean(z); single right-hand-side solve: RZN = the
-// new z.r until the x update adopts it, ITS = finished iterations, DP0 = initial norm, DONE.
+// new z.r until the x update adopts it, ITS = finished iterations, DP0 = initial norm, DONE;
+// BSUM = sum of the right-hand side's values (constant null space).
 enum CgScalar { S_RZ = 0, S_PW, S_DP, S_RATIO, S_ZZ, S_ZR, S_ZW, S_RR, S_BB, S_ALPHA, S_PROJ, S_MU, S_RZN, S_ITS,
-                S_DP0, S_DONE, S_NSCAL };
+                S_DP0, S_DONE, S_BSUM, S_NSCAL };
 
 // What the device tells the host about the stopping test, in pinned host memory: the norm after
 // iteration i in dp[i % 4] (i = 0: the initial one), then seq = i + 1.  The host queues at most one
