@@ -395,7 +395,7 @@ cg_p_fused_kernel(uint32_t n, int null_space, int flexible, const double* __rest
       const uint32_t i = i0 + u * stride;
       if (i < n) p[i] = first ? zi[u] - mu : (zi[u] - mu) + ratio * pi[u];
     }
-    fetch(i0 + CG_UNROLL * stride);
+    if (i0 + CG_UNROLL * stride < n) fetch(i0 + CG_UNROLL * stride);
   }
 }
 
@@ -450,7 +450,7 @@ cg_xr_fused_kernel(uint32_t n, int npart, const double* __restrict__ part, doubl
         rr += rn * rn;
       }
     }
-    fetch(i0 + CG_UNROLL * stride);
+    if (i0 + CG_UNROLL * stride < n) fetch(i0 + CG_UNROLL * stride);
   }
   __shared__ double red[VBLOCK / 64];
   rr = wave_sum(rr);
