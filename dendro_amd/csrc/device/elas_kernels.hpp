@@ -23,6 +23,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "kernels.hpp"
 #include "vector_kernels.hpp"
 
@@ -51,9 +54,14 @@ __host__ constexpr size_t elas_lds_bytes(uint32_t max_touch) {
 // K_0 = mu L + (mu + lambda) GD of the unit-size element over its modes (factor 1/8 of the
 // inverse transform included): d0[p], d1[p] = the diagonal of component a at a mode of p
 // difference axes with bit a clear / set; o[bit] = the coupling with third axis sum / difference.
+// big: staged values from 2^big on are scaled by 2^-ELAS_UP first (fx_big; here the modes multiply the
+// transformed values before the last scale, so the modulus of K_0 counts: sums of a row's modes reach
+// 68 times the largest, and the rows themselves at least that one).
 struct ElasModes {
   double d0[4], d1[4], o[2];
+  int big;
 };
+constexpr int ELAS_UP = 8;
 __host__ inline ElasModes elas_modes(double mu, double lam) {
   ElasModes m{};
   for (int p = 1; p <= 3; ++p) {
@@ -65,6 +73,9 @@ __host__ inline ElasModes elas_modes(double mu, double lam) {
   }
   m.o[0] = (mu + lam) / 16.0;
   m.o[1] = (mu + lam) / 48.0;
+  int e = 0;
+  std::frexp(std::max(std::fabs(m.d0[1]), std::fabs(m.d1[1])), &e);   // the largest modes: p = 1
+  m.big = fx_top<double>() - std::max(0, e + 4);
   return m;
 }
 
@@ -164,8 +175,9 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
 #pragma unroll
   for (int w = 0; w < NW; ++w) xhi = max(xhi, s_xhi[w]);
   const bool finite = (xhi >> 20) < 0x7ffu;
-  const int ex = max(int(xhi >> 20) - 1022, FX_XMIN);
+  const int ex = fx_ex<double>(xhi);
   const int es = fx_scale<double>(texp[t], ex);
+  const bool big = __builtin_amdgcn_readfirstlane(ex) > md.big;
   const uint32_t own_bytes = n_own * ELAS_NSTRIDE;
   double quarter = 0.25;
   asm("" : "+s"(quarter));
@@ -183,6 +195,11 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
     for (int a = 0; a < 3; ++a) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) xe[a][k] = *lds_at<double>(XS + l[k] + 8u * a);
+      if (big) {
+        DGH_NO_SELECT;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) xe[a][k] *= 1.0 / (1 << ELAS_UP);
+      }
       hang_interp(reinterpret_cast<double(&)[1][8]>(xe[a]), hb, quarter);
       wht8(xe[a]);
       __builtin_amdgcn_sched_barrier(0);
@@ -211,7 +228,7 @@ elas_tile_kernel(const TileRec* __restrict__ tiles, int ntiles, const uint16_t* 
       xe[2][4] = md.d1[1] * z + (ozx * u + oyz * v2);
     }
     // the element's size h and 2^es in one scale
-    const double sc = ldexp(hFac, int(maxD - elas_level(lp)) + es);
+    const double sc = ldexp(hFac, int(maxD - elas_level(lp)) + (big ? es + ELAS_UP : es));
     const uint32_t own = r0 + lane < rec.n_elem ? own_bytes : 0u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {

@@ -155,6 +155,19 @@ __device__ __forceinline__ int fx_ex(uint32_t hi) {
 template <class T>
 using fx_acc_t = typename std::conditional<sizeof(T) == 8, unsigned long long, unsigned int>::type;
 
+// The factored products add up to eight staged values before they scale them: values of at least
+// 2^fx_top are first multiplied by 2^-FX_UP (exact but for bits far below the fixed-point grid of
+// such values) and the scale of the terms by 2^FX_UP, so that no intermediate overflows where the
+// product itself does not.  ex is the same in a workgroup's threads; the branch not taken costs at
+// most 0.08 us of 9.0 (FP64, 318k elements), nothing elsewhere.
+constexpr int FX_UP = 4;
+template <class T>
+__host__ __device__ constexpr int fx_top() { return sizeof(T) == 8 ? 1020 : 124; }
+template <class T>
+__device__ __forceinline__ bool fx_big(int ex) {
+  return __builtin_amdgcn_readfirstlane(ex) > fx_top<T>();
+}
+
 // Scale exponent of a tile: every contribution times 2^es stays below the fixed-point bound.
 template <class T>
 __device__ __forceinline__ int fx_scale(int2 te, int ex) {
@@ -496,9 +509,10 @@ __device__ __forceinline__ void load_rec_fact(RecF<T>& R, uint32_t g, const uint
 }
 
 // u1 = lap_fac hFac / 2, u2 = mass_fac hFac^3 / 8: the factors of a uniform-coefficient
-// element of level lev are u1 2^(maxD - lev) and u2 8^(maxD - lev).
+// element of level lev are u1 2^(maxD - lev) and u2 8^(maxD - lev).  big (uniform): see fx_big; es
+// holds FX_UP then.
 template <class T, bool MASS, uint32_t XS, bool UNI>
-__device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, int es, double u1, double u2,
+__device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, int es, bool big, double u1, double u2,
                                           uint32_t maxD) {
   const uint4 lp = R.lp;
   const uint32_t w[4] = {lp.x, lp.y, lp.z, lp.w};
@@ -509,6 +523,11 @@ __device__ __forceinline__ void eval_fact(const RecF<T>& R, uint32_t own_bytes, 
   T v[1][8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[0][j] = *lds_at<T>(XS + l[j]);
+  if (big) {
+    DGH_NO_SELECT;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[0][j] *= T(1.0 / (1 << FX_UP));
+  }
   T f1, f2 = T(0);
   if (UNI) {
     const int hs = int(maxD - (rec_class(lp) >> 5));
@@ -667,13 +686,14 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
   const bool finite = (xhi >> 20) < 0x7ffu;
   const int ex = MODE == OP_DIAG ? 1 : fx_ex<T>(xhi);
   const int es = fx_scale<T>(texp[t], ex);
+  const bool big = FACT && fx_big<T>(ex);
   const uint32_t own_bytes = n_own * uint32_t(sizeof(T));
   for (uint32_t r0 = w0; r0 < rec.n_elem; r0 += BLOCK) {
     const bool in = r0 + lane < rec.n_elem;
     if constexpr (FACT) {   // the next records' loads are in flight during the evaluation
       decltype(R) Rn;
       load(Rn, r0 + BLOCK);
-      eval_fact<T, MASS, XS, UNI>(R, in ? own_bytes : 0u, es, lap_fac, mass_fac, maxD);
+      eval_fact<T, MASS, XS, UNI>(R, in ? own_bytes : 0u, big ? es + FX_UP : es, big, lap_fac, mass_fac, maxD);
       R = Rn;
     } else {
       if (in) {
@@ -813,14 +833,15 @@ tile_pair_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__
   __syncthreads();
   max_x();
   bool finite = (xhi >> 20) < 0x7ffu;
-  int es = fx_scale<T>(texp[t], fx_ex<T>(xhi));
+  int ex = fx_ex<T>(xhi), es = fx_scale<T>(texp[t], ex);
   auto sweep = [&](uint32_t n_elem, uint32_t n_own) {
     const uint32_t own_bytes = n_own * uint32_t(sizeof(T));
+    const bool big = fx_big<T>(ex);
     for (uint32_t r0 = w0; r0 < n_elem; r0 += BLOCK) {
       RecF<T> Rn;
       // the last round loads the first records again, for the next sweep
       load(Rn, r0 + BLOCK < n_elem ? r0 + BLOCK : w0);
-      eval_fact<T, MASS, XS, UNI>(R, r0 + lane < n_elem ? own_bytes : 0u, es, u1, u2, maxD);
+      eval_fact<T, MASS, XS, UNI>(R, r0 + lane < n_elem ? own_bytes : 0u, big ? es + FX_UP : es, big, u1, u2, maxD);
       R = Rn;
     }
   };
@@ -842,7 +863,8 @@ tile_pair_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__
   __syncthreads();
   max_x();
   finite = (xhi >> 20) < 0x7ffu;
-  es = fx_scale<T>(texp[t], fx_ex<T>(xhi));
+  ex = fx_ex<T>(xhi);
+  es = fx_scale<T>(texp[t], ex);
   sweep(rec.n_elem2, rec.n_own2);
   __syncthreads();
 #pragma unroll

@@ -75,13 +75,13 @@ __device__ __forceinline__ unsigned long long fx_pack(unsigned int lo, unsigned 
 }
 
 // One record for CPL columns.  n_own = 0 adds nothing; d[p]: the record's mode factors scaled by
-// the tile's bound, cs[q]: the column's scale; node l's values sit at LDS byte address
+// the tile's bound, cs[q]: the column's scale; big (uniform): see fx_big, cs holds 2^FX_UP then; node l's values sit at LDS byte address
 // xb + l RSX sizeof(T) (x) and yb + l RSY sizeof(acc) (sums), one 24-bit multiply-add each
 // (written out: the compiler shares l * stride between the two addresses and adds twice; the
 // strides are at most 64, inline constants).
 template <class T, bool MASS, int CPL, int RSX, int RSY, bool PACK>
-__device__ __forceinline__ void eval_multi(uint4 lp, uint32_t n_own, const T d[4], const T cs[CPL], uint32_t xb,
-                                           uint32_t yb) {
+__device__ __forceinline__ void eval_multi(uint4 lp, uint32_t n_own, const T d[4], const T cs[CPL], bool big,
+                                           uint32_t xb, uint32_t yb) {
   using TA = fx_acc_t<T>;
   const uint32_t w[4] = {lp.x, lp.y, lp.z, lp.w};
   uint32_t l[8];
@@ -95,6 +95,13 @@ __device__ __forceinline__ void eval_multi(uint4 lp, uint32_t n_own, const T d[4
     asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(a) : "v"(l[j]), "n"(int(RSX * sizeof(T))), "v"(xb));
 #pragma unroll
     for (int q = 0; q < CPL; ++q) v[q][j] = *lds_at<T>(a + q * uint32_t(sizeof(T)));
+  }
+  if (big) {
+    DGH_NO_SELECT;
+#pragma unroll
+    for (int q = 0; q < CPL; ++q)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[q][j] *= T(1.0 / (1 << FX_UP));
   }
   T quarter = T(0.25);
   asm("" : "+s"(quarter));
@@ -219,9 +226,19 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
     return h;
   };
   const int es0 = fx_scale<T>(texp[t], 0);
+  // One column of fx_big scales the whole slice (a wavefront's lanes hold all its columns): for the
+  // others that is exact too, but for bits below their grid.
   T cs[CPL];
+  int cex[CPL];
+  bool past = false;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) cs[q] = T(ldexp(1.0, -fx_ex<T>(col_hi(c + q))));
+  for (int q = 0; q < CPL; ++q) {
+    cex[q] = fx_ex<T>(col_hi(c + q));
+    past = past || cex[q] > fx_top<T>();
+  }
+  const bool big = __ballot(past) != 0;
+#pragma unroll
+  for (int q = 0; q < CPL; ++q) cs[q] = T(ldexp(1.0, (big ? FX_UP : 0) - cex[q]));
   // LDS byte addresses of the lane's first column in row 0 of the staged x and of the sums
   const uint32_t xbase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<T>)(xs + c)));
   const uint32_t ybase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<TA>)(ys + c)));
@@ -254,7 +271,7 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
     }
     T d[4];
     fact_modes<T, MASS>(f1, f2, d);
-    eval_multi<T, MASS, CPL, RS, RSY, PACK>(Rc.lp, r0 + uint32_t(es) < rec.n_elem ? n_own : 0u, d, cs, xbase, ybase);
+    eval_multi<T, MASS, CPL, RS, RSY, PACK>(Rc.lp, r0 + uint32_t(es) < rec.n_elem ? n_own : 0u, d, cs, big, xbase, ybase);
   }
   // the store's right-hand sides and diagonals of the kept owned nodes: loaded before the
   // barrier, so they are in flight while the other wavefronts finish their records
