@@ -1,9 +1,9 @@
 // One level of the octree mesh (the reference's ot::DA on a single process) and the
 // fine-node -> coarse-element transfer map between two levels.
 #include <algorithm>
-#include <thread>
 
 #include "octree.hpp"
+#include "workers.hpp"
 
 namespace dgh {
 
@@ -12,19 +12,12 @@ namespace {
 // Runs f(begin, end) over [0, n) on up to 16 host threads.
 template <class F>
 void parallel_for(size_t n, F&& f) {
-  unsigned nt = std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
-  if (n < 65536 || nt == 1) {
-    f(size_t(0), n);
-    return;
-  }
-  std::vector<std::thread> th;
+  const unsigned nt = n < 65536 ? 1u : worker_count(n, 1);
   const size_t chunk = (n + nt - 1) / nt;
-  for (unsigned t = 0; t < nt; ++t) {
-    const size_t b = t * chunk, e = std::min(n, b + chunk);
-    if (b >= e) break;
-    th.emplace_back([&f, b, e] { f(b, e); });
-  }
-  for (auto& t : th) t.join();
+  run_workers(nt, [&](unsigned t) {
+    const size_t b = std::min(n, t * chunk), e = std::min(n, b + chunk);
+    if (b < e || nt == 1) f(b, e);
+  });
 }
 
 // exact (anchor, level) lookup in the sorted octant array

@@ -15,9 +15,9 @@
 // type t', and the kernel needs the 18 child-0 stencils only.
 #include <algorithm>
 #include <numeric>
-#include <thread>
 
 #include "octree.hpp"
+#include "workers.hpp"
 
 namespace dgh {
 
@@ -200,15 +200,11 @@ static void concatenate(const std::vector<std::vector<uint32_t>>& t_rec, const s
   }
 }
 
-// Runs f(worker, tile) for every tile on a few threads.
+// Runs f(w, nt) on nt workers; worker w takes every nt-th tile from w on.
 template <class F>
 static void for_tiles(uint32_t ntiles, F f) {
-  unsigned nt = std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
-  nt = std::min(nt, std::max(1u, ntiles / 16u));   // a worker's start costs as much as a dozen small tiles
-  std::vector<std::thread> th;
-  for (unsigned w = 0; w < nt; ++w)
-    th.emplace_back([&f, w, nt, ntiles] { f(w, nt, ntiles); });
-  for (auto& x : th) x.join();
+  const unsigned nt = worker_count(ntiles, 16);   // a worker's start costs as much as a dozen small tiles
+  run_workers(nt, [&](unsigned w) { f(w, nt); });
 }
 
 static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
@@ -257,8 +253,7 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
   plan.tiles.resize(ntiles);
   std::vector<std::vector<uint32_t>> t_rec(ntiles), t_nodes(ntiles);
   std::vector<std::vector<uint16_t>> t_lid(ntiles);
-  std::vector<int> err(16, 0);
-  for_tiles(ntiles, [&](unsigned w, unsigned nt, uint32_t) {
+  for_tiles(ntiles, [&](unsigned w, unsigned nt) {
       std::vector<int32_t> lid_of(N, -1);
       std::vector<uint32_t> cls_end(1024), sorted;
       for (uint32_t t = w; t < ntiles; t += nt) {
@@ -284,10 +279,7 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
         std::sort(extra.begin(), extra.end());
         for (size_t i = 0; i < extra.size(); ++i) lid_of[extra[i]] = int32_t(n_own + i);
         nodes.insert(nodes.end(), extra.begin(), extra.end());
-        if (nodes.size() > 65535) {
-          err[w] = 1;
-          break;
-        }
+        if (nodes.size() > 65535) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
         auto& lids = t_lid[t];
         lids.resize(recs.size() * 8);
         for (size_t r = 0; r < recs.size(); ++r) {
@@ -301,8 +293,6 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
         plan.tiles[t].n_elem = uint32_t(recs.size());
       }
   });
-  for (int e : err)
-    if (e) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
@@ -324,8 +314,7 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
   }
   std::vector<std::vector<uint32_t>> t_rec(ntiles), t_nodes(ntiles);
   std::vector<std::vector<uint16_t>> t_lid(ntiles);
-  std::vector<int> err(16, 0);
-  for_tiles(ntiles, [&](unsigned w, unsigned nt, uint32_t) {
+  for_tiles(ntiles, [&](unsigned w, unsigned nt) {
     std::vector<int32_t> lid_of(N, -1);
     std::vector<uint32_t> emark(E, 0), cls_end(1024), sorted;
     for (uint32_t t = w; t < ntiles; t += nt) {
@@ -365,7 +354,7 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
       add_nodes(r2, false);
       order_records(recs.data(), r2, tp.data(), lev, cls_end, sorted);
       order_records(recs.data() + r2, recs.size() - r2, tp.data(), lev, cls_end, sorted);
-      if (nodes.size() > 65535) err[w] = 1;
+      if (nodes.size() > 65535) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
       auto& lids = t_lid[t];
       lids.resize(recs.size() * 8);
       for (size_t r = 0; r < recs.size(); ++r)
@@ -379,8 +368,6 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
       tr.n_elem2 = uint32_t(r2);
     }
   });
-  for (int e : err)
-    if (e) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
@@ -390,7 +377,7 @@ bool build_gather(uint32_t nrows, const uint32_t* rowptr, const uint32_t* col, c
   std::vector<std::vector<uint32_t>> cols(nb);
   plan.ent.resize(rowptr[nrows]);
   std::vector<int> bad(16, 0);
-  for_tiles(nb, [&](unsigned wk, unsigned nt, uint32_t) {
+  for_tiles(nb, [&](unsigned wk, unsigned nt) {
     // the block's columns in an open-addressed table of twice the most it may hold
     constexpr uint32_t HS = 2u << GATHER_BITS;
     std::vector<uint32_t> key(HS), owner(HS, 0xffffffffu), slot(HS);
