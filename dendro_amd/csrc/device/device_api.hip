@@ -9,9 +9,9 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
-#include <thread>
 #include <vector>
 
+#include "host/workers.hpp"
 #include "internal.hpp"
 
 namespace dgh {
@@ -156,16 +156,12 @@ static void launch_smooth(dgh_mesh m, const T* x, const T* b, const T* invd, T o
   launch_op<T, OP_SMOOTH>(m, x, OpIO<T>{x_out, b, invd, omega}, st);
 }
 
-// Whether two sweeps of the mesh run in one launch.
-template <class T>
-static bool op_paired(const dgh_mesh m) {
-  return op_factored(m) && !m->pair.plan.tiles.empty() && (sizeof(T) == 4 || m->E <= PAIR_MAX_ELEMS64);
-}
+// Whether two sweeps of a level run in one launch.
+static bool op_paired(const dgh_solver s, int l) { return s->pair[l] && op_factored(s->meshes[l]); }
 
-// x = the iterate after one sweep of x, y and r as PairMode says
+// x = the iterate after one sweep of x, y and r as PairMode says; d: the two-sweep tiles of m
 template <class T, int MODE>
-static void launch_pair(dgh_mesh m, const T* x, const PairIO<T>& io, hipStream_t st) {
-  const DevTiles& d = m->pair;
+static void launch_pair(const dgh_mesh_s* m, const DevTiles& d, const T* x, const PairIO<T>& io, hipStream_t st) {
   const int nt = int(d.plan.tiles.size());
   const unsigned grid = unsigned(NXCD * ((nt + NXCD - 1) / NXCD));
   const size_t lds = sizeof(T) == 8 ? d.lds64 : d.lds32;
@@ -308,8 +304,8 @@ static void class_rows(dgh_mesh m) {
 //   |fac1| max_k sum_j |L_t[k][j]| + |fac2| max_k sum_j |M_t[k][j]| < 2^e
 // over the tile's records, factors formed as the kernel forms them (elem_factors), and
 // texp[t].y = v with every owned node of the tile receiving at most 2^v terms.
-void upload_coefs(dgh_mesh m, DevTiles& d) {
-  ++m->gen;
+// Only reads the mesh: the tiling may be a solver's.
+static void upload_coefs(const dgh_mesh_s* m, DevTiles& d) {
   d.rk64.release();
   d.rm64.release();
   d.rk32.release();
@@ -344,10 +340,7 @@ void upload_coefs(dgh_mesh m, DevTiles& d) {
     te[t] = make_int2(std::max(e, -1022), v);
   }
   d.texp.upload(te.data(), te.size());
-  if (!per_elem) {
-    if (&d == &m->op) class_rows(m);
-    return;
-  }
+  if (!per_elem) return;
   std::vector<double> k(R);
   std::vector<float> kf(R);
   // per-record element factors, formed as elem_factors forms them
@@ -416,6 +409,7 @@ void build_devtiles(dgh_mesh m, DevTiles& d, uint32_t T, size_t (*lds)(const Dev
     d.node_tab.upload(d.plan.node_tab.data(), d.plan.node_tab.size());
   }
   upload_coefs(m, d);
+  if (&d == &m->op) class_rows(m);
 }
 
 static size_t op_lds_f64(const DevTiles& d) { return d.lds64; }
@@ -434,27 +428,25 @@ static void upload_pitched(DevTiles& d) {
   d.node_tab.upload(tab.data(), tab.size());
 }
 
-// Two-sweep tiles of the meshes a V-cycle smooths (once per mesh; the meshes are planned at the same time).
-static void build_pairs(const std::vector<dgh_mesh>& meshes) {
-  std::vector<std::thread> th;
-  for (dgh_mesh m : meshes)
-    th.emplace_back([m] {
-      try {
-        for (uint32_t T = std::max(32u, m->E / 256u);; T /= 2) {   // one tile per CU; E/128 and E/512 within 2%
-          TilePlan& p = m->pair.plan;
-          build_pair_tiles(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(), T, p);
-          if (p.max_touch <= uint32_t(PAIR_XC * PAIR_BLOCK) && p.max_own <= uint32_t(PAIR_OC * PAIR_BLOCK)) return;
-          if (T < 16) break;   // too dense a neighbourhood
-        }
-      } catch (...) {
-      }
-      m->pair.plan = TilePlan();   // single sweeps
-    });
-  for (auto& t : th) t.join();
-  for (dgh_mesh m : meshes) {
-    m->pair_tried = true;
-    DevTiles& d = m->pair;
-    if (d.plan.tiles.empty()) continue;
+// Two-sweep tiles of the levels a solver's V-cycle smooths so (all planned at the same time).  They
+// are the solver's own: its meshes may be in use by other solvers on other threads and are only read.
+static void build_pairs(dgh_solver s) {
+  std::vector<int> levels;
+  s->pair.resize(s->nlevels);
+  for (int l = 1; l < s->nlevels && !s->dirichlet; ++l)
+    if ((s->prm.coarse_op == DGH_COARSE_JAC2 || l == s->nlevels - 1) &&
+        s->meshes[l]->E <= (s->prm.vcycle_prec == DGH_F32 ? PAIR_MAX_ELEMS : PAIR_MAX_ELEMS64))
+      levels.push_back(l);
+  run_workers(unsigned(levels.size()), [&](unsigned w) {
+    const dgh_mesh_s* m = s->meshes[levels[w]];
+    auto d = std::make_unique<DevTiles>();
+    if (plan_pairs(m->E, m->N, m->h_nl.data(), m->h_child.data(), m->h_hn.data(), m->h_lev.data(),
+                   uint32_t(PAIR_XC * PAIR_BLOCK), uint32_t(PAIR_OC * PAIR_BLOCK), d->plan))
+      s->pair[levels[w]] = std::move(d);
+  });
+  for (int l : levels) {
+    if (!s->pair[l]) continue;
+    DevTiles& d = *s->pair[l];
     d.block = PAIR_BLOCK;
     d.lds64 = uint32_t(tile_lds_bytes<double>(PAIR_BLOCK, d.plan.max_touch));
     d.lds32 = uint32_t(tile_lds_bytes<float>(PAIR_BLOCK, d.plan.max_touch));
@@ -462,7 +454,7 @@ static void build_pairs(const std::vector<dgh_mesh>& meshes) {
     const std::vector<uint16_t> packed = pack_records(d.plan);
     d.lid.upload(packed.data(), packed.size());
     upload_pitched(d);
-    upload_coefs(m, d);
+    upload_coefs(s->meshes[l], d);
   }
 }
 
@@ -690,7 +682,7 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
   // threads; its 72 registers would leave one workgroup of 1024 threads per CU), its own launch
   // elsewhere: 2 us of the 143 of an FP64 V-cycle of 297k elements
   int pre = s->prm.nu_pre - 1;   // sweeps from a nonzero guess
-  if (sizeof(T) == 8 && !x1_ready && pre > 0 && !split && op_factored(m) && !op_paired<T>(m) && m->block == 512) {
+  if (sizeof(T) == 8 && !x1_ready && pre > 0 && !split && op_factored(m) && !op_paired(s, l) && m->block == 512) {
     launch_op_b<T, OP_SMOOTH0, 512>(m, nullptr, OpIO<T>{xn, b, V.invd.p, om}, st);
     std::swap(xc, xn);
     --pre;
@@ -698,12 +690,12 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
     hipLaunchKernelGGL(smooth_first_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, om, b,
                        (const T*)V.invd.p, xc);
   }
-  const bool paired = !split && op_paired<T>(m);
+  const bool paired = !split && op_paired(s, l);
   auto sweeps = [&](int n_sweeps, T* last) {   // last: where the last of them writes (nullptr: as the others)
     int it = 0;
     for (; paired && it + 2 <= n_sweeps; it += 2) {
       if (last && it + 2 == n_sweeps) xn = last;
-      launch_pair<T, PAIR_SMOOTH>(m, xc, PairIO<T>{xn, nullptr, b, V.invd.p, om}, st);
+      launch_pair<T, PAIR_SMOOTH>(m, *s->pair[l], xc, PairIO<T>{xn, nullptr, b, V.invd.p, om}, st);
       std::swap(xc, xn);
     }
     for (; it < n_sweeps; ++it) {
@@ -715,7 +707,7 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
   const bool pair_resid = paired && s->prm.nu_pre % 2 == 0;   // the last of nu_pre - 1 sweeps and the residual
   sweeps(pre - (pair_resid ? 1 : 0), nullptr);
   if (pair_resid) {
-    launch_pair<T, PAIR_RESID>(m, xc, PairIO<T>{xn, V.r.p, b, V.invd.p, om}, st);
+    launch_pair<T, PAIR_RESID>(m, *s->pair[l], xc, PairIO<T>{xn, V.r.p, b, V.invd.p, om}, st);
     std::swap(xc, xn);
   } else if (split) {
     apply(xc);
@@ -1018,6 +1010,7 @@ void refresh_operators(dgh_solver s) {
     if (m->bdy_gen != s->bdy_gen[l])
       fail(DGH_ERR_STATE, "boundary flags of level %d changed after dgh_solver_create", l);
     if (m->coef_gen == s->coef_gen[l]) continue;
+    if (s->pair[l]) upload_coefs(m, *s->pair[l]);
     s->coef_gen[l] = m->coef_gen;
     const uint32_t n = m->N;
     auto& V = s->v64[l];
@@ -1302,9 +1295,10 @@ int dgh_mesh_set_coefficients(dgh_mesh m, const double* kappa, const double* mas
     m->h_mass.clear();
     if (kappa) m->h_kappa.assign(kappa, kappa + m->E);
     if (mass) m->h_mass.assign(mass, mass + m->E);
+    ++m->gen;   // captured graphs hold the factors' buffers
     upload_coefs(m, m->op);
+    class_rows(m);
     if (!m->mop.plan.tiles.empty()) upload_coefs(m, m->mop);
-    if (!m->pair.plan.tiles.empty()) upload_coefs(m, m->pair);
     ++m->coef_gen;
   });
 }
@@ -1620,13 +1614,7 @@ int dgh_solver_create(int nlevels, const dgh_mesh* meshes, const dgh_transfer* t
     s->S.alloc(S_NSCAL);
     s->part.alloc(size_t(MAXQ) * RED_BLOCKS);
     s->part_p.alloc(MAXQ * RED_BLOCKS);
-    std::vector<dgh_mesh> paired;
-    for (int l = 1; l < nlevels && !s->dirichlet; ++l)
-      if (!meshes[l]->pair_tried && (params->coarse_op == DGH_COARSE_JAC2 || l == nlevels - 1) &&
-          meshes[l]->E <= (params->vcycle_prec == DGH_F32 ? PAIR_MAX_ELEMS : PAIR_MAX_ELEMS64) &&
-          std::find(paired.begin(), paired.end(), meshes[l]) == paired.end())
-        paired.push_back(meshes[l]);
-    build_pairs(paired);
+    build_pairs(s.get());
     // per-level vectors and Jacobi diagonals
     s->v64.resize(nlevels);
     if (params->vcycle_prec == DGH_F32) s->v32.resize(nlevels);

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -71,7 +72,7 @@ constexpr size_t CLASS_ROWS_MIN_TILES = 1024;
 // 1024-thread tiles, from LARGE_MESH_ELEMS up of at most 8192 elements.
 constexpr uint32_t MID_MESH_ELEMS = 1200000;
 constexpr uint32_t LARGE_MESH_ELEMS = 4000000;
-// Largest mesh smoothed two sweeps per launch (build_pairs).  The first sweep of a tile takes 7 times
+// Largest level smoothed two sweeps per launch (build_pairs).  The first sweep of a tile takes 7 times
 // its elements' records (a single sweep 1.5 to 2), which a launch of a small mesh has room for: V-cycle
 // with the levels up to 60k elements paired / single, FP64: finest 11k elements 86.1 / 96.7 us, 64k 107.2 /
 // 110.5, 297k 147.8 / 148.4, where its level of 37k gains nothing; pairing levels of 64k and 100k
@@ -181,8 +182,6 @@ struct dgh_mesh_s {
   DevTiles op;
   int block = 512;              // threads per operator workgroup (256, 512 or 1024)
   DevTiles mop;
-  DevTiles pair;                // two sweeps per launch (build_pairs; no tiles: the mesh takes single ones)
-  bool pair_tried = false;
   uint32_t mtile = 0;           // batched tile size (0: default)
   int mvariant = 6;             // batched FP32 products (multi_api.hip): 1 matrix cores, others vector ALUs
   uint64_t gen = 0;             // bumped whenever device tilings or coefficients are rebuilt
@@ -265,6 +264,7 @@ void cg_wait_seq(const unsigned long long* seq, int it, hipStream_t st);
 struct dgh_solver_s {
   int nlevels = 0;
   std::vector<dgh_mesh> meshes;
+  std::vector<std::unique_ptr<DevTiles>> pair;   // levels smoothed two sweeps per launch (build_pairs), else null
   std::vector<dgh_transfer> transfers;
   dgh_solver_params prm{};
   std::vector<LevelVecs<double>> v64;
@@ -330,7 +330,6 @@ struct dgh_solver_s {
 };
 
 namespace dgh {
-void upload_coefs(dgh_mesh m, DevTiles& d);
 // Sum of the generations of a solver's meshes: captured graphs hold their buffers.
 inline uint64_t mesh_generation(dgh_solver s) {
   uint64_t g = 0;

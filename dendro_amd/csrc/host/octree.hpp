@@ -80,6 +80,11 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
 // reads the nodes of those (n_touch).
 void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                       const uint8_t* lev, uint32_t T, TilePlan& plan);
+// Such tiles of E/256 elements (at least 32; E/128 and E/512 run within 2%: one tile per CU), halved
+// until none touches more than max_touch nodes or updates more than max_own in its first sweep.  False,
+// and an empty plan, if not even 8 elements do.
+bool plan_pairs(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                const uint8_t* lev, uint32_t max_touch, uint32_t max_own, TilePlan& plan);
 // Blocks of B consecutive rows of a sparse matrix (CSR, weights multiples of 1/32 in (0, 1]) for
 // kernels that gather each block's distinct columns once: list holds block b's columns, ascending,
 // at [b * pitch, ...), padded with its last one, and ent, per CSR entry, (32 w - 1) << 11 | index in

@@ -371,6 +371,21 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
+bool plan_pairs(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                const uint8_t* lev, uint32_t max_touch, uint32_t max_own, TilePlan& plan) {
+  for (uint32_t T = std::max(32u, E / 256u); T >= 8; T /= 2) {
+    try {
+      build_pair_tiles(E, N, nl, child, hn, lev, T, plan);
+    } catch (const Error& e) {
+      if (e.code != DGH_ERR_ARG) throw;   // too many nodes for its vertex ids
+      continue;
+    }
+    if (plan.max_touch <= max_touch && plan.max_own <= max_own) return true;
+  }
+  plan = TilePlan();
+  return false;
+}
+
 bool build_gather(uint32_t nrows, const uint32_t* rowptr, const uint32_t* col, const float* w, uint32_t B,
                   GatherPlan& plan) {
   const uint32_t nb = (nrows + B - 1) / B;
