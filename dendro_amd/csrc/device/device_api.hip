@@ -987,10 +987,14 @@ static void setup_coarse(dgh_solver s) {
                        s->c1.p);
     HIP_CHECK(hipGetLastError());
   }
-  if (s->prm.vcycle_prec == DGH_F32) {
+  // FP32 inverse: of an FP32 V-cycle, and of the batched V-cycle (ensure_multi_buffers) once it has run
+  if (s->prm.vcycle_prec == DGH_F32 || s->Ainv32.p) {
     s->Ainv32.alloc(size_t(n) * ld);
     hipLaunchKernelGGL((convert_kernel<float, double>), dim3(blocks_for(size_t(n) * ld)), dim3(VBLOCK), 0, 0,
                        uint32_t(size_t(n) * ld), (const double*)s->Ainv64.p, s->Ainv32.p);
+    HIP_CHECK(hipGetLastError());
+  }
+  if (s->prm.vcycle_prec == DGH_F32) {
     s->Ap32.alloc(size_t(nblk) * SB * SB);
     hipLaunchKernelGGL(sym_pack_kernel<float>, dim3(nblk), dim3(256), 0, 0, n, ld, (const float*)s->Ainv32.p, s->Ap32.p);
     HIP_CHECK(hipGetLastError());
