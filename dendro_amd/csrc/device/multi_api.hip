@@ -505,7 +505,8 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
       HIP_CHECK(hipGraphInstantiate(&s->mgexec, s->mgraph, nullptr, nullptr, 0));
     }
     int it = 0, queued = 0;
-    bool bad = false;
+    bool bad = false;            // a column broke down while iterating
+    unsigned int broken = 0;     // columns with a norm that is not finite: not converged, though frozen
     auto queue = [&] {
       if (s->mgexec)
         HIP_CHECK(hipGraphLaunch(s->mgexec, st));
@@ -527,9 +528,13 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
       for (int j = 0; j < k; ++j) {
         if (q == 0) {
           dp0[j] = dp[j];
+          if (!std::isfinite(dp[j])) broken |= 1u << j;
         } else if ((before >> j) & 1u) {
           its[j] = q;
-          if (!std::isfinite(dp[j])) bad = true;
+          if (!std::isfinite(dp[j])) {
+            broken |= 1u << j;
+            bad = true;
+          }
         }
         if ((act >> j) & 1u) worst = std::max(worst, dp[j] / dp0[j]);
       }
@@ -565,7 +570,7 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
       HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
       for (int j = 0; j < k; ++j) {
         stats[j].iterations = its[j];
-        stats[j].converged = ((act >> j) & 1u) ? 0 : 1;
+        stats[j].converged = (((act | broken) >> j) & 1u) ? 0 : 1;
         stats[j].rnorm0 = dp0[j];
         stats[j].rnorm = s->hmS[S_DP * MAXK + j];
         const double bnorm = std::sqrt(s->hmS[S_BB * MAXK + j]);
@@ -573,7 +578,7 @@ int dgh_solver_solve_multi(dgh_solver s, int k, const double* B, double* X, dgh_
         stats[j].seconds = ms * 1e-3;
       }
     }
-    if (bad) fail(DGH_ERR_DIVERGED, "CG breakdown: non-finite residual at iteration %d", it);
+    if (broken) fail(DGH_ERR_DIVERGED, "CG breakdown: non-finite residual by iteration %d", it);
   });
 }
 

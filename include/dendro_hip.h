@@ -411,7 +411,9 @@ int dgh_solver_solve(dgh_solver s, const double* b_dev, double* x_dev, dgh_solve
  * row-major on the device, 16-byte aligned.  Each column runs the KSPSolve CG of dgh_solver_solve with its
  * own scalars and stopping test; all columns share one batched FP32 V-cycle per iteration
  * (FP64 outer CG, flexible update), captured as one hipGraph when params.use_graph is set.
- * A converged column is frozen.  stats: array of k (may be NULL).  Replaces k calls of
+ * A converged column is frozen.  A column whose norm is not finite ends with DGH_ERR_DIVERGED and
+ * converged = 0: after the solve of the others if it is so from the start, else at once (stats and X
+ * are written either way).  stats: array of k (may be NULL).  Replaces k calls of
  * DAMGSolve (omg.C:1121) on one hierarchy. */
 int dgh_solver_solve_multi(dgh_solver s, int k, const double* B_dev, double* X_dev, dgh_solve_stats* stats,
                            void* stream);
