@@ -657,6 +657,12 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
         v[q] = bf[q] ? T(0) : v[q];
         if (q < OP_OC) own_bdy |= (bf[q] ? 1u : 0u) << q;
       }
+      // The ids are taken as new values here, so that the store forms its addresses from them again:
+      // the compiler otherwise keeps the gather's 64-bit offsets to the end, and the FP64 form with kappa
+      // and mass takes 68 registers, above the 64 of two 1024-thread workgroups per CU (56 so: 2.8M
+      // elements 45.0 -> 37.7 us, 1.5M 26.3 -> 23.9; 512-thread tiles 37.4 and 23.9).
+#pragma unroll
+      for (int q = 0; q < OP_OC; ++q) asm volatile("" : "+v"(nid[q]));
     }
     if (EARLY) load_own();
 #pragma unroll
