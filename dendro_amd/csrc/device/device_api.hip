@@ -1243,37 +1243,36 @@ int dgh_mesh_autotune(dgh_mesh m, int prec, uint32_t* tile_elems, uint32_t* bloc
     HIP_CHECK(hipEventCreate(&e1));
     float best = 1e30f;
     uint32_t bt = 0, bb = 0;
+    // the default tiling first: no other is kept unless it is faster
+    uint32_t dt = 0;
+    int db = 0;
+    default_tiling(m->E, dt, db);
+    std::vector<std::pair<uint32_t, int>> cand{{dt, db}};
+    for (uint32_t T : {128u, 256u, 512u, 1024u, 2048u, 4096u, 8192u})
+      for (int B : {256, 512, 1024})
+        if (T != dt || B != db) cand.push_back({T, B});
     // the factored product, which beats every stencil-row source on every tiling measured (64 to
     // 8192 elements per tile, 9k to 10M elements): the row source is back to the default's
     m->rows_auto = true;
-    // small levels need small tiles: enough workgroups to fill the device
-    for (uint32_t T : {128u, 256u, 512u, 1024u, 2048u, 4096u, 8192u}) {
-      for (int B : {256, 512, 1024}) {
-        m->block = B;
-        try {
-          plan_mesh(m, T);
-        } catch (const Error&) {
-          continue;
-        }
-        if (m->op.plan.tile_elems != T) continue;   // reduced to fit LDS: tried already
-        auto run = [&] {
-          if (prec == DGH_F64)
-            launch_matvec<double>(m, xb.p, yb.p, nullptr);
-          else
-            launch_matvec<float>(m, reinterpret_cast<const float*>(xb.p), reinterpret_cast<float*>(yb.p), nullptr);
-        };
-        for (int i = 0; i < 3; ++i) run();
-        HIP_CHECK(hipEventRecord(e0, nullptr));
-        for (int i = 0; i < 10; ++i) run();
-        HIP_CHECK(hipEventRecord(e1, nullptr));
-        HIP_CHECK(hipEventSynchronize(e1));
-        float ms = 0.f;
-        HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-        if (ms < best) {
-          best = ms;
-          bt = T;
-          bb = uint32_t(B);
-        }
+    for (const auto& [T, B] : cand) {
+      m->block = B;
+      try {
+        plan_mesh(m, T);
+      } catch (const Error&) {
+        continue;
+      }
+      if (m->op.plan.tile_elems != T) continue;   // reduced to fit LDS: tried already
+      auto run = [&] {
+        if (prec == DGH_F64)
+          launch_matvec<double>(m, xb.p, yb.p, nullptr);
+        else
+          launch_matvec<float>(m, reinterpret_cast<const float*>(xb.p), reinterpret_cast<float*>(yb.p), nullptr);
+      };
+      const float ms = autotune_ms(e0, e1, 10, run);
+      if (ms < best) {
+        best = ms;
+        bt = T;
+        bb = uint32_t(B);
       }
     }
     HIP_CHECK(hipEventDestroy(e0));

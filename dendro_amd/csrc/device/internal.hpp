@@ -330,6 +330,24 @@ struct dgh_solver_s {
 };
 
 namespace dgh {
+// Time of n launches of a tuning candidate: the shortest of three batches after two launches, so that
+// one disturbed batch does not reject a candidate.
+template <class F>
+float autotune_ms(hipEvent_t e0, hipEvent_t e1, int n, F run) {
+  float best = 1e30f;
+  for (int i = 0; i < 2; ++i) run();
+  for (int r = 0; r < 3; ++r) {
+    HIP_CHECK(hipEventRecord(e0, nullptr));
+    for (int i = 0; i < n; ++i) run();
+    HIP_CHECK(hipEventRecord(e1, nullptr));
+    HIP_CHECK(hipEventSynchronize(e1));
+    float ms = 0.f;
+    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+    best = ms < best ? ms : best;
+  }
+  return best;
+}
+
 // Sum of the generations of a solver's meshes: captured graphs hold their buffers.
 inline uint64_t mesh_generation(dgh_solver s) {
   uint64_t g = 0;

@@ -404,7 +404,12 @@ int dgh_mesh_autotune_multi(dgh_mesh m, int k, uint32_t* tile_elems, int* varian
     float best = 1e30f;
     uint32_t bt = 0;
     int bv = 0;
-    for (uint32_t T : {256u, 512u, 1024u, 2048u}) {
+    // the default tile size first: no other is kept unless it is faster
+    const uint32_t dt = multi_tile_elems(m->E);
+    std::vector<uint32_t> cand{dt};
+    for (uint32_t T : {256u, 512u, 1024u, 2048u})
+      if (T != dt) cand.push_back(T);
+    for (uint32_t T : cand) {
       try {
         plan_multi(m, T);
       } catch (const Error&) {
@@ -414,13 +419,7 @@ int dgh_mesh_autotune_multi(dgh_mesh m, int k, uint32_t* tile_elems, int* varian
       for (int variant = 0; variant < NVARIANT; ++variant) {
         m->mvariant = variant;
         auto run = [&] { launch_multi<float, OP_MATVEC>(m, MultiIO<float>{xb.p, yb.p, nullptr, nullptr, 0.f, k}, nullptr); };
-        for (int i = 0; i < 2; ++i) run();
-        HIP_CHECK(hipEventRecord(e0, nullptr));
-        for (int i = 0; i < 5; ++i) run();
-        HIP_CHECK(hipEventRecord(e1, nullptr));
-        HIP_CHECK(hipEventSynchronize(e1));
-        float ms = 0.f;
-        HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        const float ms = autotune_ms(e0, e1, 5, run);
         if (ms < best) {
           best = ms;
           bt = T;

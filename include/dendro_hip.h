@@ -218,7 +218,7 @@ int dgh_mesh_tile_info(dgh_mesh m, uint32_t* tile_elems, uint32_t* n_tiles, uint
 int dgh_mesh_set_lane_stencils(dgh_mesh m, int on);
 int dgh_mesh_lane_stencils(dgh_mesh m, int* on);
 /* Autotuner: times the operator kernel of precision prec on this mesh for every candidate
- * (tile size, block) choice and keeps the fastest.  Synchronous; uses scratch
+ * (tile size, block) choice, the default one among them, and keeps the fastest.  Synchronous; uses scratch
  * vectors it allocates itself.  Outputs (any may be NULL): the chosen tile size and block
  * and the time per launch.  No reference counterpart. */
 int dgh_mesh_autotune(dgh_mesh m, int prec, uint32_t* tile_elems, uint32_t* block, float* us);
@@ -274,8 +274,8 @@ int dgh_matvec_multi(dgh_mesh m, int prec, int k, const void* x_dev, void* y_dev
  * lane).  The default is variant 6 with 96 to 512 elements by mesh size.  No reference
  * counterpart (tuning hook). */
 int dgh_mesh_set_tile_multi(dgh_mesh m, uint32_t tile_elems, int variant);
-/* Times the FP32 batched operator for k columns over the candidate tile sizes and all
- * product variants and keeps the fastest; outputs (may be NULL) the tile size, the variant
+/* Times the FP32 batched operator for k columns over the candidate tile sizes, the default
+ * one among them, and all product variants and keeps the fastest; outputs (may be NULL) the tile size, the variant
  * and its time per launch.  No reference counterpart. */
 int dgh_mesh_autotune_multi(dgh_mesh m, int k, uint32_t* tile_elems, int* variant, float* us);
 
