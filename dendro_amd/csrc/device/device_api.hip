@@ -682,11 +682,16 @@ static T* vcycle(dgh_solver s, int l, const T* b, hipStream_t st, bool x1_ready 
   // threads; its 72 registers would leave one workgroup of 1024 threads per CU), its own launch
   // elsewhere: 2 us of the 143 of an FP64 V-cycle of 297k elements
   int pre = s->prm.nu_pre - 1;   // sweeps from a nonzero guess
-  if (sizeof(T) == 8 && !x1_ready && pre > 0 && !split && op_factored(m) && !op_paired(s, l) && m->block == 512) {
-    launch_op_b<T, OP_SMOOTH0, 512>(m, nullptr, OpIO<T>{xn, b, V.invd.p, om}, st);
-    std::swap(xc, xn);
-    --pre;
-  } else if (!x1_ready) {
+  bool first = !x1_ready;
+  if constexpr (sizeof(T) == 8) {
+    if (first && pre > 0 && !split && op_factored(m) && !op_paired(s, l) && m->block == 512) {
+      launch_op_b<T, OP_SMOOTH0, 512>(m, nullptr, OpIO<T>{xn, b, V.invd.p, om}, st);
+      std::swap(xc, xn);
+      --pre;
+      first = false;
+    }
+  }
+  if (first) {
     hipLaunchKernelGGL(smooth_first_kernel<T>, dim3(blocks_for(n)), dim3(VBLOCK), 0, st, n, om, b,
                        (const T*)V.invd.p, xc);
   }
@@ -1065,7 +1070,6 @@ int dgh_init(int device) {
           K[t * KSTRIDE + tri(k, j)] = L[size_t(t) * 64 + k * 8 + j];
           K[t * KSTRIDE + 36 + tri(k, j)] = M[size_t(t) * 64 + k * 8 + j];
         }
-    g.K64.upload(K.data(), K.size());
     g.W64.upload(W.data(), W.size());
     std::vector<float> Kf(K.begin(), K.end()), Wf(W.begin(), W.end());
     g.K32.upload(Kf.data(), Kf.size());
@@ -1137,9 +1141,8 @@ int dgh_synchronize(void) {
 
 int dgh_finalize(void) {
   return guarded([&] {
-    g.K64.release();
-    g.W64.release();
     g.K32.release();
+    g.W64.release();
     g.W32.release();
     g.KF64.release();
     g.KF32.release();

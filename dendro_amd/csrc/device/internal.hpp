@@ -87,8 +87,9 @@ struct State {
   bool ready = false;
   int device = 0;
   int max_lds = 65536;            // dynamic LDS bytes a workgroup may use
-  DevBuf<double> K64, W64;        // child-0 stencil triangles [18][72]; transfer weights [144][27][8]
-  DevBuf<float> K32, W32;
+  DevBuf<float> K32;              // child-0 stencil triangles [18][72] (matrix-core batched product)
+  DevBuf<double> W64;             // transfer weights [144][27][8]
+  DevBuf<float> W32;
   DevBuf<double> KF64;            // child-0 full stencil rows [18][128] (Laplacian, mass)
   DevBuf<float> KF32;
   std::vector<double> hKF;        // host copy of KF64
@@ -105,11 +106,8 @@ inline void require_init() {
   if (!g.ready) fail(DGH_ERR_STATE, "dgh_init has not been called");
 }
 
-template <class T> const T* Ktab();
 template <class T> const T* Wtab();
-template <> inline const double* Ktab<double>() { return g.K64.p; }
 template <> inline const double* Wtab<double>() { return g.W64.p; }
-template <> inline const float* Ktab<float>() { return g.K32.p; }
 template <> inline const float* Wtab<float>() { return g.W32.p; }
 template <class T> const T* KFtab();
 template <> inline const double* KFtab<double>() { return g.KF64.p; }

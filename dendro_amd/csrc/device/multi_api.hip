@@ -86,7 +86,7 @@ static void launch_mfma(dgh_mesh m, const DevTiles& d, const float* kap, const f
   const unsigned grid = unsigned(NXCD * ((np + NXCD - 1) / NXCD));
   hipLaunchKernelGGL((tile_multi_mfma_kernel<MASS, MODE, MBLOCK>), dim3(grid), dim3(MBLOCK), multi_lds_mfma(d, MASS), st,
                      d.tiles.p, nt, io.k / KS, d.lid.p, kap, mas, m->lap_fac, m->mass_fac, m->maxD,
-                     m->hFac, Ktab<float>(), d.node_tab.p, d.ys_len, io);
+                     m->hFac, (const float*)g.K32.p, d.node_tab.p, d.ys_len, io);
 }
 
 // The batched kernels move 16-byte vectors of a node's row.

@@ -188,32 +188,6 @@ void generate_graddiv(double* GD /* [144][24][24] */) {
     }
 }
 
-// Shape functions at the 3-point Gauss nodes of the element, in the order of
-// examples/src/backend/omgRhs.C:1141-1180 (g = {0, +sqrt(3/5), -sqrt(3/5)}, m along x, n along
-// y, p along z): S[s][j][9 m + 3 n + p] = phi_j(g_m, g_n, g_p), s = 18 c + t.  Plays the role of
-// createShFnMat (examples/src/backend/handleType2Stencils.C:197-230), which reads
-// Stencils/ShFnStencils.inp.
-void generate_shfn(double* S /* [144][8][27] */) {
-  const double g[3] = {0.0, std::sqrt(3.0 / 5.0), -std::sqrt(3.0 / 5.0)};
-  for (int c = 0; c < 8; ++c)
-    for (int t = 0; t < 18; ++t) {
-      double a[8][8];
-      shape_coeffs(c, kEtypeMask[c][t], a);
-      for (int j = 0; j < 8; ++j)
-        for (int q = 0; q < 27; ++q) {
-          const double P[3] = {g[q / 9], g[(q / 3) % 3], g[q % 3]};
-          double v = 0.0;
-          for (int m = 0; m < 8; ++m) {
-            double b = a[j][m];
-            for (int d = 0; d < 3; ++d)
-              if (kExp[m][d]) b *= P[d];
-            v += b;
-          }
-          S[((size_t(c) * 18 + t) * 8 + j) * 27 + q] = v;
-        }
-    }
-}
-
 // Weights of the 8 coarse shape functions of stencil (c,t) at the 27 positions
 // {-1,0,1}^3 of the element, pos = tx + 3 ty + 9 tz: W[s][pos][k], s = 18 c + t.
 void generate_transfer_weights(double* W /* [144][27][8] */) {
