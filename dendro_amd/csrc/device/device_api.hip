@@ -467,18 +467,22 @@ static uint32_t op_budget(int block) {
 }
 
 // Elements and threads per tile of a mesh of E elements until dgh_mesh_set_tile or the autotuner
-// choose others.  FP64 / FP32 products, us, at the line's sides:
+// choose others.  FP64 / FP32 products on the same buffers, us, at the line's sides:
 //  - below 98k elements tiles of E/256, 64 to 192 elements, on 512 threads: the launch takes about 4
-//    us whatever the tile, and one pass over the records per thread finishes it (9.4k elements
-//    4.2 / 4.0 in tiles of 64, 9.6 / 8.4 of 2048; 37k 4.9 / 4.6 of 192, 10.4 / 8.9 of 2048);
+//    us whatever the tile, and one pass over the records per thread finishes it (9.7k elements
+//    3.9 / 3.9 in tiles of 64, 9.0 / 7.6 of 2048; 41k 4.7 / 4.4 of 159, 5.1 / 4.3 of 64, 9.9 / 8.5 of 2048);
 //  - up to 1.2M elements one tile of E/512 for each of 512 workgroups, at most half the slots of
-//    512-thread workgroups (297k: 8.9 / 7.3 in tiles of 512, 10.8 / 9.1 of 2048, 12.5 / 9.8 of 128,
-//    whose halo records outnumber their own; 630k: 11.8 / 9.1 of 1024, 13.4 / 10.6 of 2048);
+//    512-thread workgroups (318k: 9.7 / 7.6 in tiles of 621, 10.3 / 8.5 of 2048, 12.4 / 9.8 of 128,
+//    whose halo records outnumber their own; 630k: 11.8 / 9.1 of 1024, 13.4 / 10.6 of 2048); the middle
+//    of this range would take smaller ones (490k: 11.3 / 8.6 of 957, 10.1 / 7.8 of 512);
 //  - above, 1024 threads and whole rounds of the 512 workgroup slots with a few to spare, since
-//    the node budget cuts some tiles short (2.0M elements: 23.2 / 17.7 in 511 tiles, 24.6 / 18.9 in
-//    975 of 512 threads, 31.4 / 23.5 in 328; 2.1M: 25.9 in 512 tiles, 29.5 in 513);
-//  - from 4M elements at most 8192 elements, which the node budget cuts to about 5500 (10.5M:
-//    92 / 68 against 95 / 74 in tiles of 4160 on either block; 5.5M 49.9 / 37.7, 2048 x 512 52.0 / 39.4).
+//    the node budget cuts some tiles short (1.9M elements: 25.3 / 18.7 in 497 tiles, 24.8 / 18.3 in 958 of
+//    512 threads, 29.5 / 20.8 in 514, 28.8 / 21.0 in 359; 2.0M: 23.2 / 17.7 in 511, 24.6 / 18.9 in 975 of 512
+//    threads; the Dirichlet product of 1.5M and 2.8M elements 1 to 4% faster than in 993 and 1084 tiles of
+//    512 threads with uniform coefficients or kappa, the same with kappa and mass);
+//  - from 4M elements at most 8192 elements, which the node budget cuts to about 5500 to 5900 (10.5M:
+//    96 / 69 against 100 / 72 in tiles of 4160 x 512 and 102 / 75 x 1024; 5.5M 53.0 / 36.0, 55.1 / 37.8 of 4160
+//    x 512, 55.6 / 38.0 of 2048 x 512).
 static void default_tiling(uint32_t E, uint32_t& T, int& block) {
   block = E >= MID_MESH_ELEMS ? 1024 : 512;
   if (E >= LARGE_MESH_ELEMS) {

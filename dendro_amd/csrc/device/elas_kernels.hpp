@@ -35,9 +35,10 @@ constexpr int ELAS_NSTRIDE = 24;   // LDS bytes per node: three doubles (sums or
 
 // Threads per tile, owned-node capacity and node budget (owned capacity + touched nodes) of an
 // elasticity tile: 128 registers allow 16 wavefronts per CU, as two 512-thread workgroups with
-// half a CU's LDS each (24 B per node slot).  Products of 17k / 90k / 318k / 1.0M elements, tiles of
-// elas_tile_elems: 6.0 / 8.7 / 18.4 / 38.9 us; with 256 threads and a quarter of the LDS 7.1 / 8.9 /
-// 19.7 / 39.9.  Before (24x24 matrix rows, 256 threads, 2200 slots) 37.7 / 37.9 / 61.9 / 106 us.
+// half a CU's LDS each (24 B per node slot); 256 threads and a quarter of the LDS take 18% more at 17k
+// elements, 2 to 7% more from 90k on.  Products of 13k / 119k / 318k / 657k elements, tiles of
+// elas_tile_elems, same buffers: 5.9 / 12.4 / 20.3 / 30.9 us; before (24x24 matrix rows, 256 threads, 2200
+// slots) 37.1 / 38.0 / 49.7 / 84.8.  With another mesh and vectors each time, 318k: 63.3 -> 20.6.
 // It is bound by its 48 LDS operations per record (about 530 cycles per 64 records and CU: 20 us
 // at 1.0M elements) and, at as much again, by its vector instructions.
 constexpr int ELAS_BLOCK = 512;

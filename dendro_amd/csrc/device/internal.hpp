@@ -73,11 +73,11 @@ constexpr size_t CLASS_ROWS_MIN_TILES = 1024;
 constexpr uint32_t MID_MESH_ELEMS = 1200000;
 constexpr uint32_t LARGE_MESH_ELEMS = 4000000;
 // Largest level smoothed two sweeps per launch (build_pairs).  The first sweep of a tile takes 7 times
-// its elements' records (a single sweep 1.5 to 2), which a launch of a small mesh has room for: V-cycle
-// with the levels up to 60k elements paired / single, FP64: finest 11k elements 86.1 / 96.7 us, 64k 107.2 /
-// 110.5, 297k 147.8 / 148.4, where its level of 37k gains nothing; pairing levels of 64k and 100k
-// elements too 113.4 and 156.2.  FP32, whose records cost half: mixed PCG of 631k elements 1941 us
-// single, 1924 with the level of 10k paired, 1900 with that of 41k too.
+// its elements' records (a single sweep 1.5 to 2), which a launch of a small mesh has room for.  With these
+// limits / no pairs / limits of 110k elements, FP64 V-cycle: levels of 14k, 7k, 4k and 2k elements 67.2 /
+// 70.1 / 67.2 us; of 69k, 29k, 13k and 6k 94.9 / 93.7 / 99.6 (the level of 13k gains nothing there); of 301k,
+// 104k, 39k, 13k and 5k 139.2 / 140.0 / 148.3.  FP32, whose records cost half, mixed PCG: 92k, 31k, 10k and
+// 3k 669 / 695 / 675; 490k, 127k, 30k, 7k and 2k 1218 / 1255 / 1223.
 constexpr uint32_t PAIR_MAX_ELEMS = 60000;
 constexpr uint32_t PAIR_MAX_ELEMS64 = 20000;
 // Largest coarsest level solved with a dense inverse (n^2 doubles on the host and the device).

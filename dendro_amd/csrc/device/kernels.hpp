@@ -383,11 +383,13 @@ __device__ __forceinline__ void eval_rows_lane(const Rec& R, uint32_t own_bytes,
 // source before and this form with the next records prefetched, same tilings:
 //   9,374 elements        16.4 / 14.7 us ->  9.5 /  8.1 us
 //   318,081 elements      19.5 / 17.0    -> 10.2 /  8.9
-//   2.1M, kappa only      35.3 / 31.5    -> 26.6 / 20.9
-//   10.5M (1787 tiles)   129.1 / 100.2   -> 92.4 / 68.1 us; without the prefetch 98.4 / 75.5.
+//   2.1M, kappa only      35.5 / 31.7    -> 26.5 / 21.0
+//   10.5M (1787 tiles)   128.6 / 100.4   -> 96.3 / 72.9 us, of which the prefetch 6 to 10%.
+// (Launches back to back on the same buffers; with another mesh and vectors each time the last two take
+// 26.8 and 98.3 us in FP64.)
 // What bounds it now at 10.5M elements: 400 MB per product (records 215, node ids and x 129, y 56)
-// at 4.3 TB/s, of the 6 to 7 a copy of this size reaches; its LDS reads and additions take about
-// as long again and overlap only across workgroups.
+// at 4.2 TB/s, of the 4.65 a 4 GiB copy reaches; its LDS reads and additions take about as long
+// again and overlap only across workgroups.
 //   Laplacian on h: kappa h p 2 (1/6)^(p-1) (1/2)^(3-p); mass: m h^3 (1/6)^p (1/2)^(3-p);
 // FACT_LAP and FACT_MASS are these over 8 for the factors kappa h/2 and m h^3/8.
 __host__ __device__ constexpr double fact_lap(int p) {
@@ -756,7 +758,7 @@ tile_op_kernel(const TileRec* __restrict__ tiles, const uint32_t* __restrict__ n
 // records in the first sweep, so neighbouring tiles repeat the sweep on each other's border nodes
 // instead of exchanging them through memory and a launch.  A single sweep of a small mesh takes 4.5
 // to 5 us in a chain of dependent launches, most of it the launch and two hops to memory; the second
-// sweep here adds about 3: mixed PCG of 37k elements 1258 -> 1090 us.
+// sweep here adds about 3 (PAIR_MAX_ELEMS has what a solve gains).
 enum PairMode { PAIR_SMOOTH = 0, PAIR_RESID = 1 };
 template <class T>
 struct PairIO {
@@ -1038,9 +1040,12 @@ prolong_tile_kernel(uint32_t nf, uint32_t pitch, const uint32_t* __restrict__ li
 // launch does not fill the device 64 rows, FP64 with 8 lanes (FP64 V-cycle 149.6 -> 147.7 us, of 11k
 // elements 84.2 -> 81.9), FP32 with the 4 of restrict_kernel, whose sums it keeps; from RT_LARGE coarse
 // nodes on 128 rows with 2 lanes and two partial sums each, the same sums: there fewer workgroups and
-// shuffles count.  Both transfers in turn, FP32 / FP64 us, 461k fine and 135k coarse nodes: 2 lanes 8.5
-// / 10.4, 4 lanes 9.1 / 12.1, 8 lanes 10.5 / 13.3, the general kernels 11.3 / 14.6; 5.5M and 2.1M: 70 /
-// 89, 104 / 124, 127 / 152 and 95 / 137.
+// shuffles count.  Both transfers in turn on the same buffers, FP32 / FP64 us, in one run: 461k fine and
+// 135k coarse nodes, 2 lanes 8.5 / 10.4, 4 lanes 9.1 / 12.1, 8 lanes 10.5 / 13.3, the general kernels 11.3
+// / 14.6; 5.5M and 2.1M: 70 / 89, 104 / 124, 127 / 152 and 95 / 137.  Against the kernels before (general,
+// the restriction with packed entries): 10.5 / 13.4 -> 8.9 / 10.6 and 84 / 121 -> 67 / 83; with another
+// mesh and vectors each time, FP32, 461k nodes, 11.4 -> 10.1.  The restriction's column lists are padded
+// to the largest block's (1447 columns on this mesh, 605 on average), which is most of what is left.
 constexpr uint32_t RT_ROWS_SMALL = 64, RT_ROWS_LARGE = 128;
 constexpr uint32_t RT_LARGE = 80000;
 template <class T, int NS, int RT_LANES, int RT_ROWS>

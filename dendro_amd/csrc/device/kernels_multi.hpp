@@ -55,12 +55,13 @@ template <class T> using vec16_t = typename Vec16<T>::type;
 // FP64, 32-bit for FP32), with one scale per column of the slice; two adjacent FP32 columns of a
 // lane are added as one 64-bit integer (PACK).  Gathers and stores move 16-byte vectors of a
 // node's slice.  LDS rows are padded so the lanes of different elements spread over the banks.
-// FP32, k = 32, 630k elements with a coefficient: 316 us with stencil triangles in scalar registers
-// (tiles of 1024, one column per lane) -> 143 us in tiles of 512, two columns per lane; FP64 376 ->
-// 238.  It is bound by the vector ALUs (95% of their issue slots): about 118 instructions per element
+// FP32, k = 32, 630k elements with a coefficient, launches on the same buffers: 318 us with stencil
+// triangles in scalar registers (tiles of 1024, one column per lane) -> 145 us in tiles of 512, two
+// columns per lane, FP64 397 -> 231; with another mesh and vectors each time, whose 118 MB come from
+// memory, FP32 369 -> 163.  It is bound by the vector ALUs (95% of their issue slots): about 118 instructions per element
 // and column, 56 of them the product, 24 the conversion and packing of the sums, the rest record
 // unpacking, hanging vertices and addresses; 1.67 records per element (halo).  Eight
-// columns per lane (143 us), 256 or 1024 threads (165, 159 us) do not pay.
+// columns per lane (the same), 256 or 1024 threads (15 and 11% more) do not pay.
 // LDS: owned sums [ys_len][multi_row_y] (fixed point), touched x [max_touch][multi_row] (T).
 template <class T>
 __host__ __device__ constexpr int multi_row(int ksl) { return ksl + 1; }
@@ -75,8 +76,8 @@ __device__ __forceinline__ unsigned long long fx_pack(unsigned int lo, unsigned 
 }
 
 // One record for CPL columns.  n_own = 0 adds nothing; d[p]: the record's mode factors scaled by
-// the tile's bound, cs[q]: the column's scale; big (uniform): see fx_big, cs holds 2^FX_UP then; node l's values sit at LDS byte address
-// xb + l RSX sizeof(T) (x) and yb + l RSY sizeof(acc) (sums), one 24-bit multiply-add each
+// the tile's bound, cs[q]: the column's scale; big (uniform): see fx_big, cs holds 2^FX_UP then; node
+// l's values sit at LDS byte address xb + l RSX sizeof(T) (x) and yb + l RSY sizeof(acc) (sums), one 24-bit multiply-add each
 // (written out: the compiler shares l * stride between the two addresses and adds twice; the
 // strides are at most 64, inline constants).
 template <class T, bool MASS, int CPL, int RSX, int RSY, bool PACK>

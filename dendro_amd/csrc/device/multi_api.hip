@@ -49,13 +49,14 @@ static void plan_multi(dgh_mesh m, uint32_t T) {
 
 // Default tile size of the batched operator, with variant 6 (4 columns per slice, 2 per lane): at
 // most 512 elements, which three (FP32 k = 32: four) workgroups per CU hold, and on small meshes
-// E/100 (at least 96) so that the slices of all tiles fill the device.  FP32 / FP64 products, us:
-//   2.5k elements, k = 32   tiles of 96   5.5 /   5.8, of 512   8.6 /  10.6, of 1024  11.3 /  14.7
-//   40k, k = 32             of 384       17.7 /  24.6, of 128  20.1 /  30.4, of 1024  20.7 /  31.2
-//   630k, k = 32            of 512        143 /   238, of 192   186 /   349, of 1024   144 /   310
-//   630k, k = 8             of 512       40.3 /  62.7, of 192  50.7 /  88.0, of 1024  39.8 /  75.8
-// Variants 4 and 5 (8 columns per slice) reach 140 and 137 us at 630k, k = 32, but take 8.6 and 7.4
-// against 5.6 on the smallest meshes at k = 8, which have half as many workgroups with them.
+// E/100 (at least 96) so that the slices of all tiles fill the device.  FP32 / FP64 products on the
+// same buffers, us:
+//   3.3k elements, k = 32   tiles of 96   6.5 /   7.3, of 512   8.8 /  10.7, of 1024  11.7 /  15.2
+//   41k, k = 32             of 384       19.0 /  24.8, of 128  22.2 /  31.8, of 1024  21.3 /  31.9
+//   490k, k = 32            of 512        125 /   178, of 192   161 /   260, of 1024   125 /   179
+//   490k, k = 8             of 512       37.1 /  54.1, of 192  46.1 /  72.7, of 1024  36.9 /  53.6
+// Variants 4 and 5 (8 columns per slice) reach 123 and 118 us at 490k, k = 32, but take 17.0 and 14.6
+// against 9.0 at 41k, k = 8, where they have half as many workgroups.
 static uint32_t multi_tile_elems(uint32_t n_elem) { return std::min(512u, std::max(96u, n_elem / 100u)); }
 
 void ensure_multi(dgh_mesh m) {

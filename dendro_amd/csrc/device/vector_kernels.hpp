@@ -94,8 +94,8 @@ reduce2_kernel(int nq, const double* __restrict__ part, double* __restrict__ out
   }
 }
 
-// out[0] = part[0] + ... + part[n-1] in the order cg_alpha_kernel sums the operator's tile
-// partials (one workgroup of RED2_THREADS): the same value CG forms for p.w.
+// out[0] = part[0] + ... + part[n-1] in the order of cg_sum_partials (one workgroup of RED2_THREADS):
+// the same value CG forms for p.w.
 static __global__ void __launch_bounds__(RED2_THREADS)
 sum_partials_kernel(int n, const double* __restrict__ part, double* __restrict__ out) {
   __shared__ double red[RED2_THREADS / 64];

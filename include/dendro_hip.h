@@ -285,8 +285,8 @@ int dgh_mesh_autotune_multi(dgh_mesh m, int k, uint32_t* tile_elems, int* varian
  * stencils and GD[3k+a][3j+b] = int d_a phi_k d_b phi_j the grad-div stencils; with boundary
  * flags (dgh_mesh_set_boundary) boundary rows return x and boundary columns are dropped.
  * Replaces CreateElasticityMat / ElasticityMatMult (examples/src/backend/elasticityJac.C:129-211,
- * stencils Stencils/GDType2Stencils.inp).  set_elasticity builds the plan once (element order
- * by stencil type, node slot CSR, a [E][24] FP64 buffer of element outputs). */
+ * stencils Stencils/GDType2Stencils.inp).  set_elasticity builds the plan once
+ * (owner-computes tiles with 24-byte node slots). */
 int dgh_mesh_set_elasticity(dgh_mesh m, double mu, double lambda);
 int dgh_matvec_elasticity(dgh_mesh m, const double* x_dev, double* y_dev, void* stream);
 
