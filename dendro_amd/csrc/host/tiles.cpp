@@ -117,8 +117,12 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
   // 60 ms).
   if (own_cap && T <= (budget - own_cap) / 2) {
     tile_bounds(E, N, nl, T, 0, bounds, 0);
-    build(bounds);
-    if (plan.max_own <= own_cap && plan.max_touch <= budget - own_cap) return;
+    try {
+      build(bounds);
+      if (plan.max_own <= own_cap && plan.max_touch <= budget - own_cap) return;
+    } catch (const Error& e) {
+      if (e.code != DGH_ERR_ARG) throw;   // a tile beyond its vertex ids (elements in no spatial order)
+    }
   }
   tile_bounds(E, N, nl, T, budget, bounds, own_cap);
   build(bounds);
