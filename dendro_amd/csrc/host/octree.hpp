@@ -76,9 +76,11 @@ void build_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* chil
 // tile's second sweep needs what a tile of build_tiles holds: the nodes it owns (n_own2, first in
 // its node list) and the records touching them (n_elem2, its first records).  Its first sweep
 // updates every node of those records (n_own), which takes all records touching them (n_elem), and
-// reads the nodes of those (n_touch).
-void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
-                      const uint8_t* lev, uint32_t T, TilePlan& plan);
+// reads the nodes of those (n_touch).  False, with the plan unfinished, as soon as a tile touches more
+// than max_touch nodes or updates more than max_own.
+bool build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                      const uint8_t* lev, uint32_t T, TilePlan& plan, uint32_t max_touch = 65535u,
+                      uint32_t max_own = 65535u);
 // Such tiles of E/256 elements (at least 32; E/128 and E/512 run within 2%: one tile per CU), halved
 // until none touches more than max_touch nodes or updates more than max_own in its first sweep.  False,
 // and an empty plan, if not even 8 elements do.

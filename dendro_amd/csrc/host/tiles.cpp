@@ -14,6 +14,7 @@
 // mask.  A record therefore stores its vertex list permuted by k -> k^c and the child-0
 // type t', and the kernel needs the 18 child-0 stencils only.
 #include <algorithm>
+#include <atomic>
 #include <numeric>
 
 #include "octree.hpp"
@@ -300,8 +301,10 @@ static void build_from_bounds(uint32_t E, uint32_t N, const uint32_t* nl, const 
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
 }
 
-void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
-                      const uint8_t* lev, uint32_t T, TilePlan& plan) {
+bool build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
+                      const uint8_t* lev, uint32_t T, TilePlan& plan, uint32_t max_touch, uint32_t max_own) {
+  max_touch = std::min(max_touch, 65535u);   // 16-bit vertex ids
+  std::atomic<bool> over{false};
   plan = TilePlan();
   plan.tile_elems = T;
   const uint32_t ntiles = (E + T - 1) / T;
@@ -321,7 +324,7 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
   for_tiles(ntiles, [&](unsigned w, unsigned nt) {
     std::vector<int32_t> lid_of(N, -1);
     std::vector<uint32_t> emark(E, 0), cls_end(1024), sorted;
-    for (uint32_t t = w; t < ntiles; t += nt) {
+    for (uint32_t t = w; t < ntiles && !over.load(std::memory_order_relaxed); t += nt) {
       const uint32_t e0 = t * T, e1 = std::min(E, e0 + T);
       auto& recs = t_rec[t];
       auto& nodes = t_nodes[t];
@@ -356,9 +359,12 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
       const size_t n1 = nodes.size();
       add_elems_of(n_out);
       add_nodes(r2, false);
+      if (nodes.size() > max_touch || n1 > max_own) {
+        over = true;
+        return;
+      }
       order_records(recs.data(), r2, tp.data(), lev, cls_end, sorted);
       order_records(recs.data() + r2, recs.size() - r2, tp.data(), lev, cls_end, sorted);
-      if (nodes.size() > 65535) fail(DGH_ERR_ARG, "a tile touches more than 65535 nodes; use a smaller tile size");
       auto& lids = t_lid[t];
       lids.resize(recs.size() * 8);
       for (size_t r = 0; r < recs.size(); ++r)
@@ -372,20 +378,15 @@ void build_pair_tiles(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t*
       tr.n_elem2 = uint32_t(r2);
     }
   });
+  if (over) return false;
   concatenate(t_rec, t_nodes, t_lid, tp, lev, plan);
+  return true;
 }
 
 bool plan_pairs(uint32_t E, uint32_t N, const uint32_t* nl, const uint8_t* child, const uint8_t* hn,
                 const uint8_t* lev, uint32_t max_touch, uint32_t max_own, TilePlan& plan) {
-  for (uint32_t T = std::max(32u, E / 256u); T >= 8; T /= 2) {
-    try {
-      build_pair_tiles(E, N, nl, child, hn, lev, T, plan);
-    } catch (const Error& e) {
-      if (e.code != DGH_ERR_ARG) throw;   // too many nodes for its vertex ids
-      continue;
-    }
-    if (plan.max_touch <= max_touch && plan.max_own <= max_own) return true;
-  }
+  for (uint32_t T = std::max(32u, E / 256u); T >= 8; T /= 2)
+    if (build_pair_tiles(E, N, nl, child, hn, lev, T, plan, max_touch, max_own)) return true;
   plan = TilePlan();
   return false;
 }
