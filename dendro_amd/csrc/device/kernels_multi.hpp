@@ -230,16 +230,19 @@ tile_multi_kernel(const TileRec* __restrict__ tiles, int ntiles, int nslices,
   // One column of fx_big scales the whole slice (a wavefront's lanes hold all its columns): for the
   // others that is exact too, but for bits below their grid.
   T cs[CPL];
-  int cex[CPL];
   bool past = false;
 #pragma unroll
   for (int q = 0; q < CPL; ++q) {
-    cex[q] = fx_ex<T>(col_hi(c + q));
-    past = past || cex[q] > fx_top<T>();
+    const int ex = fx_ex<T>(col_hi(c + q));
+    past = past || ex > fx_top<T>();
+    cs[q] = T(ldexp(1.0, -ex));
   }
   const bool big = __ballot(past) != 0;
+  if (big) {
+    DGH_NO_SELECT;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) cs[q] = T(ldexp(1.0, (big ? FX_UP : 0) - cex[q]));
+    for (int q = 0; q < CPL; ++q) cs[q] *= T(1 << FX_UP);
+  }
   // LDS byte addresses of the lane's first column in row 0 of the staged x and of the sums
   const uint32_t xbase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<T>)(xs + c)));
   const uint32_t ybase = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr<TA>)(ys + c)));
