@@ -158,8 +158,8 @@ using fx_acc_t = typename std::conditional<sizeof(T) == 8, unsigned long long, u
 // The factored products add up to eight staged values before they scale them: values of at least
 // 2^fx_top are first multiplied by 2^-FX_UP (exact but for bits far below the fixed-point grid of
 // such values) and the scale of the terms by 2^FX_UP, so that no intermediate overflows where the
-// product itself does not.  ex is the same in a workgroup's threads; the branch not taken costs at
-// most 0.08 us of 9.0 (FP64, 318k elements), nothing elsewhere.
+// product itself does not.  ex is the same in a workgroup's threads; the branch not taken costs 0.08 us
+// of 9.0 (FP64, 318k elements), 0.8 of 163 in the batched product of 631k, nothing measurable elsewhere.
 constexpr int FX_UP = 4;
 template <class T>
 __host__ __device__ constexpr int fx_top() { return sizeof(T) == 8 ? 1020 : 124; }
